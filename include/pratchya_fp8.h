@@ -487,6 +487,58 @@ int pratchya_gemm_bf16_nt_ns(const void* A, int64_t lda, const void* B, int64_t 
                              int64_t N, int64_t K, const void* X, int64_t ldx, void* C, int64_t ldc,
                              hipStream_t stream);
 
+/* The 128-row-tile GEMM (K split over workgroups where the tiles alone do not
+ * fill the chip).  Workspace of a call of M x N outputs and `steps` K steps (128
+ * FP8 or 64 bf16 values per step; for pratchya_gemm_bf16_planes segs_short * K /
+ * 64): f32 partials of the K slices, 0 if K is not split. */
+int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps);
+
+/* pratchya_gemm_bs_nt on 128-row tiles (32-row tiles up to M = 32): the same
+ * operands and scale layouts, summed in another order.  Operands are read up
+ * to their last row only, e8m0 bytes one at a time.  N a multiple of 4 (f32) or
+ * 8 (bf16), groups of a power of two of blocks, B's group maxima shared by
+ * aligned runs of 4 rows (PRATCHYA_EUNSUPPORTED otherwise). */
+int pratchya_gemm_bs_t128(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, const float* a_sc32, int64_t a_rdiv,
+                          int64_t a_sr, int64_t a_sk, int64_t a_kg, const uint8_t* B, int64_t ldb,
+                          const uint8_t* b_sc8, const float* b_sc32, int64_t b_rdiv, int64_t b_sr, int64_t b_sk,
+                          int64_t b_kg, int64_t M, int64_t N, int64_t K, void* C, int64_t ldc, int c_dtype, void* ws,
+                          int64_t ws_bytes, hipStream_t stream);
+
+/* Product of operands held as bf16 planes, f32 accumulation:
+ *   C[m][n] = sum over segments s and k of A_s[m][k] * B_s[n][k]   (Q:618-622:
+ * the f32 dots of matmul_impl's backward, each operand in as few exact planes
+ * as its values need, see pratchya_planes).  Segment s multiplies plane
+ * (a_planes >> 4 s) & 15 of A (a_held planes, a_stride elements apart) with
+ * plane (b_planes >> 4 s) & 15 of B; a plane is [M, K] / [N, K] with row stride
+ * lda / ldb, or [K, M] / [K, N] (a_kmajor / b_kmajor).  K a multiple of 64.
+ * flags (device, may be null): flags[0] == 0 leaves out the segments from
+ * segs_short on (their planes are zero); flags[1] != 0 takes B's planes from
+ * b_planes_alt.  b_sc32 (may be null): B is the mode 0 plane of a
+ * [N, K] payload quantized (b_brow, b_bcol) with b_kg blocks per group and
+ * these group maxima; their mantissas multiply the sums per span of K where
+ * they are constant (a multiple of 64 values, PRATCHYA_EUNSUPPORTED otherwise).
+ * X (may be null): bf16 output 1.5 X - 0.5 C (pratchya_ns_combine's bits). */
+int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_stride, int a_kmajor, int a_held, uint32_t a_planes,
+                              const void* B, int64_t ldb, int64_t b_stride, int b_kmajor, int b_held,
+                              uint32_t b_planes, uint32_t b_planes_alt, int64_t M, int64_t N, int64_t K, int segs,
+                              int segs_short, const uint32_t* flags, const float* b_sc32, int64_t b_brow,
+                              int64_t b_bcol, int64_t b_kg, void* C, int64_t ldc, int c_dtype, const void* X,
+                              int64_t ldx, void* ws, int64_t ws_bytes, hipStream_t stream);
+
+/* bf16 planes [planes][T_pad][W] of a row-major [T, W] matrix quantized (a, b)
+ * (rows T .. T_pad zeros; W and b multiples of 8, b a power of two):
+ *   0 payload -> its power-of-two plane f32(q) * (2^(e-127) * 2^floor(log2 G)) / 128
+ *   1 payload -> the three exact pieces of the dequantized f32 value; flags[0]
+ *     |= 1 where a third piece is not zero
+ *   2 f32 (times its block's scale / 128 if sc8 is given, dequantize_impl_bwd) ->
+ *     the three pieces and the first with non-finite values as 0
+ *   3 bf16 (likewise scaled, rounded once to bf16) -> that value, and where any is
+ *     not finite (flags[1] |= 1) a second plane with those as 0
+ *   4 payload -> mode 2's planes of the dequantized f32 value
+ * flags: two words the caller has zeroed on this stream (modes 1 and 3). */
+int pratchya_planes(int mode, const void* src, const uint8_t* sc8, const float* sc32, int64_t T, int64_t W, int64_t a,
+                    int64_t b, int64_t T_pad, void* dst, uint32_t* flags, hipStream_t stream);
+
 /* Symmetric bf16 product C = A . A^T:     replaces the Gram product of newton_schulz
  *   C[m, n] = sum_k A[m, k] * A[n, k]      (pratchya/_nnx_impl/_optimizer.py:20-22,
  * A @ A.T of the wide iterate, and A.T @ A of a tall one, whose transpose is A)

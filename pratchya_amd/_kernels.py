@@ -801,6 +801,68 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
     return c if n_rows == N else c[:, :N]
 
 
+# Planes of an operand of ``gemm_planes`` (pratchya_planes)
+PLANE_POW2, PLANE_SPLIT3, PLANE_SPLIT4, PLANE_BF16, PLANE_SPLIT4Q = 0, 1, 2, 3, 4
+_PLANE_COUNT = {PLANE_POW2: 1, PLANE_SPLIT3: 3, PLANE_SPLIT4: 4, PLANE_BF16: 2, PLANE_SPLIT4Q: 4}
+_PLANE_PAYLOADS = (PLANE_POW2, PLANE_SPLIT3, PLANE_SPLIT4Q)
+
+
+def planes(mode: int, src: torch.Tensor, sc8, sc32, tgrid, flags=None, pad: int = 1) -> torch.Tensor:
+    """The bf16 planes [planes, rows padded to ``pad``, W] of a 2-D payload with
+    its scales (PLANE_POW2, PLANE_SPLIT3, PLANE_SPLIT4Q), an f32 matrix (PLANE_SPLIT4) or a bf16
+    one (PLANE_BF16), the last two taken through dequantize_impl_bwd with the
+    scales if given.  ``flags``: two zeroed uint32 words that say which planes
+    the product needs.  ``PratchyaUnsupported`` for layouts it does not take."""
+    _require_gpu(src)
+    T, W = int(src.shape[0]), int(src.shape[1])
+    Tp = -(-T // pad) * pad
+    x = _u8(src) if mode in _PLANE_PAYLOADS else src
+    x = x.contiguous()
+    if not _aligned(x, 16):
+        x = x.clone()
+    a, b = (int(tgrid[0]), int(tgrid[1])) if sc8 is not None else (1, 8)
+    e8 = _u8(sc8).contiguous() if sc8 is not None else None
+    g32 = sc32.contiguous().float() if sc8 is not None else None
+    out = torch.empty((_PLANE_COUNT[mode], Tp, W), dtype=torch.bfloat16, device=src.device)
+    _lib.check(_lib.load().pratchya_planes(mode, _ptr(x), _ptr(e8) if e8 is not None else None,
+                                           _ptr(g32) if g32 is not None else None, T, W, a, b, Tp, _ptr(out),
+                                           _ptr(flags) if flags is not None else None, _stream(x)), "planes")
+    return out
+
+
+def _nibbles(seq) -> int:
+    return sum(int(v) << (4 * i) for i, v in enumerate(seq))
+
+
+def gemm_planes(a: torch.Tensor, b: torch.Tensor, pairs, k_major: bool, out_dtype=torch.float32, short: int = 0,
+                b_alt=None, flags=None, units=None) -> torch.Tensor:
+    """``sum over (i, j) in pairs of op(a[i]) @ op(b[j])^T`` for bf16 planes
+    ``a`` [planes, M, K] and ``b`` [planes, N, K] (``k_major``: [planes, K, M] and
+    [planes, K, N]) with f32 accumulation.  ``short`` pairs are enough where
+    flags[0] is 0; ``b_alt`` are b's planes where flags[1] is not.  ``units``:
+    ``(sc32, tgrid, blocks per group)`` of the payload that b is the power-of-two
+    plane of."""
+    _require_gpu(a, b)
+    M, Kd = (int(a.shape[2]), int(a.shape[1])) if k_major else (int(a.shape[1]), int(a.shape[2]))
+    N = int(b.shape[2] if k_major else b.shape[1])
+    lib = _lib.load()
+    short = short or len(pairs)
+    c = torch.empty((M, N), dtype=out_dtype, device=a.device)
+    ws_bytes = int(lib.pratchya_gemm_t128_workspace_bytes(M, N, short * (Kd // 64)))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+    pa, pb = _nibbles(i for i, _ in pairs), _nibbles(j for _, j in pairs)
+    g32, brow, bcol, kg = (units[0].contiguous().float(), int(units[1][0]), int(units[1][1]), int(units[2])) \
+        if units is not None else (None, 1, 1, 1)
+    _lib.check(lib.pratchya_gemm_bf16_planes(
+        _ptr(a), int(a.stride(1)), int(a.stride(0)), 1 if k_major else 0, int(a.shape[0]), pa,
+        _ptr(b), int(b.stride(1)), int(b.stride(0)), 1 if k_major else 0, int(b.shape[0]), pb,
+        pb if b_alt is None else _nibbles(b_alt), M, N, Kd, len(pairs), short,
+        _ptr(flags) if flags is not None else None, _ptr(g32) if g32 is not None else None, brow, bcol, kg,
+        _ptr(c), N, _dtype_code(out_dtype), None, 0, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
+        "gemm_planes")
+    return c
+
+
 def transpose_b16(x: torch.Tensor) -> torch.Tensor:
     """[rows, cols] 16-bit matrix -> its transpose [cols, rows], contiguous."""
     _require_gpu(x)

@@ -106,6 +106,15 @@ SIGNATURES = {
     "pratchya_transpose_b16": (_c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "pratchya_split_pack_bf16": (_c_int, [_c_p, _c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
                                           ctypes.POINTER(_c_int), _c_p, _c_i64, _c_i64, _c_p]),
+    "pratchya_gemm_t128_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "pratchya_gemm_bs_t128": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
+                                       _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
+                                       _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p]),
+    "pratchya_gemm_bf16_planes": (_c_int, [_c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32,
+                                           _c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32, ctypes.c_uint32,
+                                           _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_p, _c_p, _c_i64, _c_i64,
+                                           _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p, _c_i64, _c_p]),
+    "pratchya_planes": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "pratchya_gemm_span": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
     "pratchya_transpose_u8": (_c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "pratchya_mfma_ceiling": (_c_int, [_c_p, _c_p, _c_i64, _c_int, _c_i64, _c_p, ctypes.POINTER(_c_i64), _c_p]),

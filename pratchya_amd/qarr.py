@@ -403,21 +403,97 @@ def _fp8_backward(g, x8, xs8, xs32, y8, ys8, ys32, gx, gy, need_x, need_y, pre=N
     return gxf, gyf, gx_final, gy_final
 
 
-def _matmul_cotangents(g, saved, grids, need_x, need_y):
+def _flat_scales(shape, grid) -> bool:
+    """Whether the scales of an array quantized slice by slice with ``grid``
+    are those of its rows flattened into one slice."""
+    rows, W = math.prod(shape[:-1]), int(shape[-1])
+    return len(shape) == 2 or K.group_layout(rows, W, grid)[1] == K.group_layout(int(shape[-2]), W, grid)[1]
+
+
+# Pairs of planes of the weight gradient's product of two f32 operands (their
+# planes 0, 1, 2 are the pieces, 3 the first piece's finite values): the six
+# whose weight is at least 2^-24 of the leading product; a non-finite value
+# takes part in the first only.
+_WGRAD_PAIRS_F32 = [(0, 0), (3, 1), (1, 3), (3, 2), (1, 1), (2, 3)]
+
+
+def _plane_backward(g, scales, saved, grids, need_x, need_y):
+    """f32 cotangents of dequant(x) and dequant(y) (Q:618-622) on the bf16 MFMA
+    kernel, from operands read as few exact bf16 planes, or (None, None) for
+    what its layouts do not take.  ``g``: the product's cotangent (bf16 or f32),
+    ``scales`` (sc_fp8, sc_fp32, grid): those of the output's quantization when
+    g is the cotangent before dequantize_impl_bwd, else None.
+
+    x's cotangent: a quantized weight is one bf16 plane (its e4m3fn values and
+    powers of two) times its group maxima's mantissas, which the kernel applies
+    per span of the contraction: one product per plane of g, where an f32 weight
+    takes three.  The weight's cotangent contracts over the rows of x and g as
+    they lie (K-major), x as two exact pieces where its group maxima are bf16
+    values, else three."""
+    x8, xs8, xs32, y8, ys8, ys32 = saved
+    gx, gy = grids
+    if y8.dim() != 2 or x8.dim() < 2 or g.dtype not in (torch.float32, torch.bfloat16) or int(gx[0]) != 1:
+        return None, None
+    Kd, N = int(y8.shape[0]), int(y8.shape[1])
+    rows = g.numel() // N
+    if rows == 0 or g.numel() != rows * N or x8.numel() != rows * Kd:
+        return None, None
+    gs8 = gs32 = go = None
+    if scales is not None:
+        gs8, gs32, go = scales
+        if int(go[0]) != 1 or int(go[1]) % 8 or not _flat_scales(tuple(g.shape), go):
+            g, gs8, gs32, go = K.dequantize_bwd(g, gs8, gs32, go), None, None, None
+    bf = g.dtype == torch.bfloat16
+    gxf = gyf = None
+    try:
+        flags = torch.zeros(2, dtype=torch.int32, device=g.device)
+        pg = K.planes(K.PLANE_BF16 if bf else K.PLANE_SPLIT4, g.reshape(rows, N), gs8, gs32, go, flags, pad=64)
+    except K.PratchyaUnsupported:
+        return None, None
+    if need_x:
+        try:
+            pw = K.planes(K.PLANE_POW2, y8, ys8, ys32, gy)
+            gxf = K.gemm_planes(pg[:1 if bf else 3, :rows], pw, [(i, 0) for i in range(1 if bf else 3)], False,
+                                units=(ys32, gy, K.group_layout(Kd, N, gy)[1]))
+            gxf = gxf.reshape(tuple(g.shape[:-1]) + (Kd,))
+        except K.PratchyaUnsupported:
+            gxf = None
+    if need_y and _flat_scales(tuple(x8.shape), gx):
+        try:
+            px = K.planes(K.PLANE_SPLIT3 if bf else K.PLANE_SPLIT4Q, x8.reshape(rows, Kd), xs8, xs32, gx, flags, pad=64)
+            if bf:
+                gyf = K.gemm_planes(px, pg, [(0, 0), (1, 0), (2, 0)], True, short=2, b_alt=[0, 1, 1], flags=flags)
+            else:
+                gyf = K.gemm_planes(px, pg, _WGRAD_PAIRS_F32, True)
+        except K.PratchyaUnsupported:
+            gyf = None
+    return gxf, gyf
+
+
+def _matmul_cotangents(g, saved, grids, need_x, need_y, scales=None):
     """f32 cotangents of dequant(x) and dequant(y) from the product's cotangent
     ``g`` (f32, or bf16 holding exact values): the FP8 MFMA dgrad / wgrad in
     the "fp8" mode where the layouts fit, else the reference's f32 dots of the
-    dequantized operands (Q:618-622)."""
+    dequantized operands (Q:618-622).  ``scales`` (sc_fp8, sc_fp32, grid): g is
+    the cotangent before the output's dequantize_impl_bwd."""
     x8, xs8, xs32, y8, ys8, ys32 = saved
     gx, gy = grids
-    res = _fp8_backward(g, x8, xs8, xs32, y8, ys8, ys32, gx, gy, need_x, need_y) \
-        if _backward_mode == "fp8" else None
-    if res is not None:
-        return res[:2]
-    if g.dtype != torch.bfloat16:
-        g = g.float()
-    gxf = _mm_f32(g, _deq32(y8, ys8, ys32, gy), b_t=True) if need_x else None
-    gyf = _mm_f32(_deq32(x8, xs8, xs32, gx), g, a_t=True) if need_y else None
+    if _backward_mode == "fp8":
+        if scales is not None:
+            g, scales = K.dequantize_bwd(g, *scales), None
+        res = _fp8_backward(g, x8, xs8, xs32, y8, ys8, ys32, gx, gy, need_x, need_y)
+        if res is not None:
+            return res[:2]
+    gxf, gyf = _plane_backward(g, scales, saved, grids, need_x, need_y)
+    if (need_x and gxf is None) or (need_y and gyf is None):
+        if scales is not None:
+            g = K.dequantize_bwd(g, *scales)
+        if g.dtype != torch.bfloat16:
+            g = g.float()
+        if need_x and gxf is None:
+            gxf = _mm_f32(g, _deq32(y8, ys8, ys32, gy), b_t=True)
+        if need_y and gyf is None:
+            gyf = _mm_f32(_deq32(x8, xs8, xs32, gx), g, a_t=True)
     return gxf, gyf
 
 
@@ -524,8 +600,7 @@ def _qlinear_grads(ctx, g):
     if res is not None:
         gxf, gyf, gx_final, gy_final = res
     else:
-        g1 = K.dequantize_bwd(g, os8, os32, go)
-        gxf, gyf = _matmul_cotangents(g1, ctx.saved, (gx, gy), need_x, need_y)
+        gxf, gyf = _matmul_cotangents(g, ctx.saved, (gx, gy), need_x, need_y, (os8, os32, go))
     grad_x = grad_y = None
     if need_x:
         grad_x = gxf if gx_final else _requant_cotangent(_reduce_broadcast(gxf, x8.shape), gx, ctx.dtypes[0])

@@ -1,0 +1,101 @@
+"""The 128-row-tile GEMM and the planes of its bf16 operands, at the edges of
+its tiles (128 / 32 rows, 128 columns), its K slices and its scale spans, against
+float64 products of the dequantized operands.
+
+Tolerances: products of bf16 values are exact in f32, so a sum of K of them is
+within K * 2^-24 of the sum of their magnitudes in any order; over random signs
+the relative Frobenius error stays well below 2e-6 at these K (the f32 GEMM
+tests' bound is 1e-5).
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-6
+
+
+def _K():
+    from pratchya_amd import _kernels
+    return _kernels
+
+
+def _randn(shape, seed, dtype=torch.float32, scale=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(shape, generator=g, device="cuda") * scale).to(dtype)
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("M,N,Kd", [(1, 8, 64), (32, 128, 128), (33, 136, 64), (127, 260, 192), (129, 128, 4096),
+                                    (1000, 2944, 2176), (640, 384, 12288)])
+def test_bf16_product(M, N, Kd):
+    K = _K()
+    a, b = _randn((1, M, Kd), 1, torch.bfloat16), _randn((1, N, Kd), 2, torch.bfloat16)
+    ref = a[0].double() @ b[0].double().T
+    c = K.gemm_planes(a, b, [(0, 0)], False)
+    assert _rel(c, ref) <= TOL
+    if M % 8 == 0 and M > 32 and N % 8 == 0:      # K-major operands: the same sums
+        assert torch.equal(c, K.gemm_planes(a.transpose(1, 2).contiguous(), b.transpose(1, 2).contiguous(), [(0, 0)],
+                                            True))
+
+
+@pytest.mark.parametrize("rows,Kd,N,blk,dtype", [
+    (100, 256, 512, 16, torch.bfloat16), (300, 1024, 768, 128, torch.bfloat16), (64, 2176, 2944, 128, torch.bfloat16),
+    (257, 512, 640, 32, torch.bfloat16), (130, 512, 1024, 128, torch.float32), (65, 1280, 640, 16, torch.float32)])
+def test_backward_products(rows, Kd, N, blk, dtype):
+    """Both f32 cotangents of a quantized product whose output scales the
+    cotangent carries, against float64 (blocks of very different sizes, group
+    maxima that change along the contraction); bf16 sources need two pieces of
+    x, f32 ones three."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    w = (_randn((Kd, N), 3) * torch.exp(_randn((Kd, N), 4)) * 0.02).to(dtype)
+    xq = K.quantize(_randn((rows, Kd), 5, dtype), (1, blk))
+    wq = K.quantize(w, (blk, blk))
+    oq = K.quantize(_randn((rows, N), 6, scale=3.0), (1, blk))
+    g = _randn((rows, N), 7, dtype)
+    g1 = K.dequantize_bwd(g, oq[1], oq[2], (1, blk)).double()
+    wd, xd = K.dequantize(*wq, torch.float32, (blk, blk)).double(), K.dequantize(*xq, torch.float32, (1, blk)).double()
+    gx, gw = Q._plane_backward(g, (oq[1], oq[2], (1, blk)), xq + wq, ((1, blk), (blk, blk)), True, True)
+    assert _rel(gx, g1 @ wd.T) <= TOL and _rel(gw, xd.T @ g1) <= TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_backward_products_non_finite(dtype):
+    """inf and NaN cotangents, a zero weight group and an x too large to
+    dequantize: the same elements are inf, -inf and NaN as in the f32 products
+    of the dequantized operands."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    rows, Kd, N, blk = 192, 256, 384, 128
+    x, w, g = _randn((rows, Kd), 1, dtype), _randn((Kd, N), 2, dtype), _randn((rows, N), 3, dtype)
+    x[5, 3], w[:128] = 3e38, 0.0
+    g[7, 9], g[70, 11], g[100, 300] = float("inf"), float("-inf"), float("nan")
+    xq, wq = K.quantize(x, (1, blk)), K.quantize(w, (blk, blk))
+    gx, gw = Q._plane_backward(g, None, xq + wq, ((1, blk), (blk, blk)), True, True)
+    xd, wd = K.dequantize(*xq, torch.float32, (1, blk)), K.dequantize(*wq, torch.float32, (blk, blk))
+    for got, ref in ((gx, K.matmul_f32(g, wd, False, True)), (gw, K.matmul_f32(xd, g, True, False))):
+        assert torch.equal(torch.nan_to_num(got, 0.0, 1.0, -1.0)[~torch.isfinite(ref)],
+                           torch.nan_to_num(ref, 0.0, 1.0, -1.0)[~torch.isfinite(ref)])
+        assert torch.equal(torch.isfinite(got), torch.isfinite(ref))
+
+
+def test_planes_sum_to_the_value():
+    K = _K()
+    x = _randn((130, 512), 1) * torch.exp(4 * _randn((130, 512), 2))
+    q = K.quantize(x, (1, 32))
+    d = K.dequantize(*q, torch.float32, (1, 32))
+    flags = torch.zeros(2, dtype=torch.int32, device="cuda")
+    p = K.planes(K.PLANE_SPLIT3, *q, (1, 32), flags, pad=64)
+    assert p.shape == (3, 192, 512) and not p[:, 130:].any() and flags.tolist() == [1, 0]
+    assert torch.equal(p[:, :130].double().sum(0), d.double())
+    assert torch.equal(K.planes(K.PLANE_SPLIT4, d, None, None, None)[:3].double().sum(0), d.double())
+    # the power-of-two plane times the group maximum's mantissa is the value
+    pw = K.planes(K.PLANE_POW2, *q, (1, 32))[0].double()
+    mant = torch.frexp(q[2].flatten().double())[0] * 2
+    assert torch.allclose(pw * mant.repeat_interleave(64).view(130, 512), d.double(), rtol=2 ** -23, atol=0)
+    flags.zero_()
+    K.planes(K.PLANE_SPLIT3, *K.quantize(x.to(torch.bfloat16), (1, 32)), (1, 32), flags)
+    assert flags.tolist() == [0, 0]              # bf16 group maxima: no third piece
