@@ -632,13 +632,16 @@ def _word_readable(e8: torch.Tensor) -> torch.Tensor:
 
 
 def gemm_nt(a: Operand, b: Operand, out_dtype: torch.dtype = torch.bfloat16,
-            out: torch.Tensor = None) -> torch.Tensor:
+            out: torch.Tensor = None, few: bool = False) -> torch.Tensor:
     """C[M, N] = dequant(a) @ dequant(b)^T on the FP8 MFMA kernel (any M, N;
-    K a multiple of 128)."""
+    K a multiple of 128).  ``few``: a product of few tiles may run as gemm_t128,
+    whose sums are in another order."""
     _require_gpu(a.payload, b.payload)
     if a.k != b.k:
         raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
     M, N, K = a.rows, b.rows, a.k
+    if few and out is None and not a.k_major and prefers_t128(M, a.desc[3], b):
+        return gemm_t128(a, b, out_dtype)
     if a.k_major or b.k_major:
         if not (a.k_major and b.k_major):
             raise PratchyaUnsupported("gemm_nt: K-major FP8 operands are supported as a pair")
@@ -719,6 +722,16 @@ def quantize_dequantize_premax(x: torch.Tensor, block_max: torch.Tensor, tgrid, 
     return y, sc8.view(E8M0), sc32
 
 
+def few_tiles(M: int, N: int) -> bool:
+    """Whether a bf16 product leaves half of the chip idle on 256x256 tiles: it
+    then runs on 128x128 ones with its K steps split (gemm_planes).  Measured
+    (us, 256x256 / 128x128): [1024, 6144] . [6144, 1024] 124 / 27, [2048, 12288]
+    . [12288, 2048] (64 tiles) 254 / 104, [4096, 2048] . [2048, 2048] (128) 50 /
+    37, [3000, 3072] . [3072, 3000] (144) 75 / 78, [4096, 2048] . [2048, 4096]
+    (256) 64 / 70."""
+    return 0 < -(-M // GEMM_TILE_ROWS) * -(-N // GEMM_TILE_ROWS) <= 128
+
+
 def gemm_bf16_nt(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """C[M, N] = a @ b^T for bf16 ``a`` [M, K] and ``b`` [N, K] with f32
     accumulation, rounded once to ``out_dtype``: the bf16 dots of
@@ -737,6 +750,47 @@ def gemm_bf16_nt(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype = torc
     _lib.check(_lib.load().pratchya_gemm_bf16_nt(_ptr(ap), Kd, _ptr(bp), Kd, M, N, Kd, _ptr(out), N,
                                                  _dtype_code(out_dtype), _stream(ap)), "gemm_bf16")
     return out
+
+
+def prefers_t128(M: int, a_kg: int, b: Operand) -> bool:
+    """Whether an FP8 product of M rows (a_kg blocks per group) with ``b`` is one
+    that gemm_t128 takes and runs faster than on the persistent
+    256x256 kernel, which takes about 10 us and 10 us per 1024 of K however few
+    tiles there are.  Measured (us, with the output's requantization, 256x256 /
+    t128): 4 x [4096, 4096] 62.6 / 11.8; 512 x [4096, 4096] 60 / 33; 1000 x
+    [2176, 2944] 50 / 34; 2048 x [2048, 2048] (64 tiles) 41 / 37; 4096 x [1024,
+    1024] (64 tiles) 31 / 32; 2048 x [4096, 4096] (128 tiles) 60 / 63."""
+    N, Kd = b.rows, b.k
+    tiles = -(-M // GEMM_TILE_ROWS) * -(-N // GEMM_TILE_ROWS)
+    if not (M <= 32 or (tiles <= 64 and Kd >= 32 * tiles)) or b.k_major or N % 8:
+        return False
+    brd, bsr, bsk, bkg = b.desc
+    rows4 = brd % 4 == 0 or (brd == 1 and bsr > 0 and bkg % (4 * bsr) == 0 and bsk % (4 * bsr) == 0)
+    return rows4 and a_kg & (a_kg - 1) == 0 and bkg & (bkg - 1) == 0
+
+
+def gemm_t128(a: Operand, b: Operand, out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
+    """``gemm_nt(a, b, out_dtype)`` on 128-row tiles with the K steps split over
+    workgroups (pratchya_gemm_bs_t128): for products of few 256 x 256 tiles.
+    ``PratchyaUnsupported`` for K-major operands and scale layouts it does not
+    take."""
+    _require_gpu(a.payload, b.payload)
+    if a.k != b.k:
+        raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
+    if a.k_major or b.k_major:
+        raise PratchyaUnsupported("gemm_t128: K-contiguous operands only")
+    M, N, Kd = a.rows, b.rows, a.k
+    ap, bp = _u8(a.payload).contiguous(), _u8(b.payload).contiguous()
+    as8, bs8 = _u8(a.sc8).contiguous(), _u8(b.sc8).contiguous()
+    as32, bs32 = a.sc32.contiguous().float(), b.sc32.contiguous().float()
+    lib = _lib.load()
+    c = torch.empty((M, N), dtype=out_dtype, device=ap.device)
+    ws_bytes = int(lib.pratchya_gemm_t128_workspace_bytes(M, N, Kd // 128))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=ap.device) if ws_bytes else None
+    _lib.check(lib.pratchya_gemm_bs_t128(_ptr(ap), Kd, _ptr(as8), _ptr(as32), *a.desc, _ptr(bp), Kd, _ptr(bs8),
+                                         _ptr(bs32), *b.desc, M, N, Kd, _ptr(c), N, _dtype_code(out_dtype),
+                                         _ptr(ws) if ws is not None else None, ws_bytes, _stream(ap)), "gemm_t128")
+    return c
 
 
 # bf16 piece pairs of an f32 product (see pratchya_split_pack_bf16): the six
@@ -797,7 +851,10 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
     n_rows = N if N >= GEMM_TILE_ROWS else (N + 3) // 4 * 4
     A = _split_pack(a, a_t, a_planes, kp)
     B = _split_pack(b, not b_t, b_planes, kp, n_rows)
-    c = gemm_bf16_nt(A, B, torch.float32)
+    if few_tiles(M, n_rows) and n_rows % 4 == 0:
+        c = gemm_planes(A[None], B[None], [(0, 0)], False)
+    else:
+        c = gemm_bf16_nt(A, B, torch.float32)
     return c if n_rows == N else c[:, :N]
 
 
@@ -835,16 +892,18 @@ def _nibbles(seq) -> int:
 
 
 def gemm_planes(a: torch.Tensor, b: torch.Tensor, pairs, k_major: bool, out_dtype=torch.float32, short: int = 0,
-                b_alt=None, flags=None, units=None) -> torch.Tensor:
+                b_alt=None, flags=None, units=None, x=None, b_k_major=None) -> torch.Tensor:
     """``sum over (i, j) in pairs of op(a[i]) @ op(b[j])^T`` for bf16 planes
     ``a`` [planes, M, K] and ``b`` [planes, N, K] (``k_major``: [planes, K, M] and
     [planes, K, N]) with f32 accumulation.  ``short`` pairs are enough where
     flags[0] is 0; ``b_alt`` are b's planes where flags[1] is not.  ``units``:
     ``(sc32, tgrid, blocks per group)`` of the payload that b is the power-of-two
-    plane of."""
+    plane of.  ``x`` [M, N] bf16: the result is ``1.5 x - 0.5 product`` in bf16
+    (``b_k_major``: b alone is K-major)."""
     _require_gpu(a, b)
+    b_km = k_major if b_k_major is None else b_k_major
     M, Kd = (int(a.shape[2]), int(a.shape[1])) if k_major else (int(a.shape[1]), int(a.shape[2]))
-    N = int(b.shape[2] if k_major else b.shape[1])
+    N = int(b.shape[2] if b_km else b.shape[1])
     lib = _lib.load()
     short = short or len(pairs)
     c = torch.empty((M, N), dtype=out_dtype, device=a.device)
@@ -855,10 +914,11 @@ def gemm_planes(a: torch.Tensor, b: torch.Tensor, pairs, k_major: bool, out_dtyp
         if units is not None else (None, 1, 1, 1)
     _lib.check(lib.pratchya_gemm_bf16_planes(
         _ptr(a), int(a.stride(1)), int(a.stride(0)), 1 if k_major else 0, int(a.shape[0]), pa,
-        _ptr(b), int(b.stride(1)), int(b.stride(0)), 1 if k_major else 0, int(b.shape[0]), pb,
+        _ptr(b), int(b.stride(1)), int(b.stride(0)), 1 if b_km else 0, int(b.shape[0]), pb,
         pb if b_alt is None else _nibbles(b_alt), M, N, Kd, len(pairs), short,
         _ptr(flags) if flags is not None else None, _ptr(g32) if g32 is not None else None, brow, bcol, kg,
-        _ptr(c), N, _dtype_code(out_dtype), None, 0, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
+        _ptr(c), N, _dtype_code(out_dtype), _ptr(x) if x is not None else None,
+        int(x.stride(0)) if x is not None else 0, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
         "gemm_planes")
     return c
 
@@ -1017,8 +1077,16 @@ def mfma_ceiling(a: torch.Tensor, b: torch.Tensor, bf16: bool, iters: int) -> in
     return int(flop.value)
 
 
+def _few_then_requantize(a: Operand, b: Operand, out_dtype, tgrid, fix_nan, lead):
+    """gemm_nt_fq / gemm_nt_q11 of a product of few tiles, as its two steps."""
+    lead = tuple(lead) if lead else (a.rows,)
+    c = gemm_t128(a, b, torch.float32)
+    y, s8, s32 = quantize_dequantize(c.view(lead + (b.rows,)), tgrid, out_dtype, fix_nan)
+    return y.view(a.rows, b.rows), s8, s32
+
+
 def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = False, lead=None,
-               status: torch.Tensor = None):
+               status: torch.Tensor = None, few: bool = False):
     """``QArrayImpl(dequant(a) @ dequant(b)^T, (1, 128)).astype(out_dtype)``
     with the requantization in the GEMM's epilogue: returns ``(y [M, N],
     sc_fp8, sc_fp32)`` bit-identical to ``quantize_dequantize(gemm_nt(a, b,
@@ -1027,13 +1095,18 @@ def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = F
     shaped per slice as quantize_impl returns them).  Raises
     ``PratchyaUnsupported`` unless N is a multiple of 1024 and B's scale
     groups span at least 32 rows.  ``status``: an int32 device tensor that
-    receives the strip exchange's status word (0: every wait completed)."""
+    receives the strip exchange's status word (0: every wait completed).
+    ``few``: a product of few tiles may run as gemm_t128 and
+    quantize_dequantize, whose sums are in another order."""
     _require_gpu(a.payload, b.payload)
     if a.k != b.k:
         raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
     if out_dtype not in (torch.float32, torch.bfloat16):
         raise ValueError(f"gemm_nt_fq: output dtype {out_dtype} is not float32 or bfloat16")
     M, N, K = a.rows, b.rows, a.k
+    if few and status is None and N % 1024 == 0 and b.desc[0] % 32 == 0 and not a.k_major \
+            and prefers_t128(M, a.desc[3], b):
+        return _few_then_requantize(a, b, out_dtype, (1, 128), fix_nan, lead)
     lib = _lib.load()
     ws_bytes = lib.pratchya_gemm_bs_nt_fq_workspace_bytes(M, N)
     if ws_bytes <= 0:
@@ -1058,13 +1131,14 @@ def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = F
     return y, sc8.view(E8M0), sc32
 
 
-def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None):
+def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None, few: bool = False):
     """``QArrayImpl(dequant(a) @ dequant(b)^T, (1, 1)).astype(out_dtype)``
     with the requantization in the GEMM's epilogue (the output grid of a
     weight quantized (a, 1): lm_head, LoRA): returns ``(y [M, N], sc_fp8,
     sc_fp32)`` bit-identical to ``quantize_dequantize(gemm_nt(a, b, float32),
     (1, 1), out_dtype)``, the scales shaped per slice of ``lead`` as there.
-    Raises ``PratchyaUnsupported`` unless N is a multiple of 16."""
+    Raises ``PratchyaUnsupported`` unless N is a multiple of 16.  ``few``: as
+    for gemm_nt_fq."""
     _require_gpu(a.payload, b.payload)
     if a.k != b.k:
         raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
@@ -1073,6 +1147,8 @@ def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None):
     M, N, K = a.rows, b.rows, a.k
     if N % 16:
         raise PratchyaUnsupported(f"gemm_q11: N must be a multiple of 16 (got {N})")
+    if few and not a.k_major and prefers_t128(M, a.desc[3], b):
+        return _few_then_requantize(a, b, out_dtype, (1, 1), False, lead)
     lib = _lib.load()
     ap, bp = _tile_readable(_u8(a.payload).contiguous()), _tile_readable(_u8(b.payload).contiguous())
     as8, bs8 = _word_readable(_u8(a.sc8).contiguous()), _word_readable(_u8(b.sc8).contiguous())

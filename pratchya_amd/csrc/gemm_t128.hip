@@ -82,6 +82,9 @@ __device__ __forceinline__ v8i join(v4i lo, v4i hi) { return v8i{lo.x, lo.y, lo.
 __device__ __forceinline__ void dma_kb(__amdgpu_buffer_rsrc_t rs, uint8_t* lds, uint32_t off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)lds, 16, off, 0, 0, 0);
 }
+__device__ __forceinline__ uint32_t load_word(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0);
+}
 __device__ __forceinline__ uint32_t load_byte(__amdgpu_buffer_rsrc_t rs, uint32_t i) {
   return __builtin_amdgcn_raw_buffer_load_b8(rs, (int)i, 0, 0);
 }
@@ -224,6 +227,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 
   // next step's e8m0 bytes and, at a span's start, group maxima
   uint32_t ea_n[MI], eb_n[NI];
+  const bool a_words = SC == 1 && p.a.sk2 == 2 && p.a.s_r % 4 == 0;
+  int a_shift = 0;
   float ga_n[MI], gb_n[NI][4];
   int seg = k_begin / p.spp, s = k_begin - seg * p.spp;
   int in_span = s % p.span;                // of the next step to load
@@ -239,8 +244,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
       dma_kb(rs_b, st + A_BYTES + (wave * 4 + i) * 1024, ob[i] + kb);
     if constexpr (SC == 1) {
       const uint32_t ta = (uint32_t)s * p.a.sk2 >> 1, tb = (uint32_t)s * p.b.sk2 >> 1;
+      // A's bytes of consecutive steps lie side by side: one aligned word holds
+      // four steps' where every row starts on a word
+      if (!a_words) {
 #pragma unroll
-      for (int i = 0; i < MI; ++i) ea_n[i] = load_byte(rs_ea, ra[i] + ta);
+        for (int i = 0; i < MI; ++i) ea_n[i] = load_byte(rs_ea, ra[i] + ta);
+      } else if (first || (s & 3) == 0) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) ea_n[i] = load_word(rs_ea, (ra[i] + ta) & ~3u);
+      }
+      a_shift = a_words ? (s & 3) * 8 : 0;
 #pragma unroll
       for (int i = 0; i < NI; ++i) eb_n[i] = load_byte(rs_eb, rb[i] + tb);
     }
@@ -324,7 +337,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
       uint32_t ea[MI], eb[NI];
       if constexpr (SC == 1) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) ea[i] = ea_n[i];
+        for (int i = 0; i < MI; ++i) ea[i] = ea_n[i] >> a_shift;
 #pragma unroll
         for (int i = 0; i < NI; ++i) eb[i] = eb_n[i];
       }

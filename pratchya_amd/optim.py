@@ -99,26 +99,37 @@ def newton_schulz(G: torch.Tensor, steps: int = 5) -> torch.Tensor:
     # is read K-major by it, with no transposed copy
     gram_side = npad if transpose else mp
     gram_ok = gram_side % 256 == 0
+    # Short of 256x256 tiles both products run on 128x128 tiles, the first in
+    # full (its triangles hold the same sums: symmetric bit for bit).  Measured
+    # (us, Gram kernel / 128x128 tiles): sides of 1024 58 / 30, 2048 (of 8192)
+    # 105 / 87, 4096 93 / 124; the combination in the epilogue alike
+    # ([1024, 4096] 34 / 28, [2048, 2048] 57 / 36, [2048, 8192] 69 / 80).
+    gram_few, ns_few = gram_side <= 2048, K.few_tiles(mp, npad)
     for _ in range(steps):
-        # the second product's epilogue also forms 1.5 X - 0.5 B (the bits
-        # of ns_combine), into a new buffer
-        if transpose:
-            if gram_ok:
-                A = K.gemm_bf16_gram(X, k_major=True)    # X^T X     [n, n]
-            else:
-                Xt = K.transpose_b16(X)                  # [n, m]
-                A = K.gemm_bf16_nt(Xt, Xt)
-            X = K.gemm_bf16_nt_ns(X, A, X)           # 1.5 X - 0.5 X A (A = A^T)
+        # A = X X^T [m, m], or X^T X [n, n] of a tall iterate
+        if gram_few:
+            A = K.gemm_planes(X[None], X[None], [(0, 0)], transpose, torch.bfloat16)
+        elif gram_ok:
+            A = K.gemm_bf16_gram(X, k_major=transpose)
+        elif transpose:
+            Xt = K.transpose_b16(X)
+            A = K.gemm_bf16_nt(Xt, Xt)
         else:
-            A = K.gemm_bf16_gram(X) if gram_ok else K.gemm_bf16_nt(X, X)   # X X^T [m, m]
-            # 1.5 X - 0.5 A X: a wide X is read K-major (no transposed copy);
-            # for a square one the copy is cheaper than the K-major read
-            # (measured: [4096, 4096] 1.08 vs 1.13 ms, [4096, 16384] 3.83 vs
-            # 3.74 ms for 5 iterations)
-            if npad > mp:
-                X = K.gemm_bf16_nt_ns(A, X, X, b_k_major=True)
-            else:
-                X = K.gemm_bf16_nt_ns(A, K.transpose_b16(X), X)
+            A = K.gemm_bf16_nt(X, X)
+        # 1.5 X - 0.5 A X, or 1.5 X - 0.5 X A (A = A^T): the second product's
+        # epilogue forms it (the bits of ns_combine), into a new buffer.  A wide
+        # X is read K-major (no transposed copy); for a square one of more
+        # tiles the copy is cheaper than the K-major read (measured: [4096,
+        # 4096] 1.08 vs 1.13 ms, [4096, 16384] 3.83 vs 3.74 ms for 5 iterations)
+        if ns_few:
+            a, b = (X, A) if transpose else (A, X)
+            X = K.gemm_planes(a[None], b[None], [(0, 0)], False, torch.bfloat16, x=X, b_k_major=not transpose)
+        elif transpose:
+            X = K.gemm_bf16_nt_ns(X, A, X)
+        elif npad > mp:
+            X = K.gemm_bf16_nt_ns(A, X, X, b_k_major=True)
+        else:
+            X = K.gemm_bf16_nt_ns(A, K.transpose_b16(X), X)
     return X[:m, :n].contiguous() if padded else X
 
 

@@ -312,7 +312,7 @@ def _try_gemm(op_a, op_b) -> Optional[torch.Tensor]:
     if op_a is None or op_b is None:
         return None
     try:
-        return K.gemm_nt(op_a, op_b, torch.float32)
+        return K.gemm_nt(op_a, op_b, torch.float32, few=True)
     except K.PratchyaUnsupported:
         return None
 
@@ -366,7 +366,7 @@ def _fp8_backward(g, x8, xs8, xs32, y8, ys8, ys32, gx, gy, need_x, need_y, pre=N
             op_w = K.operand_rows(y8, ys8, ys32, gy)          # W [K, N]: rows K, contraction N
             if x_dtype is not None and Kd % 1024 == 0:
                 try:
-                    gxf = K.gemm_nt_fq(op_g, op_w, x_dtype, fix_nan=True)[0]
+                    gxf = K.gemm_nt_fq(op_g, op_w, x_dtype, fix_nan=True, few=True)[0]
                     gx_final = True
                 except K.PratchyaUnsupported:
                     # the epilogue requantization takes B scale groups of 32
@@ -374,7 +374,7 @@ def _fp8_backward(g, x8, xs8, xs32, y8, ys8, ys32, gx, gy, need_x, need_y, pre=N
                     # the requantization as a separate pass
                     gxf = None
             if gxf is None:
-                gxf = K.gemm_nt(op_g, op_w, torch.float32)
+                gxf = K.gemm_nt(op_g, op_w, torch.float32, few=True)
             gxf = gxf.reshape(tuple(g.shape[:-1]) + (Kd,))
         if need_y and _wgrad_k_major and Kd <= _WGRAD_K_MAJOR_ROWS:
             # both operands requantized (128, 1) in their own [tokens, channels]
@@ -525,7 +525,8 @@ def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype):
     to the f32 product followed by ``quantize_dequantize``, or None when the
     layouts do not fit.  ``go`` (1, 128), a quantized Linear's output, takes
     N a multiple of 1024 (its groups span four output tiles); (1, 1), the
-    output of a weight quantized (a, 1) (lm_head, LoRA), N a multiple of 16."""
+    output of a weight quantized (a, 1) (lm_head, LoRA), N a multiple of 16.
+    (Products of few tiles run as the two steps: ``K.prefers_t128``.)"""
     go = tuple(go)
     if go not in ((1, 128), (1, 1)) or dtype not in (torch.float32, torch.bfloat16) or y8.dim() != 2:
         return None
@@ -539,9 +540,9 @@ def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype):
     lead = tuple(x8.shape[:-1])
     try:
         if go == (1, 1):
-            res, s8, s32 = K.gemm_nt_q11(op_a, op_b, dtype, lead=lead)
+            res, s8, s32 = K.gemm_nt_q11(op_a, op_b, dtype, lead=lead, few=True)
         else:
-            res, s8, s32 = K.gemm_nt_fq(op_a, op_b, dtype, lead=lead)
+            res, s8, s32 = K.gemm_nt_fq(op_a, op_b, dtype, lead=lead, few=True)
     except K.PratchyaUnsupported:
         return None
     return res.reshape(lead + (N,)), s8, s32
@@ -1181,9 +1182,13 @@ class _LazyProduct(QArrayImpl):
         if "_pending" not in xo.__dict__ or tuple(go) != (1, 128):
             return None
         y8, ys8, ys32 = yo._QArrayImpl__value, yo._QArrayImpl__sc_fp8, yo._QArrayImpl__sc_fp32
-        if y8.dim() != 2 or int(y8.shape[1]) % 1024 or _rhs_operand(y8, ys8, ys32, gy) is None:
+        if y8.dim() != 2 or int(y8.shape[1]) % 1024:
             return None
         x = xo._pending
+        op_b = _rhs_operand(y8, ys8, ys32, gy)
+        # (a product of few tiles runs as it does without the prologue)
+        if op_b is None or K.prefers_t128(x.numel() // int(x.shape[-1]), 8, op_b):
+            return None
         with torch.set_grad_enabled(self._grad_enabled):
             sx = x if (x.requires_grad and torch.is_grad_enabled()) else None
             sy = _src(y8)

@@ -99,3 +99,59 @@ def test_planes_sum_to_the_value():
     flags.zero_()
     K.planes(K.PLANE_SPLIT3, *K.quantize(x.to(torch.bfloat16), (1, 32)), (1, 32), flags)
     assert flags.tolist() == [0, 0]              # bf16 group maxima: no third piece
+
+
+@pytest.mark.parametrize("M,N,Kd,grid", [
+    (1, 256, 128, (128, 128)), (32, 1024, 4096, (128, 128)), (33, 384, 640, (128, 128)), (7, 512, 2176, (128, 1)),
+    (129, 272, 2176, (128, 8)), (300, 2944, 512, (128, 1)), (512, 1024, 1152, (128, 64))])
+def test_fp8_product(M, N, Kd, grid):
+    """gemm_t128 on (1, 128) activations and weight grids whose group maxima
+    change along K, against the 256x256 kernel (the same MFMAs, summed in
+    another order: f32 rounding, bound as above) and float64 (the f32 tolerance
+    of the FP8 GEMM tests)."""
+    K = _K()
+    x = _randn((M, Kd), 1) * torch.exp(2 * _randn((M, 1), 2))
+    w = _randn((Kd, N), 3, scale=0.02) * torch.exp(_randn((Kd, N), 4))
+    xq, wq = K.quantize(x, (1, 128)), K.quantize(w, grid)
+    a, b = K.operand_rows(*xq, (1, 128)), K.operand_transposed(*wq, grid)
+    ref = K.dequantize(*xq, torch.float32, (1, 128)).double() @ K.dequantize(*wq, torch.float32, grid).double()
+    c = K.gemm_t128(a, b, torch.float32)
+    assert _rel(c, ref) <= 1e-3 and _rel(c, K.gemm_nt(a, b, torch.float32).double()) <= TOL
+    assert _rel(K.gemm_t128(a, b, torch.bfloat16), c.double()) <= 2.0 ** -8
+    if grid[1] % 128 == 0:                        # as the weight's rows (dgrad): group maxima per 128 rows
+        g = K.quantize(_randn((M, N), 5), (1, 128))
+        op_w = K.operand_rows(*wq, grid)
+        og = K.operand_rows(*g, (1, 128))
+        if N % 128 == 0:
+            assert _rel(K.gemm_t128(og, op_w, torch.float32), K.gemm_nt(og, op_w, torch.float32).double()) <= TOL
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 200])
+@pytest.mark.parametrize("grid,N", [((128, 128), 1024), ((128, 1), 528)])
+def test_linear_of_few_rows(rows, grid, N):
+    """A Linear of few rows (fused requantization asked for, the product on
+    gemm_t128): the same output as its steps."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    x, w = _randn((rows, 2048), 1, torch.bfloat16), _randn((2048, N), 2, torch.bfloat16, 0.02)
+    W = Q.QArrayImpl(w, grid)
+    y = (Q.QArrayImpl(x, (1, 128)) @ W).astype(torch.bfloat16)
+    xq = K.quantize(x, (1, 128))
+    c = K.gemm_t128(K.operand_rows(*xq, (1, 128)), K.operand_transposed(*W._tree_flatten()[0], grid), torch.float32)
+    assert torch.equal(y, K.quantize_dequantize(c, (1, grid[1]), torch.bfloat16)[0])
+
+
+@pytest.mark.parametrize("shape", [(64, 64), (256, 512), (320, 1024), (1024, 192), (2048, 2304), (2304, 2048)])
+def test_newton_schulz_of_few_tiles(shape):
+    """Sides at the dispatch's edges against the same iteration in float64 (the
+    bf16 tolerance of the optimizer tests)."""
+    from pratchya_amd.optim import newton_schulz
+    g = _randn(shape, 1, torch.bfloat16)
+    x = g.double() / g.double().norm()
+    x = x.T if shape[0] > shape[1] else x
+    for _ in range(5):
+        x = 1.5 * x - 0.5 * (x @ x.T) @ x
+    assert _rel(newton_schulz(g), x.T if shape[0] > shape[1] else x) <= 3e-2
+    K = _K()
+    a = K.gemm_planes(g[None], g[None], [(0, 0)], False, torch.bfloat16)
+    assert torch.equal(a, a.T)
