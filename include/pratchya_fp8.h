@@ -525,6 +525,17 @@ int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_stride, int 
                               int64_t b_bcol, int64_t b_kg, void* C, int64_t ldc, int c_dtype, const void* X,
                               int64_t ldx, void* ws, int64_t ws_bytes, hipStream_t stream);
 
+/* f32 C [M, N] = dequant(x) . dequant(W) to f32 accuracy (Q:605-608) for x
+ * quantized (1, blk) and W [K, N] quantized (blk, blk), blk 16 or 32 (the
+ * presets' grids): A [M, K] and B [K, N] are their mode 0 planes
+ * (pratchya_planes), a_sc32 and b_sc32 their group maxima (x: one block of 16 or
+ * two of 32 per group; W: b_kg blocks), whose mantissas multiply each block's
+ * exact f32 sums.  K a multiple of 64, N of blk.  ws: partials of
+ * pratchya_gemm_t128_workspace_bytes(M, N, K / 64) bytes. */
+int pratchya_gemm_fine(const void* A, int64_t lda, const float* a_sc32, const void* B, int64_t ldb, const float* b_sc32,
+                       int64_t b_kg, int64_t blk, int64_t M, int64_t N, int64_t K, float* C, int64_t ldc, void* ws,
+                       int64_t ws_bytes, hipStream_t stream);
+
 /* bf16 planes [planes][T_pad][W] of a row-major [T, W] matrix quantized (a, b)
  * (rows T .. T_pad zeros; W and b multiples of 8, b a power of two):
  *   0 payload -> its power-of-two plane f32(q) * (2^(e-127) * 2^floor(log2 G)) / 128

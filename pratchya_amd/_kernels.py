@@ -923,6 +923,27 @@ def gemm_planes(a: torch.Tensor, b: torch.Tensor, pairs, k_major: bool, out_dtyp
     return c
 
 
+def gemm_fine(a: torch.Tensor, a_sc32: torch.Tensor, b: torch.Tensor, b_sc32: torch.Tensor, b_kg: int,
+              blk: int) -> torch.Tensor:
+    """f32 ``dequant(x) @ dequant(W)`` to f32 accuracy for x [M, K] quantized
+    (1, blk) and W [K, N] quantized (blk, blk), blk 16 or 32, given as their
+    power-of-two planes ``a`` and ``b`` and group maxima (W with ``b_kg`` blocks
+    per group)."""
+    _require_gpu(a, b)
+    M, Kd, N = int(a.shape[0]), int(a.shape[1]), int(b.shape[1])
+    lib = _lib.load()
+    ag, bg = a_sc32.contiguous().float(), b_sc32.contiguous().float()
+    if ag.numel() != M * Kd // (16 if blk == 16 else 64):
+        raise PratchyaUnsupported("gemm_fine: x's groups are not one block of 16 or two of 32")
+    c = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    ws_bytes = int(lib.pratchya_gemm_t128_workspace_bytes(M, N, Kd // 64))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+    _lib.check(lib.pratchya_gemm_fine(_ptr(a), int(a.stride(0)), _ptr(ag), _ptr(b), int(b.stride(0)), _ptr(bg), b_kg, blk,
+                                      M, N, Kd, _ptr(c), N, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
+               "gemm_fine")
+    return c
+
+
 def transpose_b16(x: torch.Tensor) -> torch.Tensor:
     """[rows, cols] 16-bit matrix -> its transpose [cols, rows], contiguous."""
     _require_gpu(x)

@@ -114,6 +114,8 @@ SIGNATURES = {
                                            _c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32, ctypes.c_uint32,
                                            _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_p, _c_p, _c_i64, _c_i64,
                                            _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p, _c_i64, _c_p]),
+    "pratchya_gemm_fine": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                    _c_p, _c_i64, _c_p, _c_i64, _c_p]),
     "pratchya_planes": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "pratchya_gemm_span": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
     "pratchya_transpose_u8": (_c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),

@@ -92,6 +92,10 @@ __device__ __forceinline__ float load_f32(__amdgpu_buffer_rsrc_t rs, uint32_t i)
   return u2f(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(i * 4u), 0, 0));
 }
 
+__device__ __forceinline__ v4f load_f32x4(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+}
+
 // K-major bf16 fragment of 32 operand rows (see the K-major operand of
 // gemm.hip): the stage holds 64 K rows of 256 bytes, 16-byte chunks
 // XOR-swizzled by 4 * (k mod 4).
@@ -101,8 +105,9 @@ __device__ __forceinline__ v4i tr_pair(const uint8_t* p0, const uint8_t* p1) {
   const v2i x = __builtin_bit_cast(v2i, a), y = __builtin_bit_cast(v2i, b);
   return v4i{x.x, x.y, y.x, y.y};
 }
+template <int SECOND>                      // K row of the second MFMA's values
 __device__ __forceinline__ v8i read_frag_tn(const uint8_t* base) {
-  return join(tr_pair(base, base + 4 * 256), tr_pair(base + 8 * 256, base + 12 * 256));
+  return join(tr_pair(base, base + 4 * 256), tr_pair(base + SECOND * 256, base + (SECOND + 4) * 256));
 }
 
 // The mantissa of a group maximum, in [1, 2) ([0, 1) for a subnormal one): the
@@ -137,7 +142,12 @@ __device__ __forceinline__ void wg_barrier() {
 
 // OUT 0: f32, 1: bf16, 2: bf16 1.5 X - 0.5 C.  SC 0: no scales, 1: FP8, both
 // operands' e8m0 bytes and group maxima, 2: bf16, the mantissas of B's group
-// maxima.  flags (bf16): flags[0] == 0 says that the planes of the segments
+// maxima, 3 and 4: bf16 power-of-two planes of payloads quantized in blocks of
+// 16 or 32 along K, the mantissas of both operands' group maxima per block: an
+// MFMA's sums over one block (two MFMAs' over 32) join the total times both.
+// These two are bound by the multiply-adds that join them (16 per lane and
+// MFMA, 64 clocks beside its 32): 8192 x [4096, 4096] 402 us in blocks of 32
+// and 508 in blocks of 16, where the six-pair f32 product took 1585.  flags (bf16): flags[0] == 0 says that the planes of the segments
 // past segs_short are all zero (the segments are left out); flags[1] != 0 that
 // B's plane 0 holds non-finite values, which may take part in the first
 // segment only (0 * inf): the others then read planes_alt, a copy without.
@@ -149,6 +159,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   constexpr int WN = NI * 32;                            // columns of a wave
   constexpr int A_BYTES = TM * KB, STAGE = A_BYTES + TN * KB;
   constexpr int NA = TM / 32;                            // A DMA instructions per wave and stage
+  constexpr bool FINE = SC >= 3;
+  // The next stage's DMA goes out between the first half's MFMAs where the step
+  // is bound by its fragment reads, which it would hold up (FP8 2048 x [4096,
+  // 4096] 52 -> 48 us, blocks of 16 8192 x [4096, 4096] 549 -> 523), else at
+  // once, for the longest lead (bf16 [4096, 2048] . [2048, 8192]: 134, late 147)
+  constexpr bool LATE = SC == 1 || SC == 3;
+  constexpr int FB = SC == 3 ? 16 : 32, KBS = 64 / FB;   // block size, blocks of a step
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * STAGE];
 
   const int lane = threadIdx.x & 63;
@@ -217,7 +234,19 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) rb[i] = (uint32_t)(n0 + wn * WN + i * 32 + l32) / p.b.r_div * p.b.s_r;
   }
-  if constexpr (SC != 0) {
+  // Fine blocks: A's mantissas of a step are one row's KBS (16) or one (32: two
+  // blocks share a group) consecutive group maxima; the wave's of B, one per
+  // block of K and of its columns, are loaded one per lane and handed out as
+  // scalars.
+  uint32_t fa_row[MI];
+  const int fq_k = lane / (WN / FB) % KBS, fq_n = lane % (WN / FB);
+  uint32_t fb_n = 0;
+  if constexpr (FINE) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) fa_row[i] = (uint32_t)(m0 + wm * 64 + i * 32 + l32) * (uint32_t)p.spp * (SC == 3 ? 16u : 4u);
+    fb_n = (uint32_t)(n0 + wn * WN) / FB + (uint32_t)fq_n;
+  }
+  if constexpr (SC == 1 || SC == 2) {
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -227,21 +256,26 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 
   // next step's e8m0 bytes and, at a span's start, group maxima
   uint32_t ea_n[MI], eb_n[NI];
+  v4f fa_n[MI];
+  float fb_g = 1.0f;
   const bool a_words = SC == 1 && p.a.sk2 == 2 && p.a.s_r % 4 == 0;
   int a_shift = 0;
   float ga_n[MI], gb_n[NI][4];
   int seg = k_begin / p.spp, s = k_begin - seg * p.spp;
   int in_span = s % p.span;                // of the next step to load
   bool start_n = true;                     // the loaded step starts a span (or the slice)
+  uint8_t* dma_st = lds;
+  uint32_t dma_ka = 0, dma_kb_ = 0;
+  auto dma = [&](int i) {                  // instruction i of the stage's load
+    if (i < NA) dma_kb(rs_a, dma_st + (wave * NA + i) * 1024, oa[i] + dma_ka);
+    else dma_kb(rs_b, dma_st + A_BYTES + (wave * 4 + i - NA) * 1024, ob[i - NA] + dma_kb_);
+  };
   auto load_stage = [&](uint8_t* st, bool first) {
     const uint32_t ka = ((planes_a >> (4 * seg)) & 15u) * p.a.pstride + (uint32_t)s * step_a;
     const uint32_t kb = ((planes_b >> (4 * seg)) & 15u) * p.b.pstride + (uint32_t)s * step_b;
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-      dma_kb(rs_a, st + (wave * NA + i) * 1024, oa[i] + ka);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      dma_kb(rs_b, st + A_BYTES + (wave * 4 + i) * 1024, ob[i] + kb);
+    dma_st = st;
+    dma_ka = ka;
+    dma_kb_ = kb;
     if constexpr (SC == 1) {
       const uint32_t ta = (uint32_t)s * p.a.sk2 >> 1, tb = (uint32_t)s * p.b.sk2 >> 1;
       // A's bytes of consecutive steps lie side by side: one aligned word holds
@@ -257,7 +291,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) eb_n[i] = load_byte(rs_eb, rb[i] + tb);
     }
-    if constexpr (SC != 0) {
+    if constexpr (FINE) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if constexpr (SC == 3) fa_n[i] = load_f32x4(rs_ga, fa_row[i] + (uint32_t)s * 16u);
+        else fa_n[i].x = load_f32(rs_ga, (fa_row[i] >> 2) + (uint32_t)s);
+      }
+      fb_g = load_f32(rs_gb, (((uint32_t)s * KBS + (uint32_t)fq_k) * p.b.s_r + fb_n) >> p.b.kg_sh);
+    }
+    if constexpr (SC == 1 || SC == 2) {
       start_n = first || in_span == 0;
       if (start_n) {
         const uint32_t ta = (uint32_t)s * p.a.sk2 >> 1, tb = (uint32_t)s * p.b.sk2 >> 1;
@@ -294,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   // payloads)
   float ua[MI], ub[NI][4];
   auto flush = [&]() {
-    if constexpr (SC != 0) {
+    if constexpr (SC == 1 || SC == 2) {
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
@@ -314,14 +356,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) ch[ks][h] = ((ks * 4 + lhi * 2 + h) ^ sw) << 4;
+      for (int h = 0; h < 2; ++h) ch[ks][h] = ((ks * 4 + (FINE ? h * 2 + lhi : lhi * 2 + h)) ^ sw) << 4;
   }
   const int g16 = lane >> 4, j16 = lane & 15;
-  const int tn_kc = (16 * (g16 >> 1) + (j16 >> 2)) * 256 + (2 * (g16 & 1) + ((j16 & 3) >> 1)) * 16 + (j16 & 1) * 8;
+  // (fine blocks: an MFMA's 16 K values are consecutive, so that they are one
+  // block's: lanes 32-63 hold its upper 8)
+  const int tn_kc = ((FINE ? 8 : 16) * (g16 >> 1) + (j16 >> 2)) * 256 + (2 * (g16 & 1) + ((j16 & 3) >> 1)) * 16 + (j16 & 1) * 8;
   const int tn_s = j16 >> 2;
   // a 32-row block of 128-byte rows keeps a row's swizzle (it depends on l32)
   auto frag = [&](const uint8_t* base, auto tn, int blk, int ks) {
-    if constexpr (decltype(tn)::value) return read_frag_tn(base + tn_kc + ks * 32 * 256 + ((blk ^ tn_s) << 6));
+    if constexpr (decltype(tn)::value)
+      return read_frag_tn<FINE ? 16 : 8>(base + tn_kc + ks * 32 * 256 + ((blk ^ tn_s) << 6));
     else {
       const uint8_t* r = base + (blk * 32 + l32) * KB;
       return join(*reinterpret_cast<const v4i*>(r + ch[ks][0]), *reinterpret_cast<const v4i*>(r + ch[ks][1]));
@@ -330,6 +375,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 
   if (k_begin < k_end) {
     load_stage(lds, true);
+#pragma unroll
+    for (int i = 0; i < NA + 4; ++i) dma(i);
     for (int k = k_begin; k < k_end; ++k) {
       uint8_t* st = lds + ((k - k_begin) & 1) * STAGE;
       PINNED_WAITCNT(0);                   // this wave's share of stage k (and its reads of stage k - 1) is done
@@ -341,7 +388,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) eb[i] = eb_n[i];
       }
-      if constexpr (SC != 0) {
+      float um[MI][4], un[FINE ? KBS * (WN / FB) : 1];
+      if constexpr (FINE) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < (SC == 3 ? 4 : 1); ++j) um[i][j] = mantissa_unit(fa_n[i][j]);
+        const float b = mantissa_unit(fb_g);
+#pragma unroll
+        for (int i = 0; i < KBS * (WN / FB); ++i) un[i] = u2f(readlane_u32(f2u(b), i));
+      }
+      if constexpr (SC == 1 || SC == 2) {
         if (start_n) {
           if (k != k_begin) flush();
 #pragma unroll
@@ -353,7 +410,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
             for (int j = 0; j < 4; ++j) ub[i][j] = SC == 1 ? gb_n[i][j] * 0.0078125f : mantissa_unit(gb_n[i][j]);
         }
       }
-      if (k + 1 < k_end) load_stage(lds + ((k - k_begin + 1) & 1) * STAGE, false);
+      const bool more = k + 1 < k_end;
+      if (more) {
+        load_stage(lds + ((k - k_begin + 1) & 1) * STAGE, false);
+        if (!LATE) {
+#pragma unroll
+          for (int i = 0; i < NA + 4; ++i) dma(i);
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
@@ -366,7 +430,29 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
           for (int ni = 0; ni < NI; ++ni) {
-            if constexpr (BF) {
+            if constexpr (FINE) {
+              const v8i a = fb[ni], b = fa[mi];
+              const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3});
+              const bf16x8_t b0 = __builtin_bit_cast(bf16x8_t, v4i{b.s0, b.s1, b.s2, b.s3});
+              const bf16x8_t a1 = __builtin_bit_cast(bf16x8_t, v4i{a.s4, a.s5, a.s6, a.s7});
+              const bf16x8_t b1 = __builtin_bit_cast(bf16x8_t, v4i{b.s4, b.s5, b.s6, b.s7});
+              v16f c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, v16f{0}, 0, 0, 0);
+              if constexpr (SC == 3) {
+                const v16f d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, v16f{0}, 0, 0, 0);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                  const int kb = ks * 2 + h;
+                  const float u0 = um[mi][kb] * un[kb * (WN / FB) + ni * 2], u1 = um[mi][kb] * un[kb * (WN / FB) + ni * 2 + 1];
+#pragma unroll
+                  for (int v = 0; v < 16; ++v) tot[mi][ni][v] += (h ? d[v] : c[v]) * (v < 8 ? u0 : u1);
+                }
+              } else {
+                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, c, 0, 0, 0);
+                const float u = um[mi][0] * un[ks * (WN / FB) + ni];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) tot[mi][ni][v] += c[v] * u;
+              }
+            } else if constexpr (BF) {
               const v8i a = fb[ni], b = fa[mi];
               acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                   __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3}),
@@ -377,6 +463,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
             } else {
               acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[ni], fa[mi], acc[mi][ni], 0, 0, 0,
                                                                            (int)eb[ni], 0, (int)ea[mi]);
+            }
+            if (LATE && ks == 0) {
+              constexpr int PER = (NA + 4 + MI * NI - 1) / (MI * NI);
+              __builtin_amdgcn_sched_barrier(0);
+              if (more) {
+#pragma unroll
+                for (int i = (mi * NI + ni) * PER; i < (mi * NI + ni + 1) * PER && i < NA + 4; ++i) dma(i);
+              }
+              __builtin_amdgcn_sched_barrier(0);
             }
           }
       }
@@ -721,6 +816,58 @@ extern "C" int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_s
   } else {
     if (bf) t128_launch<true, 128, false, false, 0, 1>(p, stream);
     else t128_launch<true, 128, false, false, 0, 0>(p, stream);
+  }
+  return t128_status(who);
+}
+
+extern "C" int pratchya_gemm_fine(const void* A, int64_t lda, const float* a_sc32, const void* B, int64_t ldb,
+                                  const float* b_sc32, int64_t b_kg, int64_t blk, int64_t M, int64_t N, int64_t K,
+                                  float* C, int64_t ldc, void* ws, int64_t ws_bytes, hipStream_t stream) {
+  const char* who = "gemm_fine";
+  if (M <= 0 || N <= 0 || K <= 0) {
+    if (M < 0 || N < 0 || K < 0) return pratchya_set_error(PRATCHYA_EINVAL, "%s: negative size", who);
+    return PRATCHYA_OK;
+  }
+  const int sh = ilog2_exact(b_kg);
+  if ((blk != 16 && blk != 32) || K % 64 || N % blk || sh < 0)
+    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: blocks of 16 or 32, K a multiple of 64, groups of a power of two "
+                              "of blocks", who);
+  if (!A || !B || !a_sc32 || !b_sc32 || !C) return pratchya_set_error(PRATCHYA_EINVAL, "%s: null buffer", who);
+  if (lda < K || ldb < N || ldc < N || lda % 8 || ldb % 8 || ldc % 4 ||
+      (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C) |
+       reinterpret_cast<uintptr_t>(a_sc32)) % 16)
+    return pratchya_set_error(PRATCHYA_EINVAL, "%s: leading dimensions / alignment not supported", who);
+  const int64_t Mr = (M + 127) / 128 * 128, Nr = (N + 127) / 128 * 128, nbn = N / blk;
+  if (2 * (Mr * lda + K) > kMaxOffset || 2 * ((K + 1) * ldb + Nr) > kMaxOffset || Mr * (K / 4) > kMaxOffset ||
+      (K / blk + 1) * nbn > INT32_MAX / 4 || M > INT32_MAX / 2 || N > INT32_MAX / 2 || K > (1 << 26))
+    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: operands beyond 32-bit offsets", who);
+  T128Args p{};
+  p.a.p = static_cast<const uint8_t*>(A);
+  p.a.ld = (uint32_t)(2 * lda);
+  p.a.bytes = (uint32_t)(2 * ((M - 1) * lda + K));
+  p.a.g32 = a_sc32;
+  p.a.g32_bytes = (uint32_t)(M * (K / (blk == 16 ? 16 : 64)) * 4);
+  p.a.r_div = p.b.r_div = 1;
+  p.b.p = static_cast<const uint8_t*>(B);
+  p.b.ld = (uint32_t)(2 * ldb);
+  p.b.bytes = (uint32_t)(2 * ((K - 1) * ldb + N));
+  p.b.g32 = b_sc32;
+  p.b.g32_bytes = (uint32_t)((((K / blk) * nbn - 1) / b_kg + 1) * 4);
+  p.b.s_r = (uint32_t)nbn;
+  p.b.kg_sh = (uint32_t)sh;
+  p.C = C;
+  p.ldc = ldc;
+  p.spp = p.span = (int)(K / 64);
+  p.segs = p.segs_short = 1;
+  const int rc = t128_shape(who, &p, M, N, p.spp, ws, ws_bytes);
+  if (rc) return rc;
+  const bool small = t128_rows(M) == 32;
+  if (blk == 16) {
+    if (small) t128_launch<true, 32, false, true, 3, 0>(p, stream);
+    else t128_launch<true, 128, false, true, 3, 0>(p, stream);
+  } else {
+    if (small) t128_launch<true, 32, false, true, 4, 0>(p, stream);
+    else t128_launch<true, 128, false, true, 4, 0>(p, stream);
   }
   return t128_status(who);
 }

@@ -317,15 +317,34 @@ def _try_gemm(op_a, op_b) -> Optional[torch.Tensor]:
         return None
 
 
+def _fine_forward(x8, xs8, xs32, y8, ys8, ys32, gx, gy):
+    """f32 product of x quantized (1, b) and y (b, b), b 16 or 32, on the
+    fine-block kernel, or None for other layouts."""
+    blk = int(gx[1])
+    if blk not in (16, 32) or tuple(gx) != (1, blk) or tuple(gy) != (blk, blk) or y8.dim() != 2 or x8.dim() < 2:
+        return None
+    Kd = int(y8.shape[0])
+    if Kd % 64 or x8.numel() == 0 or int(x8.shape[-1]) != Kd or not _flat_scales(tuple(x8.shape), gx):
+        return None
+    try:
+        a = K.planes(K.PLANE_POW2, x8.reshape(-1, Kd), xs8, xs32, gx)[0]
+        b = K.planes(K.PLANE_POW2, y8, ys8, ys32, gy)[0]
+        return K.gemm_fine(a, xs32, b, ys32, K.group_layout(Kd, int(y8.shape[1]), gy)[1], blk)
+    except K.PratchyaUnsupported:
+        return None
+
+
 def _matmul_forward(x8, xs8, xs32, y8, ys8, ys32, gx, gy) -> torch.Tensor:
     """f32 dequant(x) @ dequant(y) (Q:605-608): the FP8 MFMA GEMM for every
     (a, 128) x (128, b) pair of block grids (any M, N; K a multiple of 128);
-    grids whose blocks are not 128 wide along K (blksize 16 / 32 presets)
-    take the reference's own f32 dot of the operands dequantized by the
-    kernels."""
+    (1, 16) x (16, 16) and (1, 32) x (32, 32) (the blksize 16 / 32 presets) take
+    the fine-block kernel, to f32 accuracy; other grids the reference's own f32
+    dot of the operands dequantized by the kernels."""
     op_a = _lhs_operand(x8, xs8, xs32, gx)
     op_b = _rhs_operand(y8, ys8, ys32, gy) if op_a is not None else None
     out = _try_gemm(op_a, op_b)
+    if out is None:
+        out = _fine_forward(x8, xs8, xs32, y8, ys8, ys32, gx, gy)
     if out is not None:
         return out.reshape(tuple(x8.shape[:-1]) + (int(y8.shape[1]),))
     return _mm_f32(_deq32(x8, xs8, xs32, gx), _deq32(y8, ys8, ys32, gy))

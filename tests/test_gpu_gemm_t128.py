@@ -155,3 +155,51 @@ def test_newton_schulz_of_few_tiles(shape):
     K = _K()
     a = K.gemm_planes(g[None], g[None], [(0, 0)], False, torch.bfloat16)
     assert torch.equal(a, a.T)
+
+
+@pytest.mark.parametrize("rows,Kd,N,blk,dtype", [
+    (1, 64, 16, 16, torch.bfloat16), (32, 128, 640, 16, torch.bfloat16), (33, 192, 96, 32, torch.bfloat16),
+    (129, 576, 2944, 16, torch.float32), (300, 1088, 352, 32, torch.float32), (520, 4096, 128, 16, torch.bfloat16)])
+def test_fine_block_product(rows, Kd, N, blk, dtype):
+    """The forward product of blocks of 16 and 32 against float64, group maxima
+    of very different sizes, groups of the weight that straddle its block rows
+    (2944 / 16 = 184 blocks), 3-D activations, and rows of zeros, inf and NaN."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    x = (_randn((rows, Kd), 1) * torch.exp(3 * _randn((rows, Kd // blk), 2)).repeat_interleave(blk, 1)).to(dtype)
+    w = (_randn((Kd, N), 3) * torch.exp(_randn((Kd, N), 4)) * 0.02).to(dtype)
+    xq, wq = K.quantize(x, (1, blk)), K.quantize(w, (blk, blk))
+    xd, wd = K.dequantize(*xq, torch.float32, (1, blk)), K.dequantize(*wq, torch.float32, (blk, blk))
+    c = Q._fine_forward(*xq, *wq, (1, blk), (blk, blk))
+    assert _rel(c, xd.double() @ wd.double()) <= TOL
+    if rows % 3 == 0:
+        x3 = K.quantize(x.view(3, rows // 3, Kd), (1, blk))
+        assert torch.equal(Q._matmul_forward(*x3, *wq, (1, blk), (blk, blk)).view(rows, N), c)
+    if rows > 4:
+        x[0], x[1, 3], x[2, 5], x[3, 7] = 0.0, float("inf"), float("nan"), 3e38
+        xq = K.quantize(x, (1, blk))
+        c = Q._fine_forward(*xq, *wq, (1, blk), (blk, blk))
+        ref = K.matmul_f32(K.dequantize(*xq, torch.float32, (1, blk)), wd)
+        assert torch.equal(torch.isfinite(c), torch.isfinite(ref)) and not c[0].any()
+
+
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("tgrid", [(1, 8), (1, 16), (1, 32), (1, 64)])
+@pytest.mark.parametrize("out", ["bfloat16", "float32"])
+@pytest.mark.parametrize("fix_nan", [False, True])
+def test_fake_quantization_of_narrow_row_blocks(xdt, tgrid, out, fix_nan):
+    """The one-pass fake quantization of (1, b) grids, bit for bit against the
+    oracle on the edge values (zeros, clamped groups, overflow, NaN, inf,
+    subnormals, quotients next to bf16 midpoints) and on a partial last wave."""
+    import numpy as np
+
+    from oracle import qarr_oracle as O
+    from tests.helpers import to_dev_bf16, to_dev_f32
+    from tests.test_gpu_qdq import check, edge_tensor
+    x = edge_tensor(xdt)
+    dev = to_dev_bf16(O.f32_to_bf16_bits(x)) if xdt == "bf16" else to_dev_f32(x)
+    check(dev, x, tgrid, out, fix_nan, f"edge {xdt} {tgrid}->{out} fix {fix_nan}")
+    y = np.random.default_rng(3).standard_normal((5, 192)).astype(np.float32)
+    y = O.bf16_round(y) if xdt == "bf16" else y
+    dev = to_dev_bf16(O.f32_to_bf16_bits(y)) if xdt == "bf16" else to_dev_f32(y)
+    check(dev, y, tgrid, out, fix_nan, f"ragged {xdt} {tgrid}->{out} fix {fix_nan}")
