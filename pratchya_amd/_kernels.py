@@ -6,6 +6,7 @@ the current stream of the tensor's device; there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Tuple
 
@@ -18,12 +19,21 @@ E4M3 = torch.float8_e4m3fn
 E8M0 = torch.float8_e8m0fnu
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+# The wrappers' own time is what a small call costs (a Linear of 4 tokens: 69
+# us for 12 us of kernels), so they take addresses and the current stream as
+# plain integers, allocate outputs in their own dtypes and keep the layouts of
+# shapes they have seen.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
+
+
+def _stream(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.device.index)
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _require_gpu(*ts: torch.Tensor) -> None:
@@ -55,14 +65,29 @@ def slices_hw(shape) -> Tuple[int, int, int]:
     return s, shape[-2], shape[-1]
 
 
-def group_layout(H: int, W: int, tgrid) -> Tuple[int, int, int]:
-    """(n_blk, K, M) of one [H, W] slice (pratchya/_qualia/_qarr.py:474-480)."""
+@functools.lru_cache(maxsize=4096)
+def _group_layout(H: int, W: int, a: int, b: int) -> Tuple[int, int, int]:
     lib = _lib.load()
     n_blk, K, M = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
-    _lib.check(lib.pratchya_quant_layout(H, W, int(tgrid[0]), int(tgrid[1]),
-                                         ctypes.byref(n_blk), ctypes.byref(K), ctypes.byref(M)),
+    _lib.check(lib.pratchya_quant_layout(H, W, a, b, ctypes.byref(n_blk), ctypes.byref(K), ctypes.byref(M)),
                "quantize layout")
     return n_blk.value, K.value, M.value
+
+
+def group_layout(H: int, W: int, tgrid) -> Tuple[int, int, int]:
+    """(n_blk, K, M) of one [H, W] slice (pratchya/_qualia/_qarr.py:474-480)."""
+    return _group_layout(int(H), int(W), int(tgrid[0]), int(tgrid[1]))
+
+
+@functools.lru_cache(maxsize=4096)
+def _ws_bytes_of(query: str, device: int, *sizes: int) -> int:
+    return int(getattr(_lib.load(), query)(*sizes))
+
+
+def _ws_bytes(query: str, *sizes: int) -> int:
+    """A workspace query of the library (they depend on the sizes and on the
+    device's compute units only)."""
+    return _ws_bytes_of(query, torch.cuda.current_device(), *sizes)
 
 
 def _aligned(t: torch.Tensor, n: int) -> bool:
@@ -99,21 +124,21 @@ def quantize(x: torch.Tensor, tgrid, out=None) -> Tuple[torch.Tensor, torch.Tens
     if not x.is_contiguous() or not _aligned(x, 16):
         x = x.contiguous() if not x.is_contiguous() else x.clone()
     if out is None:
-        x8 = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-        sc8 = torch.empty(lead + (M, K), dtype=torch.uint8, device=x.device)
+        x8 = torch.empty(x.shape, dtype=E4M3, device=x.device)
+        sc8 = torch.empty(lead + (M, K), dtype=E8M0, device=x.device)
         sc32 = torch.empty(lead + (M, 1, 1), dtype=torch.float32, device=x.device)
     else:
         _check_out(out, [(x.shape, 1), (lead + (M, K), 1), (lead + (M, 1, 1), 4)], "quantize")
-        x8, sc8, sc32 = _u8(out[0]), _u8(out[1]), out[2]
+        x8, sc8, sc32 = out[0].view(E4M3), out[1].view(E8M0), out[2]
     lib = _lib.load()
     code = _dtype_code(x.dtype)
-    ws_bytes = lib.pratchya_quantize_workspace_bytes(code, S, H, W, a, b)
+    ws_bytes = _ws_bytes("pratchya_quantize_workspace_bytes", code, S, H, W, a, b)
     if ws_bytes == 0 and not _aligned(x8, 8 if x.dtype == torch.bfloat16 else 4):
         ws_bytes = S * n_blk * 4      # a misaligned caller payload buffer: the general path runs
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device) if ws_bytes else None
     _lib.check(lib.pratchya_quantize(_ptr(x), code, S, H, W, a, b, _ptr(x8), _ptr(sc8), _ptr(sc32),
                                      _ptr(ws) if ws is not None else None, ws_bytes, _stream(x)), "quantize")
-    return x8.view(E4M3), sc8.view(E8M0), sc32
+    return x8, sc8, sc32
 
 
 def quantize_dequantize(x: torch.Tensor, tgrid, dtype: torch.dtype, fix_nan: bool = False, out=None):
@@ -140,22 +165,22 @@ def quantize_dequantize(x: torch.Tensor, tgrid, dtype: torch.dtype, fix_nan: boo
         x = x.contiguous() if not x.is_contiguous() else x.clone()
     if out is None:
         y = torch.empty(x.shape, dtype=dtype, device=x.device)
-        sc8 = torch.empty(lead + (M, K), dtype=torch.uint8, device=x.device)
+        sc8 = torch.empty(lead + (M, K), dtype=E8M0, device=x.device)
         sc32 = torch.empty(lead + (M, 1, 1), dtype=torch.float32, device=x.device)
     else:
         esz = 2 if dtype == torch.bfloat16 else 4
         _check_out(out, [(x.shape, esz), (lead + (M, K), 1), (lead + (M, 1, 1), 4)], "quantize_dequantize")
-        y, sc8, sc32 = out[0], _u8(out[1]), out[2]
+        y, sc8, sc32 = out[0], out[1].view(E8M0), out[2]
     lib = _lib.load()
     code = _dtype_code(x.dtype)
-    ws_bytes = lib.pratchya_quantize_dequantize_workspace_bytes(code, S, H, W, a, b)
+    ws_bytes = _ws_bytes("pratchya_quantize_dequantize_workspace_bytes", code, S, H, W, a, b)
     if ws_bytes == 0 and not (_aligned(y, 16) and _aligned(sc8, 8)):
         ws_bytes = S * n_blk * 4      # misaligned caller buffers: the general path runs
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device) if ws_bytes else None
     _lib.check(lib.pratchya_quantize_dequantize(
         _ptr(x), code, S, H, W, a, b, _ptr(y), _dtype_code(dtype), 1 if fix_nan else 0, _ptr(sc8),
         _ptr(sc32), _ptr(ws) if ws is not None else None, ws_bytes, _stream(x)), "quantize_dequantize")
-    return y, sc8.view(E8M0), sc32
+    return y, sc8, sc32
 
 
 def requantize_cotangent(g: torch.Tensor, g_sc8: torch.Tensor, g_sc32: torch.Tensor, out=None):
@@ -362,8 +387,8 @@ def dequantize(x_fp8: torch.Tensor, sc_fp8: torch.Tensor, sc_fp32: torch.Tensor,
     a, b = int(tgrid[0]), int(tgrid[1])
     S, H, W = slices_hw(x_fp8.shape)
     out_dtype = dtype if dtype in (torch.float32, torch.bfloat16) else torch.float32
-    x8 = _u8(x_fp8).contiguous()
-    sc8 = _u8(sc_fp8).contiguous()
+    x8 = x_fp8.contiguous()
+    sc8 = sc_fp8.contiguous()
     sc32 = sc_fp32.contiguous().float()
     out = torch.empty(x_fp8.shape, dtype=out_dtype, device=x_fp8.device)
     lib = _lib.load()
@@ -387,8 +412,8 @@ def gather_dequantize(x_fp8: torch.Tensor, sc_fp8: torch.Tensor, sc_fp32: torch.
     a, b = int(tgrid[0]), int(tgrid[1])
     ids = idx.reshape(-1).to(torch.int64).contiguous()
     out = torch.empty(tuple(idx.shape) + (W,), dtype=dtype, device=x_fp8.device)
-    x8 = _u8(x_fp8).contiguous()
-    sc8 = _u8(sc_fp8).contiguous()
+    x8 = x_fp8.contiguous()
+    sc8 = sc_fp8.contiguous()
     sc32 = sc_fp32.contiguous().float()
     lib = _lib.load()
     _lib.check(lib.pratchya_gather_dequantize(_ptr(x8), _ptr(sc8), _ptr(sc32), H, W, a, b, _ptr(ids),
@@ -431,7 +456,7 @@ def elementwise(op: str, x, grid_x, y, grid_y, tgrid, out=None):
         q, sc8, sc32 = _u8(out[0]), _u8(out[1]), out[2]
     (xa, xb), (ya, yb) = (int(v) for v in grid_x), (int(v) for v in grid_y)
     lib = _lib.load()
-    ws_bytes = lib.pratchya_elementwise_workspace_bytes(S, H, W, xa, xb, ya, yb, a, b)
+    ws_bytes = _ws_bytes("pratchya_elementwise_workspace_bytes", S, H, W, xa, xb, ya, yb, a, b)
     if ws_bytes == 0 and not (_aligned(xq, 16) and _aligned(yq, 16) and _aligned(q, 16)):
         ws_bytes = S * n_blk * 4          # unaligned payloads take the general path
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x8.device) if ws_bytes else None
@@ -482,7 +507,7 @@ def dequantize_bwd(g: torch.Tensor, sc_fp8: torch.Tensor, sc_fp32: torch.Tensor,
     orig = g.dtype
     gg = g if g.dtype in (torch.float32, torch.bfloat16) else g.float()
     gg = gg.contiguous()
-    sc8 = _u8(sc_fp8).contiguous()
+    sc8 = sc_fp8.contiguous()
     sc32 = sc_fp32.contiguous().float()
     out = torch.empty(gg.shape, dtype=gg.dtype, device=g.device)
     lib = _lib.load()
@@ -780,12 +805,12 @@ def gemm_t128(a: Operand, b: Operand, out_dtype: torch.dtype = torch.float32) ->
     if a.k_major or b.k_major:
         raise PratchyaUnsupported("gemm_t128: K-contiguous operands only")
     M, N, Kd = a.rows, b.rows, a.k
-    ap, bp = _u8(a.payload).contiguous(), _u8(b.payload).contiguous()
-    as8, bs8 = _u8(a.sc8).contiguous(), _u8(b.sc8).contiguous()
+    ap, bp = a.payload.contiguous(), b.payload.contiguous()
+    as8, bs8 = a.sc8.contiguous(), b.sc8.contiguous()
     as32, bs32 = a.sc32.contiguous().float(), b.sc32.contiguous().float()
     lib = _lib.load()
     c = torch.empty((M, N), dtype=out_dtype, device=ap.device)
-    ws_bytes = int(lib.pratchya_gemm_t128_workspace_bytes(M, N, Kd // 128))
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 128)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=ap.device) if ws_bytes else None
     _lib.check(lib.pratchya_gemm_bs_t128(_ptr(ap), Kd, _ptr(as8), _ptr(as32), *a.desc, _ptr(bp), Kd, _ptr(bs8),
                                          _ptr(bs32), *b.desc, M, N, Kd, _ptr(c), N, _dtype_code(out_dtype),
@@ -861,7 +886,6 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
 # Planes of an operand of ``gemm_planes`` (pratchya_planes)
 PLANE_POW2, PLANE_SPLIT3, PLANE_SPLIT4, PLANE_BF16, PLANE_SPLIT4Q = 0, 1, 2, 3, 4
 _PLANE_COUNT = {PLANE_POW2: 1, PLANE_SPLIT3: 3, PLANE_SPLIT4: 4, PLANE_BF16: 2, PLANE_SPLIT4Q: 4}
-_PLANE_PAYLOADS = (PLANE_POW2, PLANE_SPLIT3, PLANE_SPLIT4Q)
 
 
 def planes(mode: int, src: torch.Tensor, sc8, sc32, tgrid, flags=None, pad: int = 1) -> torch.Tensor:
@@ -873,12 +897,11 @@ def planes(mode: int, src: torch.Tensor, sc8, sc32, tgrid, flags=None, pad: int 
     _require_gpu(src)
     T, W = int(src.shape[0]), int(src.shape[1])
     Tp = -(-T // pad) * pad
-    x = _u8(src) if mode in _PLANE_PAYLOADS else src
-    x = x.contiguous()
+    x = src.contiguous()
     if not _aligned(x, 16):
         x = x.clone()
     a, b = (int(tgrid[0]), int(tgrid[1])) if sc8 is not None else (1, 8)
-    e8 = _u8(sc8).contiguous() if sc8 is not None else None
+    e8 = sc8.contiguous() if sc8 is not None else None
     g32 = sc32.contiguous().float() if sc8 is not None else None
     out = torch.empty((_PLANE_COUNT[mode], Tp, W), dtype=torch.bfloat16, device=src.device)
     _lib.check(_lib.load().pratchya_planes(mode, _ptr(x), _ptr(e8) if e8 is not None else None,
@@ -907,7 +930,7 @@ def gemm_planes(a: torch.Tensor, b: torch.Tensor, pairs, k_major: bool, out_dtyp
     lib = _lib.load()
     short = short or len(pairs)
     c = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    ws_bytes = int(lib.pratchya_gemm_t128_workspace_bytes(M, N, short * (Kd // 64)))
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, short * (Kd // 64))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
     pa, pb = _nibbles(i for i, _ in pairs), _nibbles(j for _, j in pairs)
     g32, brow, bcol, kg = (units[0].contiguous().float(), int(units[1][0]), int(units[1][1]), int(units[2])) \
@@ -936,7 +959,7 @@ def gemm_fine(a: torch.Tensor, a_sc32: torch.Tensor, b: torch.Tensor, b_sc32: to
     if ag.numel() != M * Kd // (16 if blk == 16 else 64):
         raise PratchyaUnsupported("gemm_fine: x's groups are not one block of 16 or two of 32")
     c = torch.empty((M, N), dtype=torch.float32, device=a.device)
-    ws_bytes = int(lib.pratchya_gemm_t128_workspace_bytes(M, N, Kd // 64))
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 64)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
     _lib.check(lib.pratchya_gemm_fine(_ptr(a), int(a.stride(0)), _ptr(ag), _ptr(b), int(b.stride(0)), _ptr(bg), b_kg, blk,
                                       M, N, Kd, _ptr(c), N, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
@@ -1038,7 +1061,7 @@ def gemm_bf16_gram(a: torch.Tensor, k_major: bool = False, status: torch.Tensor 
         raise ValueError("gemm_bf16_gram: a must be 2-D bfloat16")
     M, Kd = (int(a.shape[1]), int(a.shape[0])) if k_major else (int(a.shape[0]), int(a.shape[1]))
     lib = _lib.load()
-    ws_bytes = int(lib.pratchya_gemm_bf16_gram_workspace_bytes(M, Kd))
+    ws_bytes = _ws_bytes("pratchya_gemm_bf16_gram_workspace_bytes", M, Kd)
     if ws_bytes <= 0:
         raise PratchyaUnsupported(f"gemm_bf16_gram: M must be a multiple of 256 and K of 64 (got {M}, {Kd})")
     ap = a.contiguous()
@@ -1129,7 +1152,7 @@ def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = F
             and prefers_t128(M, a.desc[3], b):
         return _few_then_requantize(a, b, out_dtype, (1, 128), fix_nan, lead)
     lib = _lib.load()
-    ws_bytes = lib.pratchya_gemm_bs_nt_fq_workspace_bytes(M, N)
+    ws_bytes = _ws_bytes("pratchya_gemm_bs_nt_fq_workspace_bytes", M, N)
     if ws_bytes <= 0:
         raise PratchyaUnsupported(f"gemm_fq: N must be a multiple of 1024 (got {N})")
     ap, bp = _tile_readable(_u8(a.payload).contiguous()), _tile_readable(_u8(b.payload).contiguous())
