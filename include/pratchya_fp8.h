@@ -469,6 +469,11 @@ int pratchya_ns_normalize(const void* g, void* x, int64_t n, void* workspace, in
  * f32, their f32 sum (the fixed order of pratchya_ns_normalize), sqrt and the
  * sum with 1e-7 in f32, IEEE f32 quotients.  g, x: f32 [n], 16-byte aligned;
  * x may be g; workspace as pratchya_ns_normalize. */
+/* The same of `batch` bf16 arrays of n elements one after the other, each by its
+ * own norm (n a multiple of 8 unless batch is 1); workspace: batch times
+ * pratchya_ns_normalize_workspace_bytes() bytes. */
+int pratchya_ns_normalize_batch(const void* g, void* x, int64_t n, int64_t batch, void* workspace,
+                                int64_t workspace_bytes, hipStream_t stream);
 int pratchya_ns_normalize_f32(const float* g, float* x, int64_t n, void* workspace, int64_t workspace_bytes,
                               hipStream_t stream);
 
@@ -490,8 +495,8 @@ int pratchya_gemm_bf16_nt_ns(const void* A, int64_t lda, const void* B, int64_t 
 /* The 128-row-tile GEMM (K split over workgroups where the tiles alone do not
  * fill the chip).  Workspace of a call of M x N outputs and `steps` K steps (128
  * FP8 or 64 bf16 values per step; for pratchya_gemm_bf16_planes segs_short * K /
- * 64): f32 partials of the K slices, 0 if K is not split. */
-int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps);
+ * 64; 1 unless batched): f32 partials of the K slices, 0 if K is not split. */
+int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps, int64_t batch);
 
 /* pratchya_gemm_bs_nt on 128-row tiles (32-row tiles up to M = 32): the same
  * operands and scale layouts, summed in another order.  Operands are read up
@@ -517,13 +522,16 @@ int pratchya_gemm_bs_t128(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, c
  * [N, K] payload quantized (b_brow, b_bcol) with b_kg blocks per group and
  * these group maxima; their mantissas multiply the sums per span of K where
  * they are constant (a multiple of 64 values, PRATCHYA_EUNSUPPORTED otherwise).
- * X (may be null): bf16 output 1.5 X - 0.5 C (pratchya_ns_combine's bits). */
+ * X (may be null): bf16 output 1.5 X - 0.5 C (pratchya_ns_combine's bits).
+ * batch > 1: that many products of one shape, *_batch elements apart (no flags,
+ * no b_sc32). */
 int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_stride, int a_kmajor, int a_held, uint32_t a_planes,
                               const void* B, int64_t ldb, int64_t b_stride, int b_kmajor, int b_held,
                               uint32_t b_planes, uint32_t b_planes_alt, int64_t M, int64_t N, int64_t K, int segs,
                               int segs_short, const uint32_t* flags, const float* b_sc32, int64_t b_brow,
                               int64_t b_bcol, int64_t b_kg, void* C, int64_t ldc, int c_dtype, const void* X,
-                              int64_t ldx, void* ws, int64_t ws_bytes, hipStream_t stream);
+                              int64_t ldx, int64_t batch, int64_t a_batch, int64_t b_batch, int64_t c_batch,
+                              int64_t x_batch, void* ws, int64_t ws_bytes, hipStream_t stream);
 
 /* f32 C [M, N] = dequant(x) . dequant(W) to f32 accuracy (Q:605-608) for x
  * quantized (1, blk) and W [K, N] quantized (blk, blk), blk 16 or 32 (the
@@ -531,7 +539,7 @@ int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_stride, int 
  * (pratchya_planes), a_sc32 and b_sc32 their group maxima (x: one block of 16 or
  * two of 32 per group; W: b_kg blocks), whose mantissas multiply each block's
  * exact f32 sums.  K a multiple of 64, N of blk.  ws: partials of
- * pratchya_gemm_t128_workspace_bytes(M, N, K / 64) bytes. */
+ * pratchya_gemm_t128_workspace_bytes(M, N, K / 64, 1) bytes. */
 int pratchya_gemm_fine(const void* A, int64_t lda, const float* a_sc32, const void* B, int64_t ldb, const float* b_sc32,
                        int64_t b_kg, int64_t blk, int64_t M, int64_t N, int64_t K, float* C, int64_t ldc, void* ws,
                        int64_t ws_bytes, hipStream_t stream);

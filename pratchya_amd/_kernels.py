@@ -810,7 +810,7 @@ def gemm_t128(a: Operand, b: Operand, out_dtype: torch.dtype = torch.float32) ->
     as32, bs32 = a.sc32.contiguous().float(), b.sc32.contiguous().float()
     lib = _lib.load()
     c = torch.empty((M, N), dtype=out_dtype, device=ap.device)
-    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 128)
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 128, 1)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=ap.device) if ws_bytes else None
     _lib.check(lib.pratchya_gemm_bs_t128(_ptr(ap), Kd, _ptr(as8), _ptr(as32), *a.desc, _ptr(bp), Kd, _ptr(bs8),
                                          _ptr(bs32), *b.desc, M, N, Kd, _ptr(c), N, _dtype_code(out_dtype),
@@ -840,6 +840,29 @@ def _split_pack(src: torch.Tensor, transpose: bool, planes, kp: int, out_rows_mi
     return dst
 
 
+# The pairs of planes (PLANE_SPLIT4) of a product of two f32 operands: the six
+# whose weight is at least 2^-24 of the leading product (_F32_PAIRS), a
+# non-finite value in the first only
+F32_PLANE_PAIRS = ((0, 0), (3, 1), (1, 3), (3, 2), (1, 1), (2, 3))
+
+
+def _matmul_f32_planes(a, b, a_t, b_t, M, N, Kd):
+    """matmul_f32 on 128x128 tiles, the operands' planes in their own layouts
+    (each written once, no transposed copies)."""
+    if a.dtype == torch.bfloat16 or ((not a_t or b_t) and Kd % 64):
+        raise PratchyaUnsupported("matmul_f32: packed pieces")
+    if b.dtype == torch.bfloat16:
+        flags = torch.zeros(2, dtype=torch.int32, device=a.device)
+        pb = planes(PLANE_BF16, b, None, None, None, flags, pad=1 if b_t else 64)
+        pa = planes(PLANE_SPLIT4, a, None, None, None, pad=64 if a_t else 1)
+        return gemm_planes(pa, pb, ((0, 0), (1, 0), (2, 0)), a_t, b_alt=(0, 1, 1), flags=flags, b_k_major=not b_t,
+                           short=3)
+    pa = planes(PLANE_SPLIT4, a, None, None, None, pad=64 if a_t else 1)
+    same = b is a and a_t == (not b_t)
+    pb = pa if same else planes(PLANE_SPLIT4, b, None, None, None, pad=1 if b_t else 64)
+    return gemm_planes(pa, pb, F32_PLANE_PAIRS, a_t, b_k_major=not b_t)
+
+
 def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = False) -> torch.Tensor:
     """f32 ``op(a) @ op(b)`` for 2-D f32 / bf16 tensors on the bf16 MFMA
     kernel: ``op(a)`` is ``a`` [M, K] (``a_t``: ``a`` is [K, M] and is used
@@ -863,6 +886,11 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
         return torch.empty((M, N), dtype=torch.float32, device=a.device)
     if Kd == 0:
         return torch.zeros((M, N), dtype=torch.float32, device=a.device)
+    if few_tiles(M, N) and M > 32:
+        try:
+            return _matmul_f32_planes(a, b, a_t, b_t, M, N, Kd)
+        except PratchyaUnsupported:
+            pass
     na = 1 if a.dtype == torch.bfloat16 else 3
     nb = 1 if b.dtype == torch.bfloat16 else 3
     pairs = [(i, j) for i, j in _F32_PAIRS if i < na and j < nb]
@@ -876,7 +904,7 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
     n_rows = N if N >= GEMM_TILE_ROWS else (N + 3) // 4 * 4
     A = _split_pack(a, a_t, a_planes, kp)
     B = _split_pack(b, not b_t, b_planes, kp, n_rows)
-    if few_tiles(M, n_rows) and n_rows % 4 == 0:
+    if few_tiles(M, n_rows):
         c = gemm_planes(A[None], B[None], [(0, 0)], False)
     else:
         c = gemm_bf16_nt(A, B, torch.float32)
@@ -910,6 +938,7 @@ def planes(mode: int, src: torch.Tensor, sc8, sc32, tgrid, flags=None, pad: int 
     return out
 
 
+@functools.lru_cache(maxsize=64)
 def _nibbles(seq) -> int:
     return sum(int(v) << (4 * i) for i, v in enumerate(seq))
 
@@ -918,31 +947,44 @@ def gemm_planes(a: torch.Tensor, b: torch.Tensor, pairs, k_major: bool, out_dtyp
                 b_alt=None, flags=None, units=None, x=None, b_k_major=None) -> torch.Tensor:
     """``sum over (i, j) in pairs of op(a[i]) @ op(b[j])^T`` for bf16 planes
     ``a`` [planes, M, K] and ``b`` [planes, N, K] (``k_major``: [planes, K, M] and
-    [planes, K, N]) with f32 accumulation.  ``short`` pairs are enough where
-    flags[0] is 0; ``b_alt`` are b's planes where flags[1] is not.  ``units``:
-    ``(sc32, tgrid, blocks per group)`` of the payload that b is the power-of-two
-    plane of.  ``x`` [M, N] bf16: the result is ``1.5 x - 0.5 product`` in bf16
-    (``b_k_major``: b alone is K-major)."""
+    [planes, K, N]; ``b_k_major``: b's layout where it differs) with f32
+    accumulation.  ``short`` pairs are enough where flags[0] is 0; ``b_alt`` are
+    b's planes where flags[1] is not.  ``units``: ``(sc32, tgrid, blocks per
+    group)`` of the payload that b is the power-of-two plane of.  ``x`` [M, N]
+    bf16: the result is ``1.5 x - 0.5 product`` in bf16."""
     _require_gpu(a, b)
+    return _gemm_planes(a[None], b[None], pairs, k_major, out_dtype, short, b_alt, flags, units,
+                        None if x is None else x[None], b_k_major)[0]
+
+
+def gemm_planes_batch(a: torch.Tensor, b: torch.Tensor, k_major: bool, out_dtype=torch.float32, x=None,
+                      b_k_major=None) -> torch.Tensor:
+    """``gemm_planes`` of each slice's single planes: a [batch, M, K], b [batch,
+    N, K], x [batch, M, N]."""
+    _require_gpu(a, b)
+    return _gemm_planes(a[:, None], b[:, None], ((0, 0),), k_major, out_dtype, x=x, b_k_major=b_k_major)
+
+
+def _gemm_planes(a, b, pairs, k_major, out_dtype, short=0, b_alt=None, flags=None, units=None, x=None, b_k_major=None):
     b_km = k_major if b_k_major is None else b_k_major
-    M, Kd = (int(a.shape[2]), int(a.shape[1])) if k_major else (int(a.shape[1]), int(a.shape[2]))
-    N = int(b.shape[2] if b_km else b.shape[1])
-    lib = _lib.load()
+    L, ha, a0, a1 = a.shape
+    b0, b1 = b.shape[2:]
+    (M, Kd), N = ((a1, a0) if k_major else (a0, a1)), (b1 if b_km else b0)
     short = short or len(pairs)
-    c = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, short * (Kd // 64))
+    c = torch.empty((L, M, N), dtype=out_dtype, device=a.device)
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, short * (Kd // 64), L)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
-    pa, pb = _nibbles(i for i, _ in pairs), _nibbles(j for _, j in pairs)
+    pa, pb = _nibbles(tuple(i for i, _ in pairs)), _nibbles(tuple(j for _, j in pairs))
     g32, brow, bcol, kg = (units[0].contiguous().float(), int(units[1][0]), int(units[1][1]), int(units[2])) \
         if units is not None else (None, 1, 1, 1)
-    _lib.check(lib.pratchya_gemm_bf16_planes(
-        _ptr(a), int(a.stride(1)), int(a.stride(0)), 1 if k_major else 0, int(a.shape[0]), pa,
-        _ptr(b), int(b.stride(1)), int(b.stride(0)), 1 if b_km else 0, int(b.shape[0]), pb,
-        pb if b_alt is None else _nibbles(b_alt), M, N, Kd, len(pairs), short,
+    (sa, ta, lda, _), (sb, tb, ldb, _) = a.stride(), b.stride()
+    _lib.check(_lib.load().pratchya_gemm_bf16_planes(
+        _ptr(a), lda, ta, 1 if k_major else 0, ha, pa, _ptr(b), ldb, tb, 1 if b_km else 0, b.shape[1], pb,
+        pb if b_alt is None else _nibbles(tuple(b_alt)), M, N, Kd, len(pairs), short,
         _ptr(flags) if flags is not None else None, _ptr(g32) if g32 is not None else None, brow, bcol, kg,
-        _ptr(c), N, _dtype_code(out_dtype), _ptr(x) if x is not None else None,
-        int(x.stride(0)) if x is not None else 0, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
-        "gemm_planes")
+        _ptr(c), N, _dtype_code(out_dtype), _ptr(x) if x is not None else None, x.stride(1) if x is not None else 0,
+        L, sa, sb, M * N, x.stride(0) if x is not None else 0, _ptr(ws) if ws is not None else None, ws_bytes,
+        _stream(a)), "gemm_planes")
     return c
 
 
@@ -959,7 +1001,7 @@ def gemm_fine(a: torch.Tensor, a_sc32: torch.Tensor, b: torch.Tensor, b_sc32: to
     if ag.numel() != M * Kd // (16 if blk == 16 else 64):
         raise PratchyaUnsupported("gemm_fine: x's groups are not one block of 16 or two of 32")
     c = torch.empty((M, N), dtype=torch.float32, device=a.device)
-    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 64)
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 64, 1)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
     _lib.check(lib.pratchya_gemm_fine(_ptr(a), int(a.stride(0)), _ptr(ag), _ptr(b), int(b.stride(0)), _ptr(bg), b_kg, blk,
                                       M, N, Kd, _ptr(c), N, _ptr(ws) if ws is not None else None, ws_bytes, _stream(a)),
@@ -992,9 +1034,24 @@ def ns_normalize(g: torch.Tensor) -> torch.Tensor:
     gc = g.contiguous()
     out = torch.empty_like(gc)
     lib = _lib.load()
-    ws = torch.empty(int(lib.pratchya_ns_normalize_workspace_bytes()), dtype=torch.uint8, device=gc.device)
+    ws = torch.empty(_ws_bytes("pratchya_ns_normalize_workspace_bytes"), dtype=torch.uint8, device=gc.device)
     fn = lib.pratchya_ns_normalize if g.dtype == torch.bfloat16 else lib.pratchya_ns_normalize_f32
     _lib.check(fn(_ptr(gc), _ptr(out), gc.numel(), _ptr(ws), ws.numel(), _stream(gc)), "ns_normalize")
+    return out
+
+
+def ns_normalize_batch(g: torch.Tensor) -> torch.Tensor:
+    """``ns_normalize`` of each slice of a bf16 [batch, m, n] array (m * n a
+    multiple of 8)."""
+    _require_gpu(g)
+    if g.dtype != torch.bfloat16 or g.dim() != 3:
+        raise ValueError("ns_normalize_batch: g must be a 3-D bfloat16 array")
+    gc = g.contiguous()
+    out = torch.empty_like(gc)
+    L = int(g.shape[0])
+    ws = torch.empty(L * _ws_bytes("pratchya_ns_normalize_workspace_bytes"), dtype=torch.uint8, device=gc.device)
+    _lib.check(_lib.load().pratchya_ns_normalize_batch(_ptr(gc), _ptr(out), gc.numel() // max(L, 1), L, _ptr(ws),
+                                                       ws.numel(), _stream(gc)), "ns_normalize_batch")
     return out
 
 

@@ -62,6 +62,7 @@ SIGNATURES = {
     "pratchya_ns_combine": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_int, _c_p]),
     "pratchya_ns_normalize_workspace_bytes": (_c_i64, []),
     "pratchya_ns_normalize": (_c_int, [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p]),
+    "pratchya_ns_normalize_batch": (_c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_p, _c_i64, _c_p]),
     "pratchya_ns_normalize_f32": (_c_int, [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p]),
     "pratchya_apply_update": (_c_int, [_c_p, _c_int, _c_int, ctypes.c_float, _c_p, _c_int, _c_p, _c_p,
                                        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, ctypes.c_float,
@@ -106,14 +107,15 @@ SIGNATURES = {
     "pratchya_transpose_b16": (_c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p]),
     "pratchya_split_pack_bf16": (_c_int, [_c_p, _c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
                                           ctypes.POINTER(_c_int), _c_p, _c_i64, _c_i64, _c_p]),
-    "pratchya_gemm_t128_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "pratchya_gemm_t128_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "pratchya_gemm_bs_t128": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
                                        _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
                                        _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p]),
     "pratchya_gemm_bf16_planes": (_c_int, [_c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32,
                                            _c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32, ctypes.c_uint32,
                                            _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_p, _c_p, _c_i64, _c_i64,
-                                           _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p, _c_i64, _c_p]),
+                                           _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
+                                           _c_i64, _c_i64, _c_p, _c_i64, _c_p]),
     "pratchya_gemm_fine": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                     _c_p, _c_i64, _c_p, _c_i64, _c_p]),
     "pratchya_planes": (_c_int, [_c_int, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p]),

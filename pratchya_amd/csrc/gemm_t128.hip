@@ -71,6 +71,10 @@ struct T128Args {
   const uint32_t* flags;                 // bf16 planes, may be null: see k_gemm_t128
   int64_t ldc, ldx;
   int M, N, spp, segs, segs_short, span, splits, tiles_m, tiles_n;
+  // independent products of one shape: bytes (A, B) and elements (C, X) from
+  // one to the next
+  int batch;
+  int64_t a_bs, b_bs, c_bs, x_bs;
 };
 
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
@@ -176,11 +180,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   // workgroup -> (slice, tile): each XCD (workgroups are dealt to the 8 in
   // turn) takes consecutive numbers, which walk bands of up to 8 tile rows of
   // one slice, so that it shares few panels in its L2
-  const int tiles = p.tiles_m * p.tiles_n, total = tiles * p.splits;
+  const int tiles = p.tiles_m * p.tiles_n, total = tiles * p.splits * p.batch;
   int L = blockIdx.x;
   if (total % 8 == 0) L = (L & 7) * (total >> 3) + (L >> 3);
-  const int slice = L / tiles;
-  L -= slice * tiles;
+  const int unit = L / tiles;
+  L -= unit * tiles;
+  const int slice = unit % p.splits, bi = unit / p.splits;
   const int gm = p.tiles_m < 8 ? p.tiles_m : 8;
   const int band = L / (gm * p.tiles_n);
   const int in_band = min(p.tiles_m - band * gm, gm);
@@ -198,8 +203,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   const int k_end = (int)((uint32_t)(slice + 1) * (uint32_t)steps / (uint32_t)p.splits);
 
   constexpr int kFlags = 0x00020000;
-  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)p.a.p, 0, (int)p.a.bytes, kFlags);
-  const __amdgpu_buffer_rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)p.b.p, 0, (int)p.b.bytes, kFlags);
+  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.a.p + bi * p.a_bs), 0, (int)p.a.bytes, kFlags);
+  const __amdgpu_buffer_rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(p.b.p + bi * p.b_bs), 0, (int)p.b.bytes, kFlags);
   const __amdgpu_buffer_rsrc_t rs_ea = __builtin_amdgcn_make_buffer_rsrc((void*)p.a.e8, 0, (int)p.a.e8_bytes, kFlags);
   const __amdgpu_buffer_rsrc_t rs_eb = __builtin_amdgcn_make_buffer_rsrc((void*)p.b.e8, 0, (int)p.b.e8_bytes, kFlags);
   const __amdgpu_buffer_rsrc_t rs_ga = __builtin_amdgcn_make_buffer_rsrc((void*)p.a.g32, 0, (int)p.a.g32_bytes, kFlags);
@@ -505,7 +510,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
     __builtin_amdgcn_wave_barrier();
     const int row0 = m0 + wm * 64 + mi * 32;
     if (OUT == 0 || p.splits > 1) {
-      float* out = p.splits > 1 ? p.part + (int64_t)slice * p.M * p.N : static_cast<float*>(p.C);
+      float* out = p.splits > 1 ? p.part + (int64_t)unit * p.M * p.N : static_cast<float*>(p.C) + bi * p.c_bs;
       const int64_t ld = p.splits > 1 ? (int64_t)p.N : p.ldc;
 #pragma unroll
       for (int it = 0; it < WN / 8; ++it) {
@@ -514,7 +519,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
         if (row0 + r < p.M && col0 + c < p.N) *reinterpret_cast<v4f*>(out + (row0 + r) * ld + col0 + c) = v;
       }
     } else {
-      uint16_t* out = static_cast<uint16_t*>(p.C);
+      uint16_t* out = static_cast<uint16_t*>(p.C) + bi * p.c_bs;
 #pragma unroll
       for (int it = 0; it < WN / 16; ++it) {
         const int q = it * 64 + lane, r = q / (WN / 8), c = (q % (WN / 8)) * 8;
@@ -524,7 +529,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
                  (int)pack_bf16x2(x.z, x.w)};
         if (row0 + r < p.M && col0 + c < p.N) {
           if constexpr (OUT == 2) {
-            const v4i xv = *reinterpret_cast<const v4i*>(p.X + (row0 + r) * p.ldx + col0 + c);
+            const v4i xv = *reinterpret_cast<const v4i*>(p.X + bi * p.x_bs + (row0 + r) * p.ldx + col0 + c);
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[i] = (int)ns_pair((uint32_t)xv[i], (uint32_t)o[i]);
           }
@@ -539,9 +544,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
 
 // C = the slices' sum, in slice order, with k_gemm_t128's epilogues.
 template <int OUT>
-__global__ __launch_bounds__(256) void k_reduce_slices(const float* __restrict__ part, int splits, int M, int N,
-                                                       void* __restrict__ C, int64_t ldc,
-                                                       const uint16_t* __restrict__ X, int64_t ldx) {
+__global__ __launch_bounds__(256) void k_reduce_slices(const float* part, int splits, int M, int N,
+                                                       void* C, int64_t ldc,
+                                                       const uint16_t* X, int64_t ldx, int64_t c_bs,
+                                                       int64_t x_bs) {
+  part += (int64_t)blockIdx.y * splits * M * N;
+  C = static_cast<uint8_t*>(C) + (int64_t)blockIdx.y * c_bs * (OUT == 0 ? 4 : 2);
+  if constexpr (OUT == 2) X += (int64_t)blockIdx.y * x_bs;
   constexpr int CH = OUT == 0 ? 4 : 8;
   const int per_row = N / CH;
   const int64_t n = (int64_t)M * per_row, stride = (int64_t)M * N;
@@ -596,9 +605,9 @@ int t128_cus() {
 // Slices of the K steps: as many as fill two workgroups per CU, each at least
 // min_steps long (below that a slice's start and its partial cost more than
 // the steps it takes off the others).
-int t128_splits(int64_t M, int64_t N, int64_t steps) {
+int t128_splits(int64_t M, int64_t N, int64_t steps, int64_t batch) {
   const int rows = t128_rows(M);
-  const int64_t tiles = ((M + rows - 1) / rows) * ((N + TN - 1) / TN);
+  const int64_t tiles = batch * ((M + rows - 1) / rows) * ((N + TN - 1) / TN);
   const int64_t min_steps = rows == 32 ? 2 : 4;
   int64_t s = 2 * t128_cus() / tiles;
   if (s > steps / min_steps) s = steps / min_steps;
@@ -608,13 +617,13 @@ int t128_splits(int64_t M, int64_t N, int64_t steps) {
 
 template <bool BF, int TM, bool TNA, bool TNB, int SC, int OUT>
 void t128_launch(const T128Args& p, hipStream_t stream) {
-  hipLaunchKernelGGL((k_gemm_t128<BF, TM, TNA, TNB, SC, OUT>), dim3((unsigned)(p.tiles_m * p.tiles_n * p.splits)),
+  hipLaunchKernelGGL((k_gemm_t128<BF, TM, TNA, TNB, SC, OUT>), dim3((unsigned)(p.tiles_m * p.tiles_n * p.splits * p.batch)),
                      dim3(256), 0, stream, p);
   if (p.splits > 1) {
     const int64_t n = (int64_t)p.M * (p.N / (OUT == 0 ? 4 : 8));
     const int64_t blocks = (n + 255) / 256;
-    hipLaunchKernelGGL((k_reduce_slices<OUT>), dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, stream,
-                       p.part, p.splits, p.M, p.N, p.C, p.ldc, p.X, p.ldx);
+    hipLaunchKernelGGL((k_reduce_slices<OUT>), dim3((unsigned)(blocks < 2048 ? blocks : 2048), (unsigned)p.batch),
+                       dim3(256), 0, stream, p.part, p.splits, p.M, p.N, p.C, p.ldc, p.X, p.ldx, p.c_bs, p.x_bs);
   }
 }
 
@@ -631,16 +640,20 @@ int ilog2_exact(int64_t v) {
 }
 
 // Tiles, slices and the partials' workspace of one call.
-int t128_shape(const char* who, T128Args* p, int64_t M, int64_t N, int64_t steps, void* ws, int64_t ws_bytes) {
+int t128_shape(const char* who, T128Args* p, int64_t M, int64_t N, int64_t steps, void* ws, int64_t ws_bytes,
+               int64_t batch = 1) {
   const int rows = t128_rows(M);
   p->M = (int)M;
   p->N = (int)N;
   p->tiles_m = (int)((M + rows - 1) / rows);
   p->tiles_n = (int)((N + TN - 1) / TN);
-  p->splits = t128_splits(M, N, steps);
-  if (p->splits > 1 && (!ws || ws_bytes < (int64_t)p->splits * M * N * 4 || (reinterpret_cast<uintptr_t>(ws) & 15)))
-    return pratchya_set_error(PRATCHYA_EINVAL, "%s: workspace of %lld bytes (16-byte aligned) needed", who,
-                              (long long)((int64_t)p->splits * M * N * 4));
+  p->splits = t128_splits(M, N, steps, batch);
+  p->batch = (int)batch;
+  if ((int64_t)p->tiles_m * p->tiles_n * p->splits * batch > INT32_MAX / 2)
+    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: too many tiles", who);
+  const int64_t need = batch * p->splits * M * N * 4;
+  if (p->splits > 1 && (!ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 15)))
+    return pratchya_set_error(PRATCHYA_EINVAL, "%s: workspace of %lld bytes (16-byte aligned) needed", who, (long long)need);
   p->part = static_cast<float*>(ws);
   return PRATCHYA_OK;
 }
@@ -649,10 +662,10 @@ constexpr int64_t kMaxOffset = (int64_t)UINT32_MAX;
 
 }  // namespace
 
-extern "C" int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps) {
-  if (M < 1 || N < 1 || steps < 1 || M > INT32_MAX || N > INT32_MAX) return 0;
-  const int s = t128_splits(M, N, steps);
-  return s > 1 ? (int64_t)s * M * N * 4 : 0;
+extern "C" int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps, int64_t batch) {
+  if (M < 1 || N < 1 || steps < 1 || M > INT32_MAX || N > INT32_MAX || batch < 1 || batch > 65535) return 0;
+  const int s = t128_splits(M, N, steps, batch);
+  return s > 1 ? batch * s * M * N * 4 : 0;
 }
 
 extern "C" int pratchya_gemm_bs_t128(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, const float* a_sc32,
@@ -721,13 +734,16 @@ extern "C" int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_s
                                          int b_held, uint32_t b_planes, uint32_t b_planes_alt, int64_t M, int64_t N,
                                          int64_t K, int segs, int segs_short, const uint32_t* flags,
                                          const float* b_sc32, int64_t b_brow, int64_t b_bcol, int64_t b_kg, void* C,
-                                         int64_t ldc, int c_dtype, const void* X, int64_t ldx, void* ws,
+                                         int64_t ldc, int c_dtype, const void* X, int64_t ldx, int64_t batch,
+                                         int64_t a_batch, int64_t b_batch, int64_t c_batch, int64_t x_batch, void* ws,
                                          int64_t ws_bytes, hipStream_t stream) {
   const char* who = "gemm_bf16_planes";
-  if (M <= 0 || N <= 0 || K <= 0) {
-    if (M < 0 || N < 0 || K < 0) return pratchya_set_error(PRATCHYA_EINVAL, "%s: negative size", who);
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) {
+    if (M < 0 || N < 0 || K < 0 || batch < 0) return pratchya_set_error(PRATCHYA_EINVAL, "%s: negative size", who);
     return PRATCHYA_OK;
   }
+  if (batch > 1 && (batch > 65535 || a_batch % 8 || b_batch % 8 || c_batch % 8 || x_batch % 8 || flags || b_sc32))
+    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: batches of plain products, strides multiples of 8", who);
   if (c_dtype != PRATCHYA_DT_F32 && c_dtype != PRATCHYA_DT_BF16)
     return pratchya_set_error(PRATCHYA_EINVAL, "%s: unsupported output dtype %d", who, c_dtype);
   const int chunk = c_dtype == PRATCHYA_DT_BF16 ? 8 : 4;
@@ -795,7 +811,11 @@ extern "C" int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_s
     p.b.sk2 = (uint32_t)(128 / b_bcol);
     p.b.kg_sh = (uint32_t)sh;
   }
-  const int rc = t128_shape(who, &p, M, N, (int64_t)segs_short * p.spp, ws, ws_bytes);
+  p.a_bs = 2 * a_batch;
+  p.b_bs = 2 * b_batch;
+  p.c_bs = c_batch;
+  p.x_bs = x_batch;
+  const int rc = t128_shape(who, &p, M, N, (int64_t)segs_short * p.spp, ws, ws_bytes, batch);
   if (rc) return rc;
   const bool bf = c_dtype == PRATCHYA_DT_BF16, small = t128_rows(M) == 32;
   if (b_sc32) {
@@ -805,8 +825,13 @@ extern "C" int pratchya_gemm_bf16_planes(const void* A, int64_t lda, int64_t a_s
     if (small || a_kmajor) return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: the combination needs a K-contiguous A of over 32 rows", who);
     if (b_kmajor) t128_launch<true, 128, false, true, 0, 2>(p, stream);
     else t128_launch<true, 128, false, false, 0, 2>(p, stream);
-  } else if (a_kmajor != b_kmajor || (a_kmajor && small)) {
-    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: K-major operands are supported as a pair, over 32 rows", who);
+  } else if (a_kmajor && small) {
+    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: a K-major A needs over 32 rows", who);
+  } else if (a_kmajor != b_kmajor) {
+    if (bf) return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "%s: one K-major operand is supported with f32 output", who);
+    if (a_kmajor) t128_launch<true, 128, true, false, 0, 0>(p, stream);
+    else if (small) t128_launch<true, 32, false, true, 0, 0>(p, stream);
+    else t128_launch<true, 128, false, true, 0, 0>(p, stream);
   } else if (a_kmajor) {
     if (bf) t128_launch<true, 128, true, true, 0, 1>(p, stream);
     else t128_launch<true, 128, true, true, 0, 0>(p, stream);

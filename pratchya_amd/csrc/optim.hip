@@ -248,6 +248,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 __global__ __launch_bounds__(256) void k_sumsq_b16(const uint16_t* __restrict__ x, int64_t n,
                                                    float* __restrict__ part) {
+  x += (int64_t)blockIdx.y * n;             // one array per grid row
+  part += (int64_t)blockIdx.y * kNormBlocks;
   const int64_t n8 = n / 8;
   float s = 0.0f;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (int64_t)gridDim.x * 256) {
@@ -277,6 +279,9 @@ __global__ __launch_bounds__(256) void k_sumsq_b16(const uint16_t* __restrict__ 
 // thread)
 __global__ __launch_bounds__(256) void k_ns_scale_b16(const uint16_t* x, int64_t n, const float* __restrict__ part,
                                                       uint16_t* y) {
+  x += (int64_t)blockIdx.y * n;
+  y += (int64_t)blockIdx.y * n;
+  part += (int64_t)blockIdx.y * kNormBlocks;
   __shared__ float sden;
   if (threadIdx.x < 64) {
     float s = 0.0f;
@@ -498,21 +503,28 @@ extern "C" int64_t pratchya_ns_normalize_workspace_bytes(void) { return (int64_t
 
 extern "C" int pratchya_ns_normalize(const void* g, void* x, int64_t n, void* workspace, int64_t workspace_bytes,
                                      hipStream_t stream) {
-  if (n < 0) return pratchya_set_error(PRATCHYA_EINVAL, "ns_normalize: negative size");
-  if (n == 0) return PRATCHYA_OK;
+  return pratchya_ns_normalize_batch(g, x, n, 1, workspace, workspace_bytes, stream);
+}
+
+extern "C" int pratchya_ns_normalize_batch(const void* g, void* x, int64_t n, int64_t batch, void* workspace,
+                                           int64_t workspace_bytes, hipStream_t stream) {
+  if (n < 0 || batch < 0) return pratchya_set_error(PRATCHYA_EINVAL, "ns_normalize: negative size");
+  if (n == 0 || batch == 0) return PRATCHYA_OK;
   if (!g || !x || !workspace) return pratchya_set_error(PRATCHYA_EINVAL, "ns_normalize: null buffer");
-  if (workspace_bytes < (int64_t)kNormBlocks * 4 || reinterpret_cast<uintptr_t>(workspace) % 4)
-    return pratchya_set_error(PRATCHYA_EINVAL, "ns_normalize: workspace of %lld bytes (need %d, 4-byte aligned)",
-                              (long long)workspace_bytes, kNormBlocks * 4);
+  if (batch > 1 && (n % 8 || batch > 65535))
+    return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "ns_normalize: up to 65535 arrays of a multiple of 8 elements");
+  if (workspace_bytes < batch * kNormBlocks * 4 || reinterpret_cast<uintptr_t>(workspace) % 4)
+    return pratchya_set_error(PRATCHYA_EINVAL, "ns_normalize: workspace of %lld bytes (need %lld, 4-byte aligned)",
+                              (long long)workspace_bytes, (long long)(batch * kNormBlocks * 4));
   if ((reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x)) % 16)
     return pratchya_set_error(PRATCHYA_EINVAL, "ns_normalize: g and x must be 16-byte aligned");
   float* part = static_cast<float*>(workspace);
-  hipLaunchKernelGGL(k_sumsq_b16, dim3(kNormBlocks), dim3(256), 0, stream, static_cast<const uint16_t*>(g), n, part);
+  hipLaunchKernelGGL(k_sumsq_b16, dim3(kNormBlocks, (unsigned)batch), dim3(256), 0, stream, static_cast<const uint16_t*>(g), n, part);
   int rc = check_launch("ns_normalize");
   if (rc) return rc;
   const int64_t chunks = n / 8;
   const int64_t blocks = chunks / 256 + 1 < 4096 ? chunks / 256 + 1 : 4096;
-  hipLaunchKernelGGL(k_ns_scale_b16, dim3((unsigned)blocks), dim3(256), 0, stream, static_cast<const uint16_t*>(g),
+  hipLaunchKernelGGL(k_ns_scale_b16, dim3((unsigned)blocks, (unsigned)batch), dim3(256), 0, stream, static_cast<const uint16_t*>(g),
                      n, part, static_cast<uint16_t*>(x));
   return check_launch("ns_normalize");
 }

@@ -71,6 +71,15 @@ def newton_schulz(G: torch.Tensor, steps: int = 5) -> torch.Tensor:
     X = K.ns_normalize(G)                        # one fused two-pass kernel pair
     if m == 0 or n == 0:
         return X
+    if X.dtype == torch.float32 and m % 64 == 0 and n % 64 == 0 and K.few_tiles(m, n):
+        # few tiles: the iterate's and the Gram product's exact bf16 planes, each
+        # written once per step, in the layouts both products read them in
+        for _ in range(steps):
+            pX = K.planes(K.PLANE_SPLIT4, X, None, None, None)
+            pA = K.planes(K.PLANE_SPLIT4, K.gemm_planes(pX, pX, K.F32_PLANE_PAIRS, transpose), None, None, None)
+            a, b = (pX, pA) if transpose else (pA, pX)
+            X = K.ns_combine(X, K.gemm_planes(a, b, K.F32_PLANE_PAIRS, False, b_k_major=not transpose), out=X)
+        return X
     if X.dtype == torch.float32:
         # A tall G is iterated untransposed: with Y = X^T, X X^T = Y^T Y and
         # ((X X^T) X)^T = Y (Y^T Y), so Y <- 1.5 Y - 0.5 Y (Y^T Y) is the
@@ -84,31 +93,54 @@ def newton_schulz(G: torch.Tensor, steps: int = 5) -> torch.Tensor:
                 B = K.matmul_f32(A, X)                # A X     [m, n]
             X = K.ns_combine(X, B, out=X)
         return X
-    # bf16: the kernel takes sides that are multiples of 64, so the iterate
+    return _newton_schulz_bf16(X[None], steps)[0]
+
+
+def _newton_schulz_bf16(X: torch.Tensor, steps: int) -> torch.Tensor:
+    """The iteration of each slice of a normalized bf16 [layers, m, n] array."""
+    L, m, n = (int(d) for d in X.shape)
+    transpose = m > n
+    # the kernel takes sides that are multiples of 64, so the iterate
     # is zero-padded to them; the pad rows and columns stay exactly zero
     # through every product and combination, and the products over the
     # original block are sums of the same bf16 products (plus exact zeros)
     mp, npad = -(-m // 64) * 64, -(-n // 64) * 64
     padded = (mp, npad) != (m, n)
     if padded:
-        Xp = torch.zeros((mp, npad), dtype=X.dtype, device=X.device)
-        Xp[:m, :n] = X
+        Xp = torch.zeros((L, mp, npad), dtype=X.dtype, device=X.device)
+        Xp[:, :m, :n] = X
         X = Xp
+    gram_side = npad if transpose else mp
+    # Short of 256x256 tiles both products run on 128x128 tiles, the first in
+    # full (its triangles hold the same sums: symmetric bit for bit), all layers
+    # at once.  Measured (us, one layer, Gram kernel / 128x128 tiles): sides of
+    # 1024 58 / 30, 2048 (of 8192) 105 / 87, 4096 93 / 124; the combination in
+    # the epilogue alike ([1024, 4096] 34 / 28, [2048, 2048] 57 / 36, [2048,
+    # 8192] 69 / 80); two layers of [1024, 4096] cost 1.3 of one, whose K steps
+    # have to be split to fill the chip.
+    if gram_side <= 2048 and K.few_tiles(mp, npad):
+        for _ in range(steps):
+            A = K.gemm_planes_batch(X, X, transpose, torch.bfloat16)
+            a, b = (X, A) if transpose else (A, X)
+            X = K.gemm_planes_batch(a, b, False, torch.bfloat16, x=X, b_k_major=not transpose)
+    else:
+        X = [_newton_schulz_slice(X[l], gram_side, steps) for l in range(L)]
+        X = X[0][None] if L == 1 else torch.stack(X)
+    return X[:, :m, :n].contiguous() if padded else X
+
+
+def _newton_schulz_slice(X: torch.Tensor, gram_side: int, steps: int) -> torch.Tensor:
+    """The iteration of one slice (sides multiples of 64)."""
+    mp, npad = int(X.shape[0]), int(X.shape[1])
+    transpose = mp > npad
     # the Gram product computes only its upper-triangle tiles (exactly
     # symmetric result) where its side is a multiple of 256; a tall iterate
     # is read K-major by it, with no transposed copy
-    gram_side = npad if transpose else mp
-    gram_ok = gram_side % 256 == 0
-    # Short of 256x256 tiles both products run on 128x128 tiles, the first in
-    # full (its triangles hold the same sums: symmetric bit for bit).  Measured
-    # (us, Gram kernel / 128x128 tiles): sides of 1024 58 / 30, 2048 (of 8192)
-    # 105 / 87, 4096 93 / 124; the combination in the epilogue alike
-    # ([1024, 4096] 34 / 28, [2048, 2048] 57 / 36, [2048, 8192] 69 / 80).
-    gram_few, ns_few = gram_side <= 2048, K.few_tiles(mp, npad)
+    gram_few, gram_ok, ns_few = gram_side <= 2048, gram_side % 256 == 0, K.few_tiles(mp, npad)
     for _ in range(steps):
         # A = X X^T [m, m], or X^T X [n, n] of a tall iterate
         if gram_few:
-            A = K.gemm_planes(X[None], X[None], [(0, 0)], transpose, torch.bfloat16)
+            A = K.gemm_planes(X[None], X[None], ((0, 0),), transpose, torch.bfloat16)
         elif gram_ok:
             A = K.gemm_bf16_gram(X, k_major=transpose)
         elif transpose:
@@ -123,14 +155,14 @@ def newton_schulz(G: torch.Tensor, steps: int = 5) -> torch.Tensor:
         # 4096] 1.08 vs 1.13 ms, [4096, 16384] 3.83 vs 3.74 ms for 5 iterations)
         if ns_few:
             a, b = (X, A) if transpose else (A, X)
-            X = K.gemm_planes(a[None], b[None], [(0, 0)], False, torch.bfloat16, x=X, b_k_major=not transpose)
+            X = K.gemm_planes(a[None], b[None], ((0, 0),), False, torch.bfloat16, x=X, b_k_major=not transpose)
         elif transpose:
             X = K.gemm_bf16_nt_ns(X, A, X)
         elif npad > mp:
             X = K.gemm_bf16_nt_ns(A, X, X, b_k_major=True)
         else:
             X = K.gemm_bf16_nt_ns(A, K.transpose_b16(X), X)
-    return X[:m, :n].contiguous() if padded else X
+    return X
 
 
 class MiulionState(NamedTuple):
@@ -265,6 +297,40 @@ def _quantized_slice_step(path, g, m_t, p_t, tgrid, dtype, beta1, beta2, ns_step
     return upd, new_m
 
 
+# Elements of a stacked leaf that one pass takes at once (bounds its
+# intermediates: the direction and the new momentum before requantization).
+_STACK_ELEMENTS = 1 << 28
+
+
+def _quantized_stack_step(path, g, m_t, p_t, tgrid, beta1, beta2, ns_steps, lion_lr, muon_lr, wd):
+    """_quantized_slice_step of every layer of a stacked leaf (bf16), all layers
+    in one pass of each kernel: (update, new momentum triple).  ``g``: a triple
+    or a tensor of the leaf's shape."""
+    dt = torch.bfloat16
+    L, m, n = (int(d) for d in m_t[0].shape)
+    run = max(1, _STACK_ELEMENTS // max(1, m * n))
+    parts = []
+    for l in range(0, L, run):
+        at = lambda t: t[l:l + run]     # noqa: E731
+        gl = tuple(at(t) for t in g) if isinstance(g, tuple) else at(g)
+        c, nm = K.momentum(tuple(at(t) for t in m_t), gl, tgrid, dt, _as_dtype(beta1, dt), _as_dtype(1.0 - beta1, dt),
+                           _as_dtype(beta2, dt), _as_dtype(1.0 - beta2, dt))
+        new_m = K.quantize(nm, tgrid)
+        muon = _should_use_muon(path, 2)
+        lr = muon_lr if muon else lion_lr
+        if muon and m and n:
+            k = int(c.shape[0])
+            x = K.ns_normalize_batch(c) if (m * n) % 8 == 0 else torch.stack([K.ns_normalize(c[i]) for i in range(k)])
+            c = _newton_schulz_bf16(x, ns_steps)
+        upd = K.apply_update(c, not muon, _as_dtype(math.sqrt(max(m, n)), dt) if muon else 0.0,
+                             tuple(at(t) for t in p_t), tgrid, dt, lr, _f32(lr * np.float32(wd)), dt)
+        parts.append((upd,) + new_m)
+    if len(parts) == 1:
+        return parts[0][0], parts[0][1:]
+    out = [torch.cat([p[i].view(torch.uint8) if p[i].element_size() == 1 else p[i] for p in parts]) for i in range(4)]
+    return out[0], (out[1].view(m_t[0].dtype), out[2].view(m_t[1].dtype), out[3])
+
+
 def miulion_optimizer(hyperparams: MiulionHyperParams, scheduler: MiulionScheduler) -> GradientTransformation:
     """The quantized Miulion transformation (``_optimizer.py:62-217``)."""
     beta1 = hyperparams.beta1
@@ -304,6 +370,11 @@ def miulion_optimizer(hyperparams: MiulionHyperParams, scheduler: MiulionSchedul
                     g8, gs8, gs32 = _triple(g)
                 else:
                     gv = g.get_value() if _is_q(g) else g
+                if tuple((g8 if gq else gv).shape) == tuple(p8.shape) == tuple(m8.shape) and p8.shape[0] > 0:
+                    upd, triple = _quantized_stack_step(
+                        path, (g8, gs8, gs32) if gq else gv.to(torch.bfloat16), (m8, ms8, ms32), (p8, ps8, ps32),
+                        tgrid, beta1, beta2, ns_steps, lion_lr, muon_lr, wd)
+                    return upd, QArrayImpl._tree_unflatten((True, tgrid), triple)
                 ups, n8, ns8, ns32 = [], [], [], []
                 for l in range(p8.shape[0]):
                     g_l = (g8[l], gs8[l], gs32[l]) if gq else gv[l].to(torch.bfloat16)

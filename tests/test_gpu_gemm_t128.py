@@ -203,3 +203,56 @@ def test_fake_quantization_of_narrow_row_blocks(xdt, tgrid, out, fix_nan):
     y = O.bf16_round(y) if xdt == "bf16" else y
     dev = to_dev_bf16(O.f32_to_bf16_bits(y)) if xdt == "bf16" else to_dev_f32(y)
     check(dev, y, tgrid, out, fix_nan, f"ragged {xdt} {tgrid}->{out} fix {fix_nan}")
+
+
+@pytest.mark.parametrize("a_t", [False, True])
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M,N,Kd", [(40, 8, 64), (264, 136, 192), (136, 520, 200), (1024, 1024, 1024)])
+@pytest.mark.parametrize("bdt", [torch.float32, torch.bfloat16])
+def test_matmul_f32_layouts(a_t, b_t, M, N, Kd, bdt):
+    """f32 products of few tiles from planes in the operands' own layouts (and
+    the packed pieces where a layout does not fit: K = 200), with an inf in each
+    operand: finite elements to f32 accuracy, the others where float64 has them."""
+    K = _K()
+    a = _randn((Kd, M) if a_t else (M, Kd), 1) * torch.exp(_randn((1,), 2))
+    b = _randn((N, Kd) if b_t else (Kd, N), 3, bdt)
+    if Kd == 192:
+        a[3, 5], b[7, 2] = float("inf"), float("-inf")
+    ref = (a.T if a_t else a).double() @ (b.T if b_t else b).double()
+    c = K.matmul_f32(a, b, a_t, b_t)
+    ok = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(c), ok) and _rel(torch.where(ok, c, 0.0), torch.where(ok, ref, 0.0)) <= TOL
+    if a_t and not b_t and bdt == torch.float32:
+        assert _rel(K.matmul_f32(a, a, True, False), a.double().T @ a.double()) <= TOL or Kd == 192
+
+
+def test_batched_slices():
+    """Batches of products and normalizations against their slices, K split or
+    not, and a stacked optimizer leaf in runs of one layer against all at once."""
+    from pratchya_amd import optim
+    K = _K()
+    for shape in [(3, 320, 512), (2, 1024, 4096), (5, 256, 64)]:
+        x = _randn(shape, 1, torch.bfloat16)
+        for km in (False, True):
+            c = K.gemm_planes_batch(x, x, km, torch.bfloat16)
+            assert torch.equal(c, c.transpose(1, 2))
+            ref = (x.transpose(1, 2).float() @ x.float()) if km else (x.float() @ x.transpose(1, 2).float())
+            assert _rel(c.float(), ref.double()) <= 2.0 ** -8
+        a = K.gemm_planes_batch(x, x, False, torch.bfloat16)
+        y = K.gemm_planes_batch(a, x, False, torch.bfloat16, x=x, b_k_major=True)
+        for i in range(shape[0]):
+            p = (a[i].float() @ x[i].float()).to(torch.bfloat16)
+            assert _rel(y[i].float(), K.ns_combine(x[i], p).double()) <= 2.0 ** -6
+            assert torch.equal(K.ns_normalize_batch(x)[i], K.ns_normalize(x[i]))
+    grid, sh = (64, 64), (3, 128, 192)
+    mom, par = (K.quantize(_randn(sh, s) * 1e-3, grid) for s in (4, 5))
+    args = (("layers",), _randn(sh, 6, torch.bfloat16), mom, par, grid, 0.9, 0.99, 5, 3e-4, 0.02, 0.1)
+    one, prev = optim._quantized_stack_step(*args), optim._STACK_ELEMENTS
+    try:
+        optim._STACK_ELEMENTS = 1
+        runs = optim._quantized_stack_step(*args)
+    finally:
+        optim._STACK_ELEMENTS = prev
+    assert _rel(runs[0].float(), one[0].double()) <= 3e-2
+    for p, q in zip(one[1], runs[1]):
+        assert p.dtype == q.dtype and torch.equal(p.view(torch.uint8), q.view(torch.uint8))
