@@ -373,8 +373,9 @@ int pratchya_gemm_bs_nt_fq(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, 
  * (PRATCHYA_EUNSUPPORTED otherwise).  C [M, N] receives the dequantized values
  * in c_dtype, c_sc8 [M * N] the e8m0 bytes and c_sc32 [M * N] the group maxima
  * (both in row order, 16-byte aligned), the arrays quantize_impl(C_f32, (1, 1))
- * returns.  The results equal pratchya_gemm_bs_nt to f32 followed by
- * pratchya_quantize_dequantize with tgrid (1, 1) bit for bit. */
+ * returns; both null: the scales are not stored.  The results equal
+ * pratchya_gemm_bs_nt to f32 followed by pratchya_quantize_dequantize with
+ * tgrid (1, 1) bit for bit. */
 int pratchya_gemm_bs_nt_q11(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, const float* a_sc32,
                             int64_t a_rdiv, int64_t a_sr, int64_t a_sk, int64_t a_kg,
                             const uint8_t* B, int64_t ldb, const uint8_t* b_sc8, const float* b_sc32,

@@ -1232,14 +1232,16 @@ def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = F
     return y, sc8.view(E8M0), sc32
 
 
-def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None, few: bool = False):
+def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None, few: bool = False,
+                scales: bool = True):
     """``QArrayImpl(dequant(a) @ dequant(b)^T, (1, 1)).astype(out_dtype)``
     with the requantization in the GEMM's epilogue (the output grid of a
     weight quantized (a, 1): lm_head, LoRA): returns ``(y [M, N], sc_fp8,
     sc_fp32)`` bit-identical to ``quantize_dequantize(gemm_nt(a, b, float32),
     (1, 1), out_dtype)``, the scales shaped per slice of ``lead`` as there.
     Raises ``PratchyaUnsupported`` unless N is a multiple of 16.  ``few``: as
-    for gemm_nt_fq."""
+    for gemm_nt_fq.  Without ``scales`` the scale arrays, five of the seven
+    bytes written per bf16 element, are neither allocated nor stored (None)."""
     _require_gpu(a.payload, b.payload)
     if a.k != b.k:
         raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
@@ -1260,13 +1262,16 @@ def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None, few: 
         S *= int(d)
     H = M // S
     y = torch.empty((M, N), dtype=out_dtype, device=ap.device)
-    sc8 = torch.empty(tuple(lead[:-1]) + (H * N, 1), dtype=torch.uint8, device=ap.device)
-    sc32 = torch.empty(tuple(lead[:-1]) + (H * N, 1, 1), dtype=torch.float32, device=ap.device)
+    sc8 = sc32 = None
+    if scales:
+        sc8 = torch.empty(tuple(lead[:-1]) + (H * N, 1), dtype=torch.uint8, device=ap.device)
+        sc32 = torch.empty(tuple(lead[:-1]) + (H * N, 1, 1), dtype=torch.float32, device=ap.device)
     _lib.check(lib.pratchya_gemm_bs_nt_q11(_ptr(ap), K, _ptr(as8), _ptr(as32), *a.desc,
                                            _ptr(bp), K, _ptr(bs8), _ptr(bs32), *b.desc,
                                            M, N, K, _ptr(y), N, _dtype_code(out_dtype),
-                                           _ptr(sc8), _ptr(sc32), _stream(ap)), "gemm_q11")
-    return y, sc8.view(E8M0), sc32
+                                           _ptr(sc8) if scales else None, _ptr(sc32) if scales else None,
+                                           _stream(ap)), "gemm_q11")
+    return y, None if sc8 is None else sc8.view(E8M0), sc32
 
 
 def gemm_nt_qa(x: torch.Tensor, b: Operand, out_dtype: torch.dtype, fq: bool = False, lead=None,

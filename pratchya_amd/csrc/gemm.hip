@@ -1011,7 +1011,9 @@ __device__ __forceinline__ void store_block_max(uint32_t lmax, uint32_t* slot, c
 // the bytes in a pass of their own); every array leaves the slice as whole
 // 16-byte chunks, consecutive lanes on consecutive chunks of a row, so that
 // each store instruction writes whole lines (non-temporal).  N is a multiple
-// of 16, so no chunk straddles the edge of a partial tile.
+// of 16, so no chunk straddles the edge of a partial tile.  Null scale arrays
+// are left out, five of the seven bytes of a bf16 element (a forward without
+// gradients: a Linear of [2048, 2048] . [2048, 32768] 223 -> 177 us).
 template <bool OUT_BF16, int BG>
 __device__ __forceinline__ void store_tile_q11(const v16f (&acc)[2][4], const float (&gA)[2],
                                                const float (&gB)[4][BG == 1 ? 4 : 1], const uint8_t* ub,
@@ -1068,7 +1070,7 @@ __device__ __forceinline__ void store_tile_q11(const v16f (&acc)[2][4], const fl
       __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave's staging writes are done
       const int rbase = row0 + mi * 32 + p * RP;
       // group maxima |c|
-      copy_out(reinterpret_cast<uint8_t*>(sc32 + col0), (int64_t)N * 4, 0, 512, 4, rbase, true);
+      if (sc32) copy_out(reinterpret_cast<uint8_t*>(sc32 + col0), (int64_t)N * 4, 0, 512, 4, rbase, true);
       // the lane's segments: values 16 s + [0, 16) of staged row r, for
       // q = lane + 64 h (r = q / 8, s = q % 8): half h reads rows 8 h + [0, 8)
       // and writes its results back into the same rows once every lane's
@@ -1119,6 +1121,7 @@ __device__ __forceinline__ void store_tile_q11(const v16f (&acc)[2][4], const fl
       __builtin_amdgcn_s_waitcnt(0xC07F);
       uint8_t* Cb = static_cast<uint8_t*>(C) + (int64_t)col0 * ESZ;
       copy_out(Cb, ldc * ESZ, 0, 128 * ESZ, 16 / ESZ, rbase, false);
+      if (!sc8) continue;
       if constexpr (!OUT_BF16) {
         // the f32 values filled the rows: the e8m0 bytes in a pass of their own
 #pragma unroll
@@ -2084,8 +2087,8 @@ extern "C" int pratchya_gemm_bs_nt_q11(const uint8_t* A, int64_t lda, const uint
   if (N % 16)
     return pratchya_set_error(PRATCHYA_EUNSUPPORTED, "gemm_q11: N must be a multiple of 16 (got %lld)",
                               (long long)N);
-  if (!c_sc8 || !c_sc32 || (reinterpret_cast<uintptr_t>(c_sc8) & 15) || (reinterpret_cast<uintptr_t>(c_sc32) & 15))
-    return pratchya_set_error(PRATCHYA_EINVAL, "gemm_q11: the scale arrays must be 16-byte aligned device memory");
+  if ((!c_sc8) != (!c_sc32) || (reinterpret_cast<uintptr_t>(c_sc8) & 15) || (reinterpret_cast<uintptr_t>(c_sc32) & 15))
+    return pratchya_set_error(PRATCHYA_EINVAL, "gemm_q11: the scale arrays must be 16-byte aligned device memory, or both null");
   GemmPlan P;
   int rc = gemm_plan("gemm_q11", A, lda, a_sc8, a_sc32, a_rdiv, a_sr, a_sk, a_kg, B, ldb, b_sc8, b_sc32, b_rdiv,
                      b_sr, b_sk, b_kg, M, N, K, C, ldc, c_dtype, &P);

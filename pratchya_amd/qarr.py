@@ -538,14 +538,16 @@ class _Matmul(torch.autograd.Function):
         return grad_x, grad_y, None, None, None, None, None, None, None, None
 
 
-def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype):
+def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype, scales=True):
     """``QArrayImpl(matmul_impl(x, y), go).astype(dtype)`` with the
     requantization in the GEMM's epilogue: ``(y, sc_fp8, sc_fp32)`` bit-identical
     to the f32 product followed by ``quantize_dequantize``, or None when the
     layouts do not fit.  ``go`` (1, 128), a quantized Linear's output, takes
     N a multiple of 1024 (its groups span four output tiles); (1, 1), the
     output of a weight quantized (a, 1) (lm_head, LoRA), N a multiple of 16.
-    (Products of few tiles run as the two steps: ``K.prefers_t128``.)"""
+    (Products of few tiles run as the two steps: ``K.prefers_t128``.)
+    ``scales`` False: the caller keeps only y; the (1, 1) scales, larger than
+    y itself, are then not stored."""
     go = tuple(go)
     if go not in ((1, 128), (1, 1)) or dtype not in (torch.float32, torch.bfloat16) or y8.dim() != 2:
         return None
@@ -559,7 +561,7 @@ def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype):
     lead = tuple(x8.shape[:-1])
     try:
         if go == (1, 1):
-            res, s8, s32 = K.gemm_nt_q11(op_a, op_b, dtype, lead=lead, few=True)
+            res, s8, s32 = K.gemm_nt_q11(op_a, op_b, dtype, lead=lead, few=True, scales=scales)
         else:
             res, s8, s32 = K.gemm_nt_fq(op_a, op_b, dtype, lead=lead, few=True)
     except K.PratchyaUnsupported:
@@ -1259,7 +1261,7 @@ class _LazyProduct(QArrayImpl):
             if sx is not None or sy is not None:
                 res = _QLinear.apply(sx, sy, x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype)
             else:
-                fused = _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype)
+                fused = _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype, scales=False)
                 if fused is not None:
                     res = fused[0]
                 else:

@@ -226,6 +226,20 @@ def test_matmul_f32_layouts(a_t, b_t, M, N, Kd, bdt):
         assert _rel(K.matmul_f32(a, a, True, False), a.double().T @ a.double()) <= TOL or Kd == 192
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(4300, 256, 2048), (4353, 384, 1040), (70000, 128, 48)])
+def test_one_by_one_epilogue_without_scales(shape, dt):
+    """The (1, 1) epilogue with its scale arrays left out stores the same values."""
+    K = _K()
+    M, Kd, N = shape
+    a = K.operand_rows(*K.quantize(_randn((M, Kd), 1, torch.bfloat16), (1, 128)), (1, 128))
+    b = K.operand_transposed(*K.quantize(_randn((Kd, N), 2, torch.bfloat16) * 0.02, (128, 1)), (128, 1))
+    y, s8, s32 = K.gemm_nt_q11(a, b, dt)
+    z, n8, n32 = K.gemm_nt_q11(a, b, dt, scales=False)
+    assert n8 is None and n32 is None and s8 is not None and s32 is not None
+    assert torch.equal(y, z)
+
+
 def test_batched_slices():
     """Batches of products and normalizations against their slices, K split or
     not, and a stacked optimizer leaf in runs of one layer against all at once."""
