@@ -21,9 +21,11 @@
 //   * one pass: result grid (1, b) with b a multiple of 16 and groups of at
 //     most 1024 contiguous elements.  A wave owns 1024 results (16 per lane):
 //     block and group maxima by lane shuffles, e8m0 scales, payload;
-//   * general (any grid, four launches): the block maxima of the results into
-//     a workspace with atomics, the group scales, then a second pass that
-//     recomputes the results and casts them.  The operands are read twice.
+//   * general (any grid): the block maxima of the results into a workspace,
+//     then a second pass that recomputes the results and casts them (two
+//     launches, a workgroup per block, where tile_fits; else four: a fill,
+//     maxima with atomics, the group scales, the cast).  The operands are
+//     read twice.
 // The operands may have block grids of their own (QArrayImpl's operators on
 // arrays quantized with different grids dequantize each with its own grid);
 // every grid divides the slice shape.
@@ -360,6 +362,79 @@ __global__ __launch_bounds__(256) void k_ew_cast(QOperand X, QOperand Y, uint8_t
   }
 }
 
+// Workgroup per result block (tile_fits), 16 results per thread and step.
+template <int OP>
+__global__ __launch_bounds__(256) void k_ew_tile_max(QOperand X, QOperand Y, uint32_t* __restrict__ ws, int64_t W,
+                                                     int a, int b, int seg_log2) {
+  constexpr int U = 4;
+  __shared__ uint32_t lds[4];
+  const uint32_t blk = blockIdx.x, bpr = (uint32_t)(W / b), bi = blk / bpr, bj = blk - bi * bpr;
+  const int RT = 256 >> seg_log2, r0 = threadIdx.x >> seg_log2;
+  const int64_t i0 = (int64_t)bi * a, c = (int64_t)bj * b + (threadIdx.x & ((1 << seg_log2) - 1)) * 16;
+  uint32_t m = 0;
+  for (int r = r0; r < a; r += U * RT) {
+    float z[U][16];
+    // (past the last row: that row once more)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      ew_chunk<OP, 16, true, int64_t>(X, Y, i0 + (r + u * RT < a ? r + u * RT : a - 1), c, W, z[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < 16; ++k) m = umax(m, abs_bits(z[u][k]));
+  }
+  m = tile_umax(m, lds);
+  if (threadIdx.x == 0) ws[blk] = m;
+}
+
+template <int OP>
+__global__ __launch_bounds__(256) void k_ew_tile_cast(QOperand X, QOperand Y, uint8_t* __restrict__ q,
+                                                      const uint32_t* __restrict__ ws, uint8_t* __restrict__ sc8,
+                                                      float* __restrict__ sc32, int64_t W, int a, int b, int64_t K,
+                                                      int seg_log2) {
+  constexpr int U = 4;
+  __shared__ uint32_t lds[4];
+  const uint32_t blk = blockIdx.x, bpr = (uint32_t)(W / b), bi = blk / bpr, bj = blk - bi * bpr;
+  const int RT = 256 >> seg_log2, r0 = threadIdx.x >> seg_log2;
+  const int64_t i0 = (int64_t)bi * a, c = (int64_t)bj * b + (threadIdx.x & ((1 << seg_log2) - 1)) * 16;
+  // the first step's loads are in flight while the scales are found
+  float z[U][16];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    ew_chunk<OP, 16, true, int64_t>(X, Y, i0 + (r0 + u * RT < a ? r0 + u * RT : a - 1), c, W, z[u]);
+  uint32_t e;
+  float G;
+  tile_scales(ws, blk, K, sc8, sc32, lds, e, G);
+  const float sG = e8m0_decode(e) * G;
+  const float S = quant_scale(e, G);
+  const bool ok = sG >= kClamp && sG <= 3.0e38f;
+  const float yv = 128.0f / S;
+  for (int r = r0; r < a; r += U * RT) {
+    if (r != r0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        ew_chunk<OP, 16, true, int64_t>(X, Y, i0 + (r + u * RT < a ? r + u * RT : a - 1), c, W, z[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (r + u * RT >= a) break;
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float* v = z[u] + 4 * j;
+        if (ok) {
+          const float t0 = v[0] * yv, t1 = v[1] * yv, t2 = v[2] * yv, t3 = v[3] * yv;
+          w[j] = cvt4_hw(t0, t1, t2, t3);
+          if (mid_key4(t0, t1, t2, t3) <= kMidKey) w[j] = cvt4_exact(v[0], v[1], v[2], v[3], S);
+        } else {
+          w[j] = cvt4_exact(v[0], v[1], v[2], v[3], S);
+        }
+      }
+      store_stream16(q + (i0 + r + u * RT) * W + c, u32x4_t{w[0], w[1], w[2], w[3]});
+    }
+  }
+}
+
 // --------------------------------------------------------------------------
 // Host side
 // --------------------------------------------------------------------------
@@ -444,6 +519,15 @@ template <int OP, int CH, bool VEC, typename I>
 void launch_general_t(const QOperand& X, const QOperand& Y, uint8_t* q, uint8_t* sc8, float* sc32, uint32_t* ws,
                       int64_t n, int64_t W, int64_t a, int64_t b, int64_t K, int64_t n_blk_total,
                       int64_t n_groups, const EwPlan& p, hipStream_t st) {
+  if constexpr (CH == 16 && VEC) {
+    if (tile_fits(a, b, 16, 16, 1, n_blk_total)) {
+      const dim3 grid((unsigned)n_blk_total);
+      hipLaunchKernelGGL((k_ew_tile_max<OP>), grid, dim3(256), 0, st, X, Y, ws, W, (int)a, (int)b, log2_of(b / 16));
+      hipLaunchKernelGGL((k_ew_tile_cast<OP>), grid, dim3(256), 0, st, X, Y, q, ws, sc8, sc32, W, (int)a, (int)b, K,
+                         log2_of(b / 16));
+      return;
+    }
+  }
   const unsigned fill = blocks_for(n_blk_total, 256);
   hipLaunchKernelGGL(k_fill_u32, dim3(fill > 4096 ? 4096 : fill), dim3(256), 0, st, ws, n_blk_total, 0u);
   const int64_t n_chunks = n / CH;

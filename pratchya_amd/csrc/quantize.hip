@@ -528,6 +528,42 @@ __global__ __launch_bounds__(256) void k_blockmax(const void* __restrict__ x,
   }
 }
 
+// CH (a multiple of 4) values of one block as output words, 4 at a time on
+// the hardware conversions: the division-free cast where the block's scale is
+// neither clamped nor huge, each 4-value word with a value near a bf16
+// rounding midpoint redone exactly (the arithmetic of k_quant_g8 and
+// fake_quant4).  OUT as k_cast_general.
+template <int CH, int OUT>
+__device__ __forceinline__ void cast_words(const float (&xv)[CH], float yv, float S, bool ok, float dq,
+                                           uint32_t (&w)[CH / (OUT == 0 ? 4 : (OUT == 1 ? 2 : 1))]) {
+  const bool one = dequant_one_mul(dq);
+  const float dqx = one ? dq * 0.0078125f : dq;
+#pragma unroll
+  for (int q = 0; q < CH / 4; ++q) {
+    float x0 = xv[4 * q], x1 = xv[4 * q + 1], x2 = xv[4 * q + 2], x3 = xv[4 * q + 3];
+    if constexpr (OUT == 0) {
+      if (ok) {
+        const float t0 = x0 * yv, t1 = x1 * yv, t2 = x2 * yv, t3 = x3 * yv;
+        w[q] = cvt4_hw(t0, t1, t2, t3);
+        if (mid_key4(t0, t1, t2, t3) <= kMidKey) w[q] = cvt4_exact(x0, x1, x2, x3, S);
+      } else {
+        w[q] = cvt4_exact(x0, x1, x2, x3, S);
+      }
+    } else {
+      fake_quant4(x0, x1, x2, x3, yv, S, ok, dqx, one);
+      if constexpr (OUT == 1) {
+        w[2 * q] = pack_bf16x2(x0, x1);
+        w[2 * q + 1] = pack_bf16x2(x2, x3);
+      } else {
+        w[4 * q] = f2u(x0);
+        w[4 * q + 1] = f2u(x1);
+        w[4 * q + 2] = f2u(x2);
+        w[4 * q + 3] = f2u(x3);
+      }
+    }
+  }
+}
+
 // Elementwise cast, thread per chunk of CH elements of one block row segment.
 // OUT 0 writes the payload; OUT 1 / 2 write it dequantized as bf16 / f32
 // (fake quantization, with the NaN-e8m0 repair when fix_nan is set), as the
@@ -566,44 +602,19 @@ __global__ __launch_bounds__(256) void k_cast_general(const void* __restrict__ x
   const float dq = e8m0_decode((fix_nan && e == 0xFFu) ? 0x7Fu : e) * G;
   float xv[CH];
   load_chunk<IS_BF16, CH, VEC && (CH * (IS_BF16 ? 2 : 4) >= 16)>(x, (int64_t)off, xv);
+  constexpr int PER = OUT == 0 ? 4 : (OUT == 1 ? 2 : 1);        // elements per output word
   uint32_t ov[CH];                              // output element bits
   if constexpr (CH % 4 == 0) {
-    // 4 values at a time on the hardware conversions: the division-free cast
-    // where the block's scale is neither clamped nor huge, each 4-value word
-    // with a value near a bf16 rounding midpoint redone exactly (the
-    // arithmetic of k_quant_g8 and fake_quant4)
-    const bool one = dequant_one_mul(dq);
-    const float dqx = one ? dq * 0.0078125f : dq;
-#pragma unroll
-    for (int q = 0; q < CH / 4; ++q) {
-      float x0 = xv[4 * q], x1 = xv[4 * q + 1], x2 = xv[4 * q + 2], x3 = xv[4 * q + 3];
-      if constexpr (OUT == 0) {
-        uint32_t w;
-        if (ok) {
-          const float t0 = x0 * yv, t1 = x1 * yv, t2 = x2 * yv, t3 = x3 * yv;
-          w = cvt4_hw(t0, t1, t2, t3);
-          if (mid_key4(t0, t1, t2, t3) <= kMidKey) w = cvt4_exact(x0, x1, x2, x3, S);
-        } else {
-          w = cvt4_exact(x0, x1, x2, x3, S);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ov[4 * q + i] = (w >> (8 * i)) & 0xFFu;
-      } else {
-        fake_quant4(x0, x1, x2, x3, yv, S, ok, dqx, one);
-        if constexpr (OUT == 1) {
-          const uint32_t p0 = pack_bf16x2(x0, x1), p1 = pack_bf16x2(x2, x3);
-          ov[4 * q] = p0 & 0xFFFFu;
-          ov[4 * q + 1] = p0 >> 16;
-          ov[4 * q + 2] = p1 & 0xFFFFu;
-          ov[4 * q + 3] = p1 >> 16;
-        } else {
-          ov[4 * q] = f2u(x0);
-          ov[4 * q + 1] = f2u(x1);
-          ov[4 * q + 2] = f2u(x2);
-          ov[4 * q + 3] = f2u(x3);
-        }
-      }
+    uint32_t w[CH / PER];
+    cast_words<CH, OUT>(xv, yv, S, ok, dq, w);
+    if constexpr (VEC) {
+      static_assert(CH / PER == 4, "a vector chunk is 16 output bytes");
+      char* o = static_cast<char*>(outv) + (int64_t)off * (4 / PER);
+      store_stream16(o, u32x4_t{w[0], w[1], w[2], w[3]});   // a wave's stores: one contiguous span
+      return;
     }
+#pragma unroll
+    for (int k = 0; k < CH; ++k) ov[k] = PER == 1 ? w[k] : (w[k / PER] >> (32 / PER * (k % PER))) & ((1u << (32 / PER % 32)) - 1u);
   } else {
 #pragma unroll
     for (int k = 0; k < CH; ++k) {
@@ -621,28 +632,84 @@ __global__ __launch_bounds__(256) void k_cast_general(const void* __restrict__ x
       }
     }
   }
-  if constexpr (VEC) {
-    // pack into 32-bit words and store them as one 16-byte vector
-    constexpr int PER = OUT == 0 ? 4 : (OUT == 1 ? 2 : 1);      // elements per word
-    static_assert(CH / PER == 4, "a vector chunk is 16 output bytes");
-    uint32_t w[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (PER == 4)
-        w[j] = ov[4 * j] | (ov[4 * j + 1] << 8) | (ov[4 * j + 2] << 16) | (ov[4 * j + 3] << 24);
-      else if constexpr (PER == 2)
-        w[j] = ov[2 * j] | (ov[2 * j + 1] << 16);
-      else
-        w[j] = ov[j];
+  for (int k = 0; k < CH; ++k) {
+    if constexpr (OUT == 0) static_cast<uint8_t*>(outv)[off + k] = (uint8_t)ov[k];
+    else if constexpr (OUT == 1) static_cast<uint16_t*>(outv)[off + k] = (uint16_t)ov[k];
+    else static_cast<float*>(outv)[off + k] = u2f(ov[k]);
+  }
+}
+
+// Workgroup per block (tile_fits).  The threads lie on the block's row
+// segments, RT = 256 >> seg_log2 rows at a time, four steps' loads in flight.
+// [2048, 8192] in blocks of 128, flat kernels before: bf16 to payloads 25.7 ->
+// 12.2 us, f32 to bf16 (a weight's gradient) 36.5 -> 29.2 us; [512, 1024]
+// 10.2 -> 7.1 and 10.8 -> 9.5 us; [4096, 16384] 60 -> 61 and 104 -> 99 us.
+template <bool IS_BF16>
+__global__ __launch_bounds__(256) void k_tile_max(const void* __restrict__ x, uint32_t* __restrict__ ws, int64_t W,
+                                                  int a, int b, int seg_log2) {
+  constexpr int CH = IS_BF16 ? 8 : 4, U = 4;
+  __shared__ uint32_t lds[4];
+  const uint32_t blk = blockIdx.x, bpr = (uint32_t)(W / b), bi = blk / bpr, bj = blk - bi * bpr;
+  const int RT = 256 >> seg_log2, r0 = threadIdx.x >> seg_log2, c = (threadIdx.x & ((1 << seg_log2) - 1)) * CH;
+  const int64_t base = (int64_t)bi * a * W + (int64_t)bj * b + c;
+  uint32_t m = 0;
+  for (int r = r0; r < a; r += U * RT) {
+    float v[U][CH];
+    // (past the last row: that row once more)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      load_chunk<IS_BF16, CH, true>(x, base + (int64_t)(r + u * RT < a ? r + u * RT : a - 1) * W, v[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < CH; ++k) m = umax(m, abs_bits(v[u][k]));
+  }
+  m = tile_umax(m, lds);
+  if (threadIdx.x == 0) ws[blk] = m;
+}
+
+// (elements per thread: 16 bytes of the output, and of the input at least)
+constexpr int tile_cast_chunk(bool bf16, int out) { return out == 0 ? 16 : (out == 1 || bf16 ? 8 : 4); }
+
+template <bool IS_BF16, int OUT>
+__global__ __launch_bounds__(256) void k_tile_cast(const void* __restrict__ x, void* __restrict__ outv,
+                                                   const uint32_t* __restrict__ ws, uint8_t* __restrict__ sc8,
+                                                   float* __restrict__ sc32, int64_t W, int a, int b, int64_t K,
+                                                   int seg_log2, int fix_nan) {
+  constexpr int CH = tile_cast_chunk(IS_BF16, OUT), OSZ = OUT == 0 ? 1 : (OUT == 1 ? 2 : 4), U = 4;
+  __shared__ uint32_t lds[4];
+  const uint32_t blk = blockIdx.x, bpr = (uint32_t)(W / b), bi = blk / bpr, bj = blk - bi * bpr;
+  const int RT = 256 >> seg_log2, r0 = threadIdx.x >> seg_log2, c = (threadIdx.x & ((1 << seg_log2) - 1)) * CH;
+  const int64_t base = (int64_t)bi * a * W + (int64_t)bj * b + c;
+  // the first step's loads are in flight while the scales are found
+  float v[U][CH];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    load_chunk<IS_BF16, CH, true>(x, base + (int64_t)(r0 + u * RT < a ? r0 + u * RT : a - 1) * W, v[u]);
+  uint32_t e;
+  float G;
+  tile_scales(ws, blk, K, sc8, sc32, lds, e, G);
+  const float sG = e8m0_decode(e) * G;
+  const float S = quant_scale(e, G);
+  const bool ok = sG >= kClamp && sG <= 3.0e38f;
+  const float yv = 128.0f / S;
+  const float dq = e8m0_decode((fix_nan && e == 0xFFu) ? 0x7Fu : e) * G;
+  for (int r = r0; r < a; r += U * RT) {
+    if (r != r0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        load_chunk<IS_BF16, CH, true>(x, base + (int64_t)(r + u * RT < a ? r + u * RT : a - 1) * W, v[u]);
     }
-    char* o = static_cast<char*>(outv) + (int64_t)off * (OUT == 0 ? 1 : (OUT == 1 ? 2 : 4));
-    store_stream16(o, u32x4_t{w[0], w[1], w[2], w[3]});   // a wave's stores: one contiguous span
-  } else {
 #pragma unroll
-    for (int k = 0; k < CH; ++k) {
-      if constexpr (OUT == 0) static_cast<uint8_t*>(outv)[off + k] = (uint8_t)ov[k];
-      else if constexpr (OUT == 1) static_cast<uint16_t*>(outv)[off + k] = (uint16_t)ov[k];
-      else static_cast<float*>(outv)[off + k] = u2f(ov[k]);
+    for (int u = 0; u < U; ++u) {
+      if (r + u * RT >= a) break;
+      uint32_t w[CH * OSZ / 4];
+      cast_words<CH, OUT>(v[u], yv, S, ok, dq, w);
+#pragma unroll
+      for (int j = 0; j < CH * OSZ / 16; ++j)
+        store_stream16(static_cast<char*>(outv) + (base + (int64_t)(r + u * RT) * W) * OSZ + 16 * j,
+                       u32x4_t{w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]});
     }
   }
 }
@@ -1134,6 +1201,16 @@ int launch_general(const void* x, void* q, uint8_t* sc8, float* sc32, uint32_t* 
                    const Layout& L, hipStream_t st, int fix_nan = 0, bool premax = false) {
   const int64_t n_blocks_total = L.S * L.n_blk;
   const int64_t n_groups = L.S * L.M;
+  constexpr int CIN = IS_BF16 ? 8 : 4, COUT = tile_cast_chunk(IS_BF16, OUT);
+  if (tile_fits(L.a, L.b, CIN, COUT, OUT == 0 ? 1 : (OUT == 1 ? 2 : 4), n_blocks_total) && aligned(x, 16) && aligned(q, 16)) {
+    const dim3 grid((unsigned)n_blocks_total);
+    if (!premax)
+      hipLaunchKernelGGL((k_tile_max<IS_BF16>), grid, dim3(256), 0, st, x, ws, L.W, (int)L.a, (int)L.b,
+                         ilog2(L.b / CIN));
+    hipLaunchKernelGGL((k_tile_cast<IS_BF16, OUT>), grid, dim3(256), 0, st, x, q, ws, sc8, sc32, L.W, (int)L.a,
+                       (int)L.b, L.K, ilog2(L.b / COUT), fix_nan);
+    return check_launch("quantize(block)");
+  }
   if (!premax)
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n_blocks_total, 256) > 4096 ? 4096 : grid_for(n_blocks_total, 256)),
                        dim3(256), 0, st, ws, n_blocks_total, 0u);

@@ -1,0 +1,69 @@
+"""Quantization with a workgroup per block (grids whose block is 4096 to 65536
+elements in rows of 64 or more) against the oracle and, bit for bit, against
+the flat kernels, which take the same values from an unaligned buffer."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import qarr_oracle as O
+from tests.helpers import assert_bytes_equal, assert_f32_bits_equal, f32, u8
+
+pytestmark = pytest.mark.gpu
+
+# (shape, grid): rows not a multiple of a step, one row step, several slices,
+# the widest and smallest blocks, one group over the array, one block per group
+CASES = [((3, 256, 384), (128, 128)), ((200, 192), (100, 64)), ((64, 64), (64, 64)), ((130, 1024), (65, 128)),
+         ((256, 512), (128, 512)), ((48, 1024), (16, 256)), ((1024, 64), (1024, 64)), ((1024, 1024), (128, 128)),
+         ((96, 128), (32, 128)), ((255, 256), (255, 256))]
+
+
+def _values(shape, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(shape, generator=g, device="cuda") * torch.exp2(
+        torch.randint(-12, 13, shape[:-1] + (1,), generator=g, device="cuda").float())
+    x = x.view(-1, shape[-1])
+    x[:, 5] = 0.0
+    if x.shape[0] >= 200:
+        x[: x.shape[0] // 2, : shape[-1] // 2] *= 1e-12
+        x[-1, -1], x[-2, 0] = float("inf"), float("nan")
+    return x.view(shape).to(dtype)
+
+
+def _unaligned(x):
+    buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)
+    y = buf[1:].view(x.shape)
+    y.copy_(x)
+    return y
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,grid", CASES, ids=lambda v: "x".join(map(str, v)))
+def test_block_per_workgroup(shape, grid, dtype):
+    from pratchya_amd import _kernels as K
+    x = _values(shape, dtype, 7)
+    other = _unaligned(x)
+    q, s8, s32 = K.quantize(x, grid)
+    for got, want in zip(K.quantize(other, grid), (q, s8, s32)):
+        assert_bytes_equal(u8(got.contiguous().view(torch.uint8)), u8(want.contiguous().view(torch.uint8)), "flat")
+    wq, we, wg = O.quantize_impl(f32(x), grid)
+    assert_bytes_equal(u8(s8).reshape(-1), we.view(np.uint8).reshape(-1), "e8m0")
+    assert_f32_bits_equal(f32(s32).reshape(-1), wg.reshape(-1), "group maxima")
+    for out in (torch.bfloat16, torch.float32):
+        for fix in (False, True):
+            a, b = K.quantize_dequantize(x, grid, out, fix), K.quantize_dequantize(other, grid, out, fix)
+            for got, want in zip(a, b):
+                assert torch.equal(got.contiguous().view(torch.uint8), want.contiguous().view(torch.uint8))
+
+
+@pytest.mark.parametrize("ids_shape,out_grid", [((256,), (128, 128)), ((2, 192), (64, 64)), ((100,), (50, 128)),
+                                                ((640,), (128, 256))])
+def test_gathered_rows(ids_shape, out_grid):
+    """Looked-up rows requantized with a workgroup per block against the rows'
+    values quantized by themselves; indices out of range, negative and equal."""
+    from pratchya_amd import _kernels as K
+    table = K.quantize(_values((384, 512), torch.bfloat16, 3), (128, 128))
+    ids = torch.randint(-384, 384, ids_shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    ids.view(-1)[:4] = torch.tensor([0, 383, 100000, -100000], device="cuda")
+    rows = K.gather_dequantize(*table, (128, 128), ids, torch.float32)
+    for got, want in zip(K.gather_quantize(*table, (128, 128), ids, out_grid), K.quantize(rows, out_grid)):
+        assert torch.equal(got.contiguous().view(torch.uint8), want.contiguous().view(torch.uint8))
