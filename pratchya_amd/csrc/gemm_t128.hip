@@ -120,8 +120,9 @@ __device__ __forceinline__ v8i read_frag_tn(const uint8_t* base) {
 // finite).
 __device__ __forceinline__ float mantissa_unit(float g) {
   const uint32_t b = f2u(g) & 0x7FFFFFFFu;
-  if (b == 0u || b >= 0x7F800000u) return 1.0f;
-  return b < 0x00800000u ? g * 0x1p126f : u2f((f2u(g) & 0x807FFFFFu) | 0x3F800000u);
+  const float normal = u2f((f2u(g) & 0x807FFFFFu) | 0x3F800000u);
+  const float unit = b < 0x00800000u ? g * 0x1p126f : normal;
+  return b - 1u < 0x7F7FFFFFu ? unit : 1.0f;    // selects: branches here would cut the step into pieces
 }
 
 // 1.5 x - 0.5 b on bf16 pairs, each operation rounded (k_ns_combine's bits).
@@ -149,9 +150,10 @@ __device__ __forceinline__ void wg_barrier() {
 // maxima, 3 and 4: bf16 power-of-two planes of payloads quantized in blocks of
 // 16 or 32 along K, the mantissas of both operands' group maxima per block: an
 // MFMA's sums over one block (two MFMAs' over 32) join the total times both.
-// These two are bound by the multiply-adds that join them (16 per lane and
-// MFMA, 64 clocks beside its 32): 8192 x [4096, 4096] 402 us in blocks of 32
-// and 508 in blocks of 16, where the six-pair f32 product took 1585.  flags (bf16): flags[0] == 0 says that the planes of the segments
+// The joins (16 multiply-adds per lane and MFMA, 64 clocks beside its 32) run
+// as a pipeline with the MFMAs (fine_step), where one after the other they left
+// both units waiting: forward of 8192 x [4096, 4096] in blocks of 32 469 -> 426
+// us, of which the product is about 330 (the six-pair f32 product took 1585).  flags (bf16): flags[0] == 0 says that the planes of the segments
 // past segs_short are all zero (the segments are left out); flags[1] != 0 that
 // B's plane 0 holds non-finite values, which may take part in the first
 // segment only (0 * inf): the others then read planes_alt, a copy without.
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   // is bound by its fragment reads, which it would hold up (FP8 2048 x [4096,
   // 4096] 52 -> 48 us, blocks of 16 8192 x [4096, 4096] 549 -> 523), else at
   // once, for the longest lead (bf16 [4096, 2048] . [2048, 8192]: 134, late 147)
-  constexpr bool LATE = SC == 1 || SC == 3;
+  constexpr bool LATE = SC == 1;
   constexpr int FB = SC == 3 ? 16 : 32, KBS = 64 / FB;   // block size, blocks of a step
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * STAGE];
 
@@ -378,6 +380,77 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
     }
   };
 
+  // Fine blocks: a step's units (a 32x32 output tile, half a step of K) run as a
+  // pipeline, unit u's MFMAs issued ahead of the multiply-adds that join unit
+  // u - 1's sums to the totals; the last unit's join carries over to the next
+  // step, under its fragment reads.  The next stage's DMA goes out without a
+  // branch, also in the last step (range-checked bytes that nobody reads).
+  v16f pc[SC == 3 ? 2 : 1];
+  float pu[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (FINE) {
+#pragma unroll
+    for (int h = 0; h < (SC == 3 ? 2 : 1); ++h) pc[h] = v16f{0};
+  }
+  auto fine_join = [&](int mi, int ni) {
+    if constexpr (SC == 3) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) tot[mi][ni][v] += pc[h][v] * pu[h * 2 + (v >> 3)];
+    } else if constexpr (SC == 4) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[mi][ni][v] += pc[0][v] * pu[0];
+    }
+  };
+  auto fine_step = [&](const uint8_t* st, const float (&um)[MI][4], const float* un) {
+    if constexpr (FINE) {
+      constexpr int UNITS = MI * NI;                       // per half step
+      constexpr int PER = (NA + 4 + UNITS - 1) / UNITS;    // DMA instructions beside each unit of the first half
+      v8i fa[2][MI], fb[2][NI];
+      auto reads = [&](int ks) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[ks][i] = frag(st, std::bool_constant<TNA>{}, wm * 2 + i, ks);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) fb[ks][i] = frag(st + A_BYTES, std::bool_constant<TNB>{}, wn * NI + i, ks);
+      };
+      reads(0);
+      __builtin_amdgcn_sched_barrier(0);
+      fine_join(MI - 1, NI - 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 2 * UNITS; ++u) {
+        const int ks = u / UNITS, mi = u % UNITS / NI, ni = u % NI;
+        const v8i a = fb[ks][ni], b = fa[ks][mi];
+        const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3});
+        const bf16x8_t b0 = __builtin_bit_cast(bf16x8_t, v4i{b.s0, b.s1, b.s2, b.s3});
+        const bf16x8_t a1 = __builtin_bit_cast(bf16x8_t, v4i{a.s4, a.s5, a.s6, a.s7});
+        const bf16x8_t b1 = __builtin_bit_cast(bf16x8_t, v4i{b.s4, b.s5, b.s6, b.s7});
+        v16f c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, v16f{0}, 0, 0, 0), d;
+        if constexpr (SC == 3) d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, v16f{0}, 0, 0, 0);
+        else c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, c, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (u == 0) reads(1);
+        if (ks == 0) {
+#pragma unroll
+          for (int i = u * PER; i < (u + 1) * PER && i < NA + 4; ++i) dma(i);
+        }
+        if (u > 0) fine_join((u - 1) % UNITS / NI, (u - 1) % NI);
+        pc[0] = c;
+        if constexpr (SC == 3) {
+          pc[1] = d;
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+              pu[h * 2 + q] = um[mi][ks * 2 + h] * un[(ks * 2 + h) * (WN / FB) + ni * 2 + q];
+        } else {
+          pu[0] = um[mi][0] * un[ks * (WN / FB) + ni];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
   if (k_begin < k_end) {
     load_stage(lds, true);
 #pragma unroll
@@ -416,6 +489,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
         }
       }
       const bool more = k + 1 < k_end;
+      if constexpr (FINE) {
+        load_stage(lds + ((k - k_begin + 1) & 1) * STAGE, false);
+        fine_step(st, um, un);
+        continue;
+      }
       if (more) {
         load_stage(lds + ((k - k_begin + 1) & 1) * STAGE, false);
         if (!LATE) {
@@ -435,29 +513,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
           for (int ni = 0; ni < NI; ++ni) {
-            if constexpr (FINE) {
-              const v8i a = fb[ni], b = fa[mi];
-              const bf16x8_t a0 = __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3});
-              const bf16x8_t b0 = __builtin_bit_cast(bf16x8_t, v4i{b.s0, b.s1, b.s2, b.s3});
-              const bf16x8_t a1 = __builtin_bit_cast(bf16x8_t, v4i{a.s4, a.s5, a.s6, a.s7});
-              const bf16x8_t b1 = __builtin_bit_cast(bf16x8_t, v4i{b.s4, b.s5, b.s6, b.s7});
-              v16f c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, v16f{0}, 0, 0, 0);
-              if constexpr (SC == 3) {
-                const v16f d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, v16f{0}, 0, 0, 0);
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                  const int kb = ks * 2 + h;
-                  const float u0 = um[mi][kb] * un[kb * (WN / FB) + ni * 2], u1 = um[mi][kb] * un[kb * (WN / FB) + ni * 2 + 1];
-#pragma unroll
-                  for (int v = 0; v < 16; ++v) tot[mi][ni][v] += (h ? d[v] : c[v]) * (v < 8 ? u0 : u1);
-                }
-              } else {
-                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, c, 0, 0, 0);
-                const float u = um[mi][0] * un[ks * (WN / FB) + ni];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) tot[mi][ni][v] += c[v] * u;
-              }
-            } else if constexpr (BF) {
+            if constexpr (BF) {
               const v8i a = fb[ni], b = fa[mi];
               acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                   __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3}),
@@ -482,6 +538,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
       }
     }
     flush();
+    if constexpr (FINE) {
+      fine_join(MI - 1, NI - 1);
+      PINNED_WAITCNT(0);                   // the last step's DMA
+    }
   }
 
   // Epilogue: 32 rows of the wave's columns at a time through the wave's part
