@@ -510,6 +510,18 @@ int pratchya_gemm_bs_t128(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, c
                           int64_t b_kg, int64_t M, int64_t N, int64_t K, void* C, int64_t ldc, int c_dtype, void* ws,
                           int64_t ws_bytes, hipStream_t stream);
 
+/* pratchya_gemm_bs_t128 to f32 followed by pratchya_quantize_dequantize with
+ * (1, 128) blocks in groups of 8 (M * N a multiple of 1024, N of 128), bit for
+ * bit, in two launches: the K slices are summed as the requantization reads
+ * them.  y [M, N] contiguous, 16-byte aligned; sc_fp8 [M * N / 128] and sc_fp32
+ * [M * N / 1024], or both null (not stored).  Workspace: the _fq query's. */
+int64_t pratchya_gemm_t128_fq_workspace_bytes(int64_t M, int64_t N, int64_t steps);
+int pratchya_gemm_bs_t128_fq(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, const float* a_sc32,
+                             int64_t a_rdiv, int64_t a_sr, int64_t a_sk, int64_t a_kg, const uint8_t* B, int64_t ldb,
+                             const uint8_t* b_sc8, const float* b_sc32, int64_t b_rdiv, int64_t b_sr, int64_t b_sk,
+                             int64_t b_kg, int64_t M, int64_t N, int64_t K, void* y, int y_dtype, int fix_nan,
+                             uint8_t* sc_fp8, float* sc_fp32, void* ws, int64_t ws_bytes, hipStream_t stream);
+
 /* Product of operands held as bf16 planes, f32 accumulation:
  *   C[m][n] = sum over segments s and k of A_s[m][k] * B_s[n][k]   (Q:618-622:
  * the f32 dots of matmul_impl's backward, each operand in as few exact planes

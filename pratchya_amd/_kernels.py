@@ -1179,15 +1179,48 @@ def mfma_ceiling(a: torch.Tensor, b: torch.Tensor, bf16: bool, iters: int) -> in
 
 
 def _few_then_requantize(a: Operand, b: Operand, out_dtype, tgrid, fix_nan, lead):
-    """gemm_nt_fq / gemm_nt_q11 of a product of few tiles, as its two steps."""
+    """gemm_nt_q11 of a product of few tiles, as its two steps."""
     lead = tuple(lead) if lead else (a.rows,)
     c = gemm_t128(a, b, torch.float32)
     y, s8, s32 = quantize_dequantize(c.view(lead + (b.rows,)), tgrid, out_dtype, fix_nan)
     return y.view(a.rows, b.rows), s8, s32
 
 
+def gemm_t128_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = False, lead=None,
+                 scales: bool = True):
+    """``gemm_t128(a, b, float32)`` and its requantization as gemm_nt_fq
+    returns them, in two launches: the slices of K are summed as the
+    requantization reads them.  N a multiple of 128 and every slice of ``lead``
+    whole groups of 8 blocks (``PratchyaUnsupported`` otherwise).  ``scales``
+    False: the scale arrays are not stored (None)."""
+    _require_gpu(a.payload, b.payload)
+    if a.k != b.k:
+        raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
+    M, N, Kd = a.rows, b.rows, a.k
+    lead = tuple(lead) if lead else (M,)
+    H = int(lead[-1])
+    if a.k_major or b.k_major or N % 128 or H * N % 1024 or M < 1:
+        raise PratchyaUnsupported("gemm_t128_fq: K-contiguous operands, outputs in whole groups of 8 blocks")
+    ap, bp = a.payload.contiguous(), b.payload.contiguous()
+    as8, bs8 = a.sc8.contiguous(), b.sc8.contiguous()
+    as32, bs32 = a.sc32.contiguous().float(), b.sc32.contiguous().float()
+    lib, dev = _lib.load(), ap.device
+    y = torch.empty((M, N), dtype=out_dtype, device=dev)
+    sc8 = sc32 = None
+    if scales:
+        sc8 = torch.empty(lead[:-1] + (H * N // 1024, 8), dtype=E8M0, device=dev)
+        sc32 = torch.empty(lead[:-1] + (H * N // 1024, 1, 1), dtype=torch.float32, device=dev)
+    ws_bytes = _ws_bytes("pratchya_gemm_t128_fq_workspace_bytes", M, N, Kd // 128)
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+    _lib.check(lib.pratchya_gemm_bs_t128_fq(
+        _ptr(ap), Kd, _ptr(as8), _ptr(as32), *a.desc, _ptr(bp), Kd, _ptr(bs8), _ptr(bs32), *b.desc, M, N, Kd, _ptr(y),
+        _dtype_code(out_dtype), 1 if fix_nan else 0, _ptr(sc8) if scales else None, _ptr(sc32) if scales else None,
+        _ptr(ws), ws_bytes, _stream(ap)), "gemm_t128_fq")
+    return y, sc8, sc32
+
+
 def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = False, lead=None,
-               status: torch.Tensor = None, few: bool = False):
+               status: torch.Tensor = None, few: bool = False, scales: bool = True):
     """``QArrayImpl(dequant(a) @ dequant(b)^T, (1, 128)).astype(out_dtype)``
     with the requantization in the GEMM's epilogue: returns ``(y [M, N],
     sc_fp8, sc_fp32)`` bit-identical to ``quantize_dequantize(gemm_nt(a, b,
@@ -1197,17 +1230,19 @@ def gemm_nt_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = F
     ``PratchyaUnsupported`` unless N is a multiple of 1024 and B's scale
     groups span at least 32 rows.  ``status``: an int32 device tensor that
     receives the strip exchange's status word (0: every wait completed).
-    ``few``: a product of few tiles may run as gemm_t128 and
-    quantize_dequantize, whose sums are in another order."""
+    ``few``: a product of few tiles may run as gemm_t128_fq, whose sums are in
+    another order; N then a multiple of 128, of 1024 where K is not split.
+    ``scales`` False: the caller keeps only y, the scales may be None."""
     _require_gpu(a.payload, b.payload)
     if a.k != b.k:
         raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
     if out_dtype not in (torch.float32, torch.bfloat16):
         raise ValueError(f"gemm_nt_fq: output dtype {out_dtype} is not float32 or bfloat16")
     M, N, K = a.rows, b.rows, a.k
-    if few and status is None and N % 1024 == 0 and b.desc[0] % 32 == 0 and not a.k_major \
-            and prefers_t128(M, a.desc[3], b):
-        return _few_then_requantize(a, b, out_dtype, (1, 128), fix_nan, lead)
+    # (N not of whole groups of a row: worth it where there are slices to sum)
+    if few and status is None and b.desc[0] % 32 == 0 and not a.k_major and prefers_t128(M, a.desc[3], b) \
+            and (N % 1024 == 0 or _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, K // 128, 1)):
+        return gemm_t128_fq(a, b, out_dtype, fix_nan, lead, scales)
     lib = _lib.load()
     ws_bytes = _ws_bytes("pratchya_gemm_bs_nt_fq_workspace_bytes", M, N)
     if ws_bytes <= 0:

@@ -111,6 +111,11 @@ SIGNATURES = {
     "pratchya_gemm_bs_t128": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
                                        _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
                                        _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p]),
+    "pratchya_gemm_t128_fq_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "pratchya_gemm_bs_t128_fq": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
+                                          _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
+                                          _c_i64, _c_i64, _c_i64, _c_p, _c_int, _c_int, _c_p, _c_p, _c_p, _c_i64,
+                                          _c_p]),
     "pratchya_gemm_bf16_planes": (_c_int, [_c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32,
                                            _c_p, _c_i64, _c_i64, _c_int, _c_int, ctypes.c_uint32, ctypes.c_uint32,
                                            _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_p, _c_p, _c_i64, _c_i64,

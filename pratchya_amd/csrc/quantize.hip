@@ -254,13 +254,18 @@ __global__ __launch_bounds__(256) void k_quant_rowgroup(
 // _qarr.py:575-601), in registers.
 // --------------------------------------------------------------------------
 
-template <bool IS_BF16, bool HW, int OUT, bool FIXNAN, bool PRE>
+// SUM: x is the sum of `parts` f32 arrays of n_groups * 1024 values one after
+// the other (a product's K slices, in slice order: the bits of their sum),
+// sc8 / sc32 may be null (not stored).  Up to 8 slices' loads are in flight at
+// once: small products have few groups, and their time is these loads' latency.
+template <bool IS_BF16, bool HW, int OUT, bool FIXNAN, bool PRE, bool SUM = false>
 __global__ __launch_bounds__(256) void k_quant_g8(const void* __restrict__ xv,
                                                   void* __restrict__ outv,
                                                   uint8_t* __restrict__ sc8,
                                                   float* __restrict__ sc32, int64_t n_groups,
                                                   const uint8_t* __restrict__ psc8,
-                                                  const float* __restrict__ psc32) {
+                                                  const float* __restrict__ psc32, int parts = 1) {
+  static_assert(!SUM || (!IS_BF16 && !PRE), "sums of f32 slices");
   constexpr int VEC = IS_BF16 ? 8 : 4;        // elements per 16-byte load
   constexpr int R = IS_BF16 ? 2 : 4;          // 64-lane rows per 1024-element group
   constexpr int BL = 128 / VEC;               // lanes per block
@@ -279,8 +284,8 @@ __global__ __launch_bounds__(256) void k_quant_g8(const void* __restrict__ xv,
   if (g >= n_groups) return;
   const char* xb = static_cast<const char*>(xv);
   // scale arrays as raw buffers (byte counts below 2^32 - 16, checked on the host)
-  const __amdgpu_buffer_rsrc_t r8 = __builtin_amdgcn_make_buffer_rsrc(sc8, 0, (int)(uint32_t)(n_groups * 8), kRawBuffer);
-  const __amdgpu_buffer_rsrc_t r32 = __builtin_amdgcn_make_buffer_rsrc(sc32, 0, (int)(uint32_t)(n_groups * 4), kRawBuffer);
+  const __amdgpu_buffer_rsrc_t r8 = __builtin_amdgcn_make_buffer_rsrc(sc8, 0, SUM && !sc8 ? 0 : (int)(uint32_t)(n_groups * 8), kRawBuffer);
+  const __amdgpu_buffer_rsrc_t r32 = __builtin_amdgcn_make_buffer_rsrc(sc32, 0, SUM && !sc32 ? 0 : (int)(uint32_t)(n_groups * 4), kRawBuffer);
 
   uint4 nxt[R];
 #pragma unroll
@@ -290,6 +295,18 @@ __global__ __launch_bounds__(256) void k_quant_g8(const void* __restrict__ xv,
     uint4 v[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = nxt[r];
+    if constexpr (SUM) {
+      const int64_t stride = n_groups * GROUP_BYTES;
+      const char* src = xb + g * GROUP_BYTES + lane * 16;
+#pragma unroll 8
+      for (int p = 1; p < parts; ++p)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint4 w = load_stream16(src + p * stride + r * 1024);
+          v[r] = make_uint4(f2u(u2f(v[r].x) + u2f(w.x)), f2u(u2f(v[r].y) + u2f(w.y)), f2u(u2f(v[r].z) + u2f(w.z)),
+                            f2u(u2f(v[r].w) + u2f(w.w)));
+        }
+    }
     if (g + wstride < n_groups) {
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -1329,6 +1346,27 @@ int launch_g8_qdq(const void* x, void* out, bool out_bf16, bool fix_nan, uint8_t
 }
 
 }  // namespace
+
+// quantize_dequantize with (1, 128) blocks in groups of 8 of the sum of `parts`
+// f32 arrays of n_groups * 1024 values, for gemm_t128.hip (which checks the
+// arguments); null scale arrays are not stored.
+int pratchya_quantize_dequantize_sum(const float* part, int parts, int64_t n_groups, void* out, bool out_bf16,
+                                     bool fix_nan, uint8_t* sc_fp8, float* sc_fp32, hipStream_t st) {
+  const dim3 grid((unsigned)n_groups), block(64);
+  const void* x = part;
+#define PRATCHYA_SUM(OUT, FIX)                                                                                   \
+  hipLaunchKernelGGL((k_quant_g8<false, PRATCHYA_HW_CVT != 0, OUT, FIX, false, true>), grid, block, 0, st, x,    \
+                     out, sc_fp8, sc_fp32, n_groups, nullptr, nullptr, parts)
+  if (out_bf16) {
+    if (fix_nan) PRATCHYA_SUM(1, true);
+    else PRATCHYA_SUM(1, false);
+  } else {
+    if (fix_nan) PRATCHYA_SUM(2, true);
+    else PRATCHYA_SUM(2, false);
+  }
+#undef PRATCHYA_SUM
+  return check_launch("quantize_dequantize_sum");
+}
 
 extern "C" int pratchya_quant_layout(int64_t H, int64_t W, int64_t a, int64_t b, int64_t* n_blk,
                                      int64_t* K, int64_t* M) {

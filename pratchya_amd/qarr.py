@@ -543,16 +543,17 @@ def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype, scale
     requantization in the GEMM's epilogue: ``(y, sc_fp8, sc_fp32)`` bit-identical
     to the f32 product followed by ``quantize_dequantize``, or None when the
     layouts do not fit.  ``go`` (1, 128), a quantized Linear's output, takes
-    N a multiple of 1024 (its groups span four output tiles); (1, 1), the
+    N a multiple of 1024 (its groups span four output tiles; of 128 where few
+    tiles make it K.gemm_t128_fq); (1, 1), the
     output of a weight quantized (a, 1) (lm_head, LoRA), N a multiple of 16.
-    (Products of few tiles run as the two steps: ``K.prefers_t128``.)
+    (A (1, 1) product of few tiles runs as the two steps: ``K.prefers_t128``.)
     ``scales`` False: the caller keeps only y; the (1, 1) scales, larger than
-    y itself, are then not stored."""
+    y itself, and those of a product of few tiles are then not stored."""
     go = tuple(go)
     if go not in ((1, 128), (1, 1)) or dtype not in (torch.float32, torch.bfloat16) or y8.dim() != 2:
         return None
     N = int(y8.shape[1])
-    if N % (1024 if go == (1, 128) else 16):
+    if N % (128 if go == (1, 128) else 16):
         return None
     op_a = _lhs_operand(x8, xs8, xs32, gx)
     op_b = _rhs_operand(y8, ys8, ys32, gy) if op_a is not None else None
@@ -563,7 +564,7 @@ def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype, scale
         if go == (1, 1):
             res, s8, s32 = K.gemm_nt_q11(op_a, op_b, dtype, lead=lead, few=True, scales=scales)
         else:
-            res, s8, s32 = K.gemm_nt_fq(op_a, op_b, dtype, lead=lead, few=True)
+            res, s8, s32 = K.gemm_nt_fq(op_a, op_b, dtype, lead=lead, few=True, scales=scales)
     except K.PratchyaUnsupported:
         return None
     return res.reshape(lead + (N,)), s8, s32

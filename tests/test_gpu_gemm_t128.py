@@ -270,3 +270,37 @@ def test_batched_slices():
     assert _rel(runs[0].float(), one[0].double()) <= 3e-2
     for p, q in zip(one[1], runs[1]):
         assert p.dtype == q.dtype and torch.equal(p.view(torch.uint8), q.view(torch.uint8))
+
+
+@pytest.mark.parametrize("lead,Kd,N", [((1,), 128, 1024), ((4,), 4096, 4096), ((8,), 128, 128), ((33,), 256, 1024),
+                                       ((1000,), 2176, 2944), ((2, 8), 512, 384), ((640,), 4096, 1152)])
+@pytest.mark.parametrize("dt,fix_nan", [(torch.bfloat16, False), (torch.float32, True)])
+def test_requantized_sum_of_slices(lead, Kd, N, dt, fix_nan):
+    """The requantization that sums the K slices itself: the bits of the
+    reduced product's, scales stored or not."""
+    K = _K()
+    rows = 1
+    for d in lead:
+        rows *= d
+    x = _randn((rows, Kd), 30, torch.bfloat16, 3.0)
+    x[0, :128] = 0                                   # a block of zeros
+    if rows > 4:
+        x[3] = 0
+        x[4, 5] = float("nan") if fix_nan else float("inf")
+    a = K.operand_rows(*K.quantize(x, (1, 128)), (1, 128))
+    b = K.operand_transposed(*K.quantize(_randn((Kd, N), 31, torch.bfloat16, 0.02), (128, 128)), (128, 128))
+    ref = K.quantize_dequantize(K.gemm_t128(a, b, torch.float32).view(lead + (N,)), (1, 128), dt, fix_nan)
+    got = K.gemm_t128_fq(a, b, dt, fix_nan, lead)
+    bare = K.gemm_t128_fq(a, b, dt, fix_nan, lead, scales=False)
+    assert got[0].shape == (rows, N) and [t.shape for t in got[1:]] == [t.shape for t in ref[1:]]
+    for r, t in zip(ref, got):
+        assert torch.equal(r.reshape(-1).view(torch.uint8), t.reshape(-1).view(torch.uint8))
+    assert torch.equal(bare[0].view(torch.uint8), got[0].view(torch.uint8)) and bare[1:] == (None, None)
+
+
+def test_requantized_sum_refusals():
+    K = _K()
+    a = K.operand_rows(*K.quantize(_randn((5, 256), 1, torch.bfloat16), (1, 128)), (1, 128))
+    b = K.operand_transposed(*K.quantize(_randn((256, 384), 2, torch.bfloat16), (128, 128)), (128, 128))
+    with pytest.raises(K.PratchyaUnsupported):
+        K.gemm_t128_fq(a, b, torch.bfloat16)         # 15 blocks: not whole groups of 8
