@@ -168,11 +168,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   constexpr int A_BYTES = TM * KB, STAGE = A_BYTES + TN * KB;
   constexpr int NA = TM / 32;                            // A DMA instructions per wave and stage
   constexpr bool FINE = SC >= 3;
-  // The next stage's DMA goes out between the first half's MFMAs where the step
-  // is bound by its fragment reads, which it would hold up (FP8 2048 x [4096,
-  // 4096] 52 -> 48 us, blocks of 16 8192 x [4096, 4096] 549 -> 523), else at
-  // once, for the longest lead (bf16 [4096, 2048] . [2048, 8192]: 134, late 147)
-  constexpr bool LATE = SC == 1;
   constexpr int FB = SC == 3 ? 16 : 32, KBS = 64 / FB;   // block size, blocks of a step
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * STAGE];
 
@@ -453,6 +448,86 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
     }
   };
 
+  // bf16.  Row-contiguous operands: the next stage's DMA goes out first, for the
+  // longest lead ([4096, 2048] . [2048, 8192] 130 us, behind the reads 138).  A
+  // K-major operand takes four times the reads: the second half's go out under
+  // the first half's MFMAs and the DMA behind the step's last read, since a read
+  // after it would wait for the DMA, which the compiler takes to write what it
+  // reads ([2048, 8192] . [8192, 8192], both K-major: 289 -> 264 us).
+  auto bf16_step = [&](const uint8_t* st, bool more, uint8_t* next) {
+    if constexpr (BF && !FINE) {
+      constexpr int UNITS = MI * NI;
+      constexpr bool EARLY = !TNA && !TNB;
+      v8i fa[2][MI], fb[2][NI];
+      auto reads = [&](int ks) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[ks][i] = frag(st, std::bool_constant<TNA>{}, wm * 2 + i, ks);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) fb[ks][i] = frag(st + A_BYTES, std::bool_constant<TNB>{}, wn * NI + i, ks);
+      };
+      auto stage_dma = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+#pragma unroll
+          for (int i = 0; i < NA + 4; ++i) dma(i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      if (more) load_stage(next, false);
+      if (EARLY) stage_dma();
+      reads(0);
+      if (!EARLY) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 2 * UNITS; ++u) {
+        const int ks = u / UNITS, mi = u % UNITS / NI, ni = u % NI;
+        if (EARLY && u == UNITS) reads(1);
+        const v8i a = fb[ks][ni], b = fa[ks][mi];
+        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3}),
+            __builtin_bit_cast(bf16x8_t, v4i{b.s0, b.s1, b.s2, b.s3}), acc[mi][ni], 0, 0, 0);
+        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            __builtin_bit_cast(bf16x8_t, v4i{a.s4, a.s5, a.s6, a.s7}),
+            __builtin_bit_cast(bf16x8_t, v4i{b.s4, b.s5, b.s6, b.s7}), acc[mi][ni], 0, 0, 0);
+        if (!EARLY && u == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          reads(1);
+          stage_dma();
+        }
+      }
+    }
+  };
+
+  // FP8: as with a K-major operand (1000 x [2176, 2944] 24.8 -> 24.0 us); the DMA
+  // of the last step goes out too (range-checked bytes that nobody reads).
+  auto fp8_step = [&](const uint8_t* st, const uint32_t* ea, const uint32_t* eb) {
+    if constexpr (!BF) {
+      constexpr int UNITS = MI * NI;
+      v8i fa[2][MI], fb[2][NI];
+      auto reads = [&](int ks) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[ks][i] = frag(st, std::bool_constant<TNA>{}, wm * 2 + i, ks);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) fb[ks][i] = frag(st + A_BYTES, std::bool_constant<TNB>{}, wn * NI + i, ks);
+      };
+      reads(0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 2 * UNITS; ++u) {
+        const int ks = u / UNITS, mi = u % UNITS / NI, ni = u % NI;
+        acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[ks][ni], fa[ks][mi], acc[mi][ni], 0, 0, 0,
+                                                                     (int)eb[ni], 0, (int)ea[mi]);
+        if (u == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          reads(1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < NA + 4; ++i) dma(i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+
   if (k_begin < k_end) {
     load_stage(lds, true);
 #pragma unroll
@@ -490,60 +565,18 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
             for (int j = 0; j < 4; ++j) ub[i][j] = SC == 1 ? gb_n[i][j] * 0.0078125f : mantissa_unit(gb_n[i][j]);
         }
       }
-      const bool more = k + 1 < k_end;
-      if constexpr (FINE) {
-        load_stage(lds + ((k - k_begin + 1) & 1) * STAGE, false);
-        fine_step(st, um, un);
-        continue;
-      }
-      if (more) {
-        load_stage(lds + ((k - k_begin + 1) & 1) * STAGE, false);
-        if (!LATE) {
-#pragma unroll
-          for (int i = 0; i < NA + 4; ++i) dma(i);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        v8i fa[MI], fb[NI];
-#pragma unroll
-        for (int i = 0; i < MI; ++i) fa[i] = frag(st, std::bool_constant<TNA>{}, wm * 2 + i, ks);
-#pragma unroll
-        for (int i = 0; i < NI; ++i) fb[i] = frag(st + A_BYTES, std::bool_constant<TNB>{}, wn * NI + i, ks);
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int ni = 0; ni < NI; ++ni) {
-            if constexpr (BF) {
-              const v8i a = fb[ni], b = fa[mi];
-              acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  __builtin_bit_cast(bf16x8_t, v4i{a.s0, a.s1, a.s2, a.s3}),
-                  __builtin_bit_cast(bf16x8_t, v4i{b.s0, b.s1, b.s2, b.s3}), acc[mi][ni], 0, 0, 0);
-              acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  __builtin_bit_cast(bf16x8_t, v4i{a.s4, a.s5, a.s6, a.s7}),
-                  __builtin_bit_cast(bf16x8_t, v4i{b.s4, b.s5, b.s6, b.s7}), acc[mi][ni], 0, 0, 0);
-            } else {
-              acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[ni], fa[mi], acc[mi][ni], 0, 0, 0,
-                                                                           (int)eb[ni], 0, (int)ea[mi]);
-            }
-            if (LATE && ks == 0) {
-              constexpr int PER = (NA + 4 + MI * NI - 1) / (MI * NI);
-              __builtin_amdgcn_sched_barrier(0);
-              if (more) {
-#pragma unroll
-                for (int i = (mi * NI + ni) * PER; i < (mi * NI + ni + 1) * PER && i < NA + 4; ++i) dma(i);
-              }
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          }
+      uint8_t* next = lds + ((k - k_begin + 1) & 1) * STAGE;
+      if constexpr (BF && !FINE) {
+        bf16_step(st, k + 1 < k_end, next);
+      } else {
+        load_stage(next, false);
+        if constexpr (FINE) fine_step(st, um, un);
+        else fp8_step(st, ea, eb);
       }
     }
     flush();
-    if constexpr (FINE) {
-      fine_join(MI - 1, NI - 1);
-      PINNED_WAITCNT(0);                   // the last step's DMA
-    }
+    if constexpr (FINE) fine_join(MI - 1, NI - 1);
+    if constexpr (FINE || !BF) PINNED_WAITCNT(0);          // the last step's DMA
   }
 
   // Epilogue: 32 rows of the wave's columns at a time through the wave's part
