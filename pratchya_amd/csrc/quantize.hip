@@ -657,6 +657,77 @@ __global__ __launch_bounds__(256) void k_cast_general(const void* __restrict__ x
   }
 }
 
+// Blocks of 16 x 16 in groups of 16 and of 32 x 32 in groups of 64 (the block
+// size 16 and 32 presets' weights and their gradients): a workgroup owns a group
+// and holds it in registers, one pass and one launch where the flat kernels take
+// four (fill, block maxima with atomics, group scales, cast).  [2048, 2048] in
+// blocks of 16: bf16 to payloads 24 -> 5.2 us, f32 to bf16 22 -> 6.2 us; in
+// blocks of 32, back to back from a graph, 12.6 -> 6.8 and 15.2 -> 12.1 us,
+// [4096, 4096] 21.0 -> 9.1 and 31.5 -> 21.8 us.  (Of 4 groups, where few CUs have
+// work, the time is one group's chain: [512, 512] f32 9.8 -> 11.2 us from a
+// graph, less than the three launches saved cost an eager caller.)  A thread holds 16 consecutive values of one row in every RG-th row of a block;
+// consecutive threads hold consecutive pieces of a row of the group's blocks.
+template <bool IS_BF16, int OUT, int B>
+__global__ __launch_bounds__(B == 16 ? 256 : 1024) void k_group_square(const void* __restrict__ x,
+                                                                       void* __restrict__ outv,
+                                                                       uint8_t* __restrict__ sc8,
+                                                                       float* __restrict__ sc32, int64_t W,
+                                                                       int fix_nan) {
+  constexpr int CH = 16, OSZ = OUT == 0 ? 1 : (OUT == 1 ? 2 : 4);
+  constexpr int K = B == 16 ? 16 : 64, P = B / CH;              // blocks of a group, pieces of a block's row
+  constexpr int RG = (B == 16 ? 256 : 1024) / (K * P), R = B / RG;
+  constexpr int NW = K * P < 64 ? RG * K * P / 64 : RG;         // maxima of a block that meet in the LDS
+  __shared__ uint32_t lds[NW][K];
+  const int c = threadIdx.x % (K * P), j = c / P, r = threadIdx.x / (K * P);
+  const int64_t blk = (int64_t)blockIdx.x * K + j, bpr = W / B, bi = blk / bpr;
+  const int64_t off = (bi * B + r) * W + (blk - bi * bpr) * B + c % P * CH;
+  float v[R][CH];
+#pragma unroll
+  for (int i = 0; i < R; ++i) load_chunk<IS_BF16, CH, true>(x, off + (int64_t)i * RG * W, v[i]);
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int k = 0; k < CH; ++k) m = umax(m, abs_bits(v[i][k]));
+  if constexpr (B == 16) {
+    m = xor_max_u32<32>(xor_max_u32<16>(m));                    // a wave holds four rows of every block
+    if ((threadIdx.x & 63) < 16) lds[threadIdx.x >> 6][j] = m;
+  } else {
+    m = lane_group_max<P>(m);
+    if (c % P == 0) lds[r][j] = m;
+  }
+  __syncthreads();
+  m = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) m = umax(m, lds[i][j]);
+  uint32_t g = m;
+  if constexpr (B != 16) {
+    // a wave's 64 lanes hold half of the group's blocks
+    const int l = threadIdx.x & 63;
+    g = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) g = umax(g, lds[i][l]);
+  }
+  const float G = u2f(lane_group_max<K>(g));
+  const uint32_t e = e8m0_of(u2f(m), G);
+  if (r == 0 && c % P == 0) sc8[blk] = (uint8_t)e;
+  if (threadIdx.x == 0) sc32[blockIdx.x] = G;
+  const float sG = e8m0_decode(e) * G;
+  const float S = quant_scale(e, G);
+  const bool ok = sG >= kClamp && sG <= 3.0e38f;
+  const float yv = 128.0f / S;
+  const float dq = e8m0_decode((fix_nan && e == 0xFFu) ? 0x7Fu : e) * G;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    uint32_t w[CH * OSZ / 4];
+    cast_words<CH, OUT>(v[i], yv, S, ok, dq, w);
+#pragma unroll
+    for (int q = 0; q < CH * OSZ / 16; ++q)
+      store_stream16(static_cast<char*>(outv) + (off + (int64_t)i * RG * W) * OSZ + 16 * q,
+                     u32x4_t{w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]});
+  }
+}
+
 // Workgroup per block (tile_fits).  The threads lie on the block's row
 // segments, RT = 256 >> seg_log2 rows at a time, four steps' loads in flight.
 // [2048, 8192] in blocks of 128, flat kernels before: bf16 to payloads 25.7 ->
@@ -1227,6 +1298,16 @@ int launch_general(const void* x, void* q, uint8_t* sc8, float* sc32, uint32_t* 
     hipLaunchKernelGGL((k_tile_cast<IS_BF16, OUT>), grid, dim3(256), 0, st, x, q, ws, sc8, sc32, L.W, (int)L.a,
                        (int)L.b, L.K, ilog2(L.b / COUT), fix_nan);
     return check_launch("quantize(block)");
+  }
+  if (!premax && L.a == L.b && ((L.a == 16 && L.K == 16) || (L.a == 32 && L.K == 64)) && n_groups <= 0x7FFFFFFF &&
+      aligned(x, 16) && aligned(q, 16)) {
+    if (L.a == 16)
+      hipLaunchKernelGGL((k_group_square<IS_BF16, OUT, 16>), dim3((unsigned)n_groups), dim3(256), 0, st, x, q, sc8,
+                         sc32, L.W, fix_nan);
+    else
+      hipLaunchKernelGGL((k_group_square<IS_BF16, OUT, 32>), dim3((unsigned)n_groups), dim3(1024), 0, st, x, q, sc8,
+                         sc32, L.W, fix_nan);
+    return check_launch("quantize(square blocks)");
   }
   if (!premax)
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n_blocks_total, 256) > 4096 ? 4096 : grid_for(n_blocks_total, 256)),

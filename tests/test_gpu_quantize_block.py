@@ -1,5 +1,5 @@
 """Quantization with a workgroup per block (grids whose block is 4096 to 65536
-elements in rows of 64 or more) against the oracle and, bit for bit, against
+elements in rows of 64 or more) or per group (blocks of 16 x 16 and 32 x 32) against the oracle and, bit for bit, against
 the flat kernels, which take the same values from an unaligned buffer."""
 import numpy as np
 import pytest
@@ -14,7 +14,13 @@ pytestmark = pytest.mark.gpu
 # the widest and smallest blocks, one group over the array, one block per group
 CASES = [((3, 256, 384), (128, 128)), ((200, 192), (100, 64)), ((64, 64), (64, 64)), ((130, 1024), (65, 128)),
          ((256, 512), (128, 512)), ((48, 1024), (16, 256)), ((1024, 64), (1024, 64)), ((1024, 1024), (128, 128)),
-         ((96, 128), (32, 128)), ((255, 256), (255, 256))]
+         ((96, 128), (32, 128)), ((255, 256), (255, 256)),
+         # groups of 16 blocks of 16 x 16: in one row of blocks, across two, several rows, several slices
+         ((16, 256), (16, 16)), ((32, 384), (16, 16)), ((256, 48), (16, 16)), ((256, 16), (16, 16)),
+         ((3, 64, 320), (16, 16)), ((208, 256), (16, 16)), ((16, 240), (16, 16)),
+         # groups of 64 blocks of 32 x 32, and fewer blocks in a group
+         ((32, 2048), (32, 32)), ((256, 256), (32, 32)), ((2, 64, 3072), (32, 32)), ((2048, 32), (32, 32)),
+         ((320, 640), (32, 32))]
 
 
 def _values(shape, dtype, seed):
