@@ -787,7 +787,7 @@ def prefers_t128(M: int, a_kg: int, b: Operand) -> bool:
     1024] (64 tiles) 31 / 32; 2048 x [4096, 4096] (128 tiles) 60 / 63."""
     N, Kd = b.rows, b.k
     tiles = -(-M // GEMM_TILE_ROWS) * -(-N // GEMM_TILE_ROWS)
-    if not (M <= 32 or (tiles <= 64 and Kd >= 32 * tiles)) or b.k_major or N % 8:
+    if 0 in (M, N, Kd) or not (M <= 32 or (tiles <= 64 and Kd >= 32 * tiles)) or b.k_major or N % 8:
         return False
     brd, bsr, bsk, bkg = b.desc
     rows4 = brd % 4 == 0 or (brd == 1 and bsr > 0 and bkg % (4 * bsr) == 0 and bsk % (4 * bsr) == 0)
@@ -904,9 +904,13 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
     n_rows = N if N >= GEMM_TILE_ROWS else (N + 3) // 4 * 4
     A = _split_pack(a, a_t, a_planes, kp)
     B = _split_pack(b, not b_t, b_planes, kp, n_rows)
+    c = None
     if few_tiles(M, n_rows):
-        c = gemm_planes(A[None], B[None], [(0, 0)], False)
-    else:
+        try:
+            c = gemm_planes(A[None], B[None], [(0, 0)], False)
+        except PratchyaUnsupported:      # few rows of more than 2^24 columns
+            pass
+    if c is None:
         c = gemm_bf16_nt(A, B, torch.float32)
     return c if n_rows == N else c[:, :N]
 
@@ -1000,6 +1004,8 @@ def gemm_fine(a: torch.Tensor, a_sc32: torch.Tensor, b: torch.Tensor, b_sc32: to
     ag, bg = a_sc32.contiguous().float(), b_sc32.contiguous().float()
     if ag.numel() != M * Kd // (16 if blk == 16 else 64):
         raise PratchyaUnsupported("gemm_fine: x's groups are not one block of 16 or two of 32")
+    if not _aligned(ag, 16):      # a view into a larger array: four maxima are one load
+        ag = ag.clone()
     c = torch.empty((M, N), dtype=torch.float32, device=a.device)
     ws_bytes = _ws_bytes("pratchya_gemm_t128_workspace_bytes", M, N, Kd // 64, 1)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None

@@ -454,8 +454,8 @@ def _plane_backward(g, scales, saved, grids, need_x, need_y):
     if y8.dim() != 2 or x8.dim() < 2 or g.dtype not in (torch.float32, torch.bfloat16) or int(gx[0]) != 1:
         return None, None
     Kd, N = int(y8.shape[0]), int(y8.shape[1])
-    rows = g.numel() // N
-    if rows == 0 or g.numel() != rows * N or x8.numel() != rows * Kd:
+    rows = math.prod(x8.shape[:-1])
+    if 0 in (rows, Kd, N) or g.numel() != rows * N or x8.numel() != rows * Kd:
         return None, None
     gs8 = gs32 = go = None
     if scales is not None:
@@ -1209,7 +1209,7 @@ class _LazyProduct(QArrayImpl):
         x = xo._pending
         op_b = _rhs_operand(y8, ys8, ys32, gy)
         # (a product of few tiles runs as it does without the prologue)
-        if op_b is None or K.prefers_t128(x.numel() // int(x.shape[-1]), 8, op_b):
+        if op_b is None or K.prefers_t128(math.prod(x.shape[:-1]), 8, op_b):
             return None
         with torch.set_grad_enabled(self._grad_enabled):
             sx = x if (x.requires_grad and torch.is_grad_enabled()) else None

@@ -304,3 +304,24 @@ def test_requantized_sum_refusals():
     b = K.operand_transposed(*K.quantize(_randn((256, 384), 2, torch.bfloat16), (128, 128)), (128, 128))
     with pytest.raises(K.PratchyaUnsupported):
         K.gemm_t128_fq(a, b, torch.bfloat16)         # 15 blocks: not whole groups of 8
+
+
+def _shifted(t, n):
+    """A copy of ``t`` that starts n elements into its buffer."""
+    buf = torch.empty(t.numel() + n, dtype=t.dtype, device=t.device)
+    return buf[n:].copy_(t.reshape(-1)).view(t.shape)
+
+
+def test_scales_inside_larger_arrays():
+    """Scale arrays that start at no multiple of 16 (of 4) bytes."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    xq, wq = K.quantize(_randn((100, 512), 1), (1, 16)), K.quantize(_randn((512, 256), 2), (16, 16))
+    c = Q._fine_forward(*xq, *wq, (1, 16), (16, 16))
+    at = xq[0], _shifted(xq[1].view(torch.uint8), 1).view(xq[1].dtype), _shifted(xq[2], 1)
+    assert at[2].data_ptr() % 16 and torch.equal(Q._fine_forward(*at, *wq, (1, 16), (16, 16)), c)
+    xq, wq = K.quantize(_randn((100, 512), 3), (1, 128)), K.quantize(_randn((512, 256), 4), (128, 128))
+    w = K.operand_transposed(*wq, (128, 128))
+    c = K.gemm_t128(K.operand_rows(*xq, (1, 128)), w)
+    at = xq[0], _shifted(xq[1].view(torch.uint8), 1).view(xq[1].dtype), _shifted(xq[2], 1)
+    assert at[1].data_ptr() % 4 and torch.equal(K.gemm_t128(K.operand_rows(*at, (1, 128)), w), c)
