@@ -117,7 +117,7 @@ __device__ __forceinline__ v8i read_frag_tn(const uint8_t* base) {
 }
 
 // The mantissa of a group maximum, in [1, 2) ([0, 1) for a subnormal one): the
-// expanded bf16 plane holds the power of two (pratchya_expand_pow2).  0 and
+// bf16 plane holds the power of two (pratchya_planes, POW2).  0 and
 // non-finite maxima count as 1 (their blocks' planes are 0, or already not
 // finite).
 __device__ __forceinline__ float mantissa_unit(float g) {
