@@ -275,17 +275,29 @@ __global__ __launch_bounds__(256) void k_sumsq_b16(const uint16_t* __restrict__ 
   if (threadIdx.x == 0) part[blockIdx.x] = (ws[0] + ws[1]) + (ws[2] + ws[3]);
 }
 
+// Bound by HBM at large sizes; below, by the chain ahead of a workgroup's first
+// store: the partials' sum, a square root, a barrier, 16 quotients per chunk.  So
+// the first chunk is loaded before the chain, and a launch has one round of
+// workgroups (kScaleBlocks, 8 per CU), not a second chain behind the first: two
+// arrays of [1024, 4096] 17.0 -> 12.3 us.  (The f32 kernel, whose chunks hold
+// half as many quotients, measured 7.7 -> 8.3 us so and stays as it is.)
 // (x and y may be the same array: each element is read and written by one
 // thread)
+constexpr int kScaleBlocks = 2048;
+
 __global__ __launch_bounds__(256) void k_ns_scale_b16(const uint16_t* x, int64_t n, const float* __restrict__ part,
                                                       uint16_t* y) {
   x += (int64_t)blockIdx.y * n;
   y += (int64_t)blockIdx.y * n;
   part += (int64_t)blockIdx.y * kNormBlocks;
+  const int64_t n8 = n / 8, stride = (int64_t)gridDim.x * 256;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  uint4 v = make_uint4(0, 0, 0, 0);
+  if (i < n8) v = *reinterpret_cast<const uint4*>(x + i * 8);
   __shared__ float sden;
   if (threadIdx.x < 64) {
     float s = 0.0f;
-    for (int i = (int)threadIdx.x; i < kNormBlocks; i += 64) s += part[i];
+    for (int k = (int)threadIdx.x; k < kNormBlocks; k += 64) s += part[k];
     s = wave_sum(s);
     if (threadIdx.x == 0) {
       const float total = bf16_rne(s);                 // the sum is a bf16 value
@@ -295,18 +307,17 @@ __global__ __launch_bounds__(256) void k_ns_scale_b16(const uint16_t* x, int64_t
   }
   __syncthreads();
   const float den = sden;
-  const int64_t n8 = n / 8;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (int64_t)gridDim.x * 256) {
-    const uint4 v = *reinterpret_cast<const uint4*>(x + i * 8);
+  for (; i < n8; i += stride) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    if (i + stride < n8) v = *reinterpret_cast<const uint4*>(x + (i + stride) * 8);
     uint32_t o[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) o[k] = pack_bf16x2(bf16_lo(w[k]) / den, bf16_hi(w[k]) / den);
     *reinterpret_cast<uint4*>(y + i * 8) = make_uint4(o[0], o[1], o[2], o[3]);
   }
   if (blockIdx.x == 0)
-    for (int64_t i = n8 * 8 + threadIdx.x; i < n; i += 256)
-      y[i] = (uint16_t)(pack_bf16x2(bf16_lo(x[i]) / den, 0.0f) & 0xFFFFu);
+    for (int64_t j = n8 * 8 + threadIdx.x; j < n; j += 256)
+      y[j] = (uint16_t)(pack_bf16x2(bf16_lo(x[j]) / den, 0.0f) & 0xFFFFu);
 }
 
 // The f32 normalization (pratchya/_nnx_impl/_optimizer.py:17 on an f32
@@ -523,7 +534,8 @@ extern "C" int pratchya_ns_normalize_batch(const void* g, void* x, int64_t n, in
   int rc = check_launch("ns_normalize");
   if (rc) return rc;
   const int64_t chunks = n / 8;
-  const int64_t blocks = chunks / 256 + 1 < 4096 ? chunks / 256 + 1 : 4096;
+  const int64_t most = batch < kScaleBlocks ? kScaleBlocks / batch : 1;
+  const int64_t blocks = chunks / 256 + 1 < most ? chunks / 256 + 1 : most;
   hipLaunchKernelGGL(k_ns_scale_b16, dim3((unsigned)blocks, (unsigned)batch), dim3(256), 0, stream, static_cast<const uint16_t*>(g),
                      n, part, static_cast<uint16_t*>(x));
   return check_launch("ns_normalize");
