@@ -1038,6 +1038,8 @@ def ns_normalize(g: torch.Tensor) -> torch.Tensor:
     if g.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError("ns_normalize: g must be bfloat16 or float32")
     gc = g.contiguous()
+    if not _aligned(gc, 16):      # a slice of a larger array
+        gc = gc.clone()
     out = torch.empty_like(gc)
     lib = _lib.load()
     ws = torch.empty(_ws_bytes("pratchya_ns_normalize_workspace_bytes"), dtype=torch.uint8, device=gc.device)
@@ -1053,6 +1055,8 @@ def ns_normalize_batch(g: torch.Tensor) -> torch.Tensor:
     if g.dtype != torch.bfloat16 or g.dim() != 3:
         raise ValueError("ns_normalize_batch: g must be a 3-D bfloat16 array")
     gc = g.contiguous()
+    if not _aligned(gc, 16):
+        gc = gc.clone()
     out = torch.empty_like(gc)
     L = int(g.shape[0])
     ws = torch.empty(L * _ws_bytes("pratchya_ns_normalize_workspace_bytes"), dtype=torch.uint8, device=gc.device)

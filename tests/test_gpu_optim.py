@@ -316,3 +316,26 @@ def test_argument_errors():
     with pytest.raises(Exception, match="f32 direction"):
         K.apply_update(torch.zeros((128, 128), device="cuda"), False, 1.0, m, (128, 128), torch.bfloat16, 0.1,
                        0.01, torch.bfloat16)
+
+
+@pytest.mark.parametrize("shape,grid", [((3, 100, 33), (4, 11)), ((2, 5, 7), (5, 7)), ((4, 33, 50), (3, 2))])
+@pytest.mark.parametrize("gq", [False, True])
+def test_stacked_leaf_of_odd_slices(shape, grid, gq):
+    """A stacked Muon leaf whose slices are no multiple of 16 bytes: each layer's
+    update (to the bf16 iteration's tolerance) and momentum (the same bytes) are
+    those of the layer stepped by itself."""
+    from pratchya_amd import optim
+    K = _K()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    mom, par, gr = (K.quantize(torch.randn(shape, generator=gen, device="cuda") * 1e-3, grid) for _ in range(3))
+    g = gr if gq else K.dequantize(*gr, torch.bfloat16, grid)
+    args = (grid, 0.9, 0.99, 5, 3e-4, 0.02, 0.1)
+    upd, new_m = optim._quantized_stack_step(("layers",), g, mom, par, *args)
+    for i in range(shape[0]):
+        gi = tuple(t[i].clone() for t in g) if gq else g[i].clone()
+        one, m1 = optim._quantized_slice_step(("layers",), gi, tuple(t[i].clone() for t in mom),
+                                              tuple(t[i].clone() for t in par), grid, torch.bfloat16, *args[1:],
+                                              torch.bfloat16)
+        assert float((upd[i].double() - one.double()).norm() / one.double().norm()) <= 3e-2
+        for a, b in zip(new_m, m1):
+            assert torch.equal(a[i].view(torch.uint8), b.view(torch.uint8))
