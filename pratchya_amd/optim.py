@@ -97,35 +97,27 @@ def newton_schulz(G: torch.Tensor, steps: int = 5) -> torch.Tensor:
 
 
 def _newton_schulz_bf16(X: torch.Tensor, steps: int) -> torch.Tensor:
-    """The iteration of each slice of a normalized bf16 [layers, m, n] array."""
+    """The iteration of each slice of a normalized bf16 [layers, m, n] array (one
+    layer unless _batched_products)."""
     L, m, n = (int(d) for d in X.shape)
     transpose = m > n
     # the kernel takes sides that are multiples of 64, so the iterate
     # is zero-padded to them; the pad rows and columns stay exactly zero
     # through every product and combination, and the products over the
     # original block are sums of the same bf16 products (plus exact zeros)
-    mp, npad = -(-m // 64) * 64, -(-n // 64) * 64
+    mp, npad = _sides(m, n)
     padded = (mp, npad) != (m, n)
     if padded:
         Xp = torch.zeros((L, mp, npad), dtype=X.dtype, device=X.device)
         Xp[:, :m, :n] = X
         X = Xp
-    gram_side = npad if transpose else mp
-    # Short of 256x256 tiles both products run on 128x128 tiles, the first in
-    # full (its triangles hold the same sums: symmetric bit for bit), all layers
-    # at once.  Measured (us, one layer, Gram kernel / 128x128 tiles): sides of
-    # 1024 58 / 30, 2048 (of 8192) 105 / 87, 4096 93 / 124; the combination in
-    # the epilogue alike ([1024, 4096] 34 / 28, [2048, 2048] 57 / 36, [2048,
-    # 8192] 69 / 80); two layers of [1024, 4096] cost 1.3 of one, whose K steps
-    # have to be split to fill the chip.
-    if gram_side <= 2048 and K.few_tiles(mp, npad):
+    if _batched_products(mp, npad):
         for _ in range(steps):
             A = K.gemm_planes_batch(X, X, transpose, torch.bfloat16)
             a, b = (X, A) if transpose else (A, X)
             X = K.gemm_planes_batch(a, b, False, torch.bfloat16, x=X, b_k_major=not transpose)
     else:
-        X = [_newton_schulz_slice(X[l], gram_side, steps) for l in range(L)]
-        X = X[0][None] if L == 1 else torch.stack(X)
+        X = _newton_schulz_slice(X[0], npad if transpose else mp, steps)[None]
     return X[:, :m, :n].contiguous() if padded else X
 
 
@@ -300,15 +292,44 @@ def _quantized_slice_step(path, g, m_t, p_t, tgrid, dtype, beta1, beta2, ns_step
 # Elements of a stacked leaf that one pass takes at once (bounds its
 # intermediates: the direction and the new momentum before requantization).
 _STACK_ELEMENTS = 1 << 28
+_MAX_BATCH = 65535                       # slices of one launch
+
+
+def _sides(m: int, n: int):
+    """The sides that the bf16 iteration of an [m, n] slice works on (multiples of 64)."""
+    return -(-m // 64) * 64, -(-n // 64) * 64
+
+
+def _batched_products(mp: int, npad: int) -> bool:
+    """Whether the slices' products run all layers at once: short of 256x256
+    tiles both run on 128x128 tiles, the first in full (its triangles hold the
+    same sums: symmetric bit for bit).  Measured (us, one layer, Gram kernel /
+    128x128 tiles): sides of 1024 58 / 30, 2048 (of 8192) 105 / 87, 4096 93 /
+    124; the combination in the epilogue alike ([1024, 4096] 34 / 28, [2048,
+    2048] 57 / 36, [2048, 8192] 69 / 80); two layers of [1024, 4096] cost 1.3
+    of one, whose K steps have to be split to fill the chip."""
+    return min(mp, npad) <= 2048 and K.few_tiles(mp, npad)
+
+
+def _layers_per_pass(m: int, n: int, muon: bool) -> int:
+    """Layers of a stacked leaf that one pass takes: one where the products take
+    them one at a time anyway, so that a single layer's intermediates are held."""
+    if muon:
+        mp, npad = _sides(m, n)
+        if not _batched_products(mp, npad):
+            return 1
+        m, n = mp, npad
+    return min(_MAX_BATCH, max(1, _STACK_ELEMENTS // max(1, m * n)))
 
 
 def _quantized_stack_step(path, g, m_t, p_t, tgrid, beta1, beta2, ns_steps, lion_lr, muon_lr, wd):
-    """_quantized_slice_step of every layer of a stacked leaf (bf16), all layers
-    in one pass of each kernel: (update, new momentum triple).  ``g``: a triple
-    or a tensor of the leaf's shape."""
+    """_quantized_slice_step of every layer of a stacked leaf (bf16), several
+    layers in one pass of each kernel: (update, new momentum triple).  ``g``: a
+    triple or a tensor of the leaf's shape."""
     dt = torch.bfloat16
     L, m, n = (int(d) for d in m_t[0].shape)
-    run = max(1, _STACK_ELEMENTS // max(1, m * n))
+    muon = _should_use_muon(path, 2)
+    run = _layers_per_pass(m, n, muon)
     parts = []
     for l in range(0, L, run):
         at = lambda t: t[l:l + run]     # noqa: E731
@@ -316,7 +337,6 @@ def _quantized_stack_step(path, g, m_t, p_t, tgrid, beta1, beta2, ns_steps, lion
         c, nm = K.momentum(tuple(at(t) for t in m_t), gl, tgrid, dt, _as_dtype(beta1, dt), _as_dtype(1.0 - beta1, dt),
                            _as_dtype(beta2, dt), _as_dtype(1.0 - beta2, dt))
         new_m = K.quantize(nm, tgrid)
-        muon = _should_use_muon(path, 2)
         lr = muon_lr if muon else lion_lr
         if muon and m and n:
             k = int(c.shape[0])

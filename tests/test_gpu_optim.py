@@ -339,3 +339,41 @@ def test_stacked_leaf_of_odd_slices(shape, grid, gq):
         assert float((upd[i].double() - one.double()).norm() / one.double().norm()) <= 3e-2
         for a, b in zip(new_m, m1):
             assert torch.equal(a[i].view(torch.uint8), b.view(torch.uint8))
+
+
+def test_stacked_leaf_passes(monkeypatch):
+    """Layers of a stacked leaf per pass: all at once where the products are
+    batched (few tiles), one at a time where they are not (nothing is gained by
+    holding several layers' intermediates), never more than a launch's batch
+    or the element bound, padded sides counted."""
+    from pratchya_amd import optim
+    K = _K()
+    passes, momentum = [], K.momentum
+    monkeypatch.setattr(K, "momentum", lambda m, *a: passes.append(int(m[0].shape[0])) or momentum(m, *a))
+
+    def step(path, shape, grid):
+        gen = torch.Generator(device="cuda").manual_seed(6)
+        mom, par = (K.quantize(torch.randn(shape, generator=gen, device="cuda") * 1e-3, grid) for _ in range(2))
+        g = torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+        passes.clear()
+        out = optim._quantized_stack_step(path, g, mom, par, grid, 0.9, 0.99, 5, 3e-4, 0.02, 0.1)
+        return out, g, mom, par
+
+    step(("layers",), (3, 256, 512), (128, 128))
+    assert passes == [3]
+    step(("layers",), (2, 2304, 2560), (128, 128))
+    assert passes == [1, 1]
+    step(("embed_tokens",), (2, 2304, 2560), (128, 128))
+    assert passes == [2]
+    monkeypatch.setattr(optim, "_STACK_ELEMENTS", 5 * 64 * 64)
+    step(("layers",), (12, 8, 16), (8, 8))                      # padded to 64 x 64
+    assert passes == [5, 5, 2]
+    monkeypatch.undo()
+    monkeypatch.setattr(K, "momentum", lambda m, *a: passes.append(int(m[0].shape[0])) or momentum(m, *a))
+    (upd, new_m), g, mom, par = step(("layers",), (65600, 8, 8), (8, 8))
+    assert sum(passes) == 65600 and max(passes) <= 65535
+    for i in (0, 65534, 65535, 65599):
+        one, m1 = optim._quantized_slice_step(("layers",), g[i], tuple(t[i] for t in mom), tuple(t[i] for t in par),
+                                              (8, 8), torch.bfloat16, 0.9, 0.99, 5, 3e-4, 0.02, 0.1, torch.bfloat16)
+        assert float((upd[i].double() - one.double()).norm() / one.double().norm()) <= 3e-2
+        assert torch.equal(new_m[0][i].view(torch.uint8), m1[0].view(torch.uint8))
