@@ -642,6 +642,14 @@ def _tile_readable(p: torch.Tensor) -> torch.Tensor:
     return padded[:rows]
 
 
+def _aligned_payload(p: torch.Tensor) -> torch.Tensor:
+    """A contiguous [rows, K] payload for the 128-row-tile kernels, which read no
+    row past the last but whole 16-byte chunks: a misaligned one that
+    _tile_readable copies for the 256x256 kernel is copied alike."""
+    p = p.contiguous()
+    return p if _aligned(p, 16) else _tile_readable(_u8(p))
+
+
 def _word_readable(e8: torch.Tensor) -> torch.Tensor:
     """An e8m0 array readable up to the next multiple of 4 bytes (the GEMM
     reads each byte as the aligned word that holds it): used in place when its
@@ -805,7 +813,7 @@ def gemm_t128(a: Operand, b: Operand, out_dtype: torch.dtype = torch.float32) ->
     if a.k_major or b.k_major:
         raise PratchyaUnsupported("gemm_t128: K-contiguous operands only")
     M, N, Kd = a.rows, b.rows, a.k
-    ap, bp = a.payload.contiguous(), b.payload.contiguous()
+    ap, bp = _aligned_payload(a.payload), _aligned_payload(b.payload)
     as8, bs8 = a.sc8.contiguous(), b.sc8.contiguous()
     as32, bs32 = a.sc32.contiguous().float(), b.sc32.contiguous().float()
     lib = _lib.load()
@@ -1211,7 +1219,7 @@ def gemm_t128_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool =
     H = int(lead[-1])
     if a.k_major or b.k_major or N % 128 or H * N % 1024 or M < 1:
         raise PratchyaUnsupported("gemm_t128_fq: K-contiguous operands, outputs in whole groups of 8 blocks")
-    ap, bp = a.payload.contiguous(), b.payload.contiguous()
+    ap, bp = _aligned_payload(a.payload), _aligned_payload(b.payload)
     as8, bs8 = a.sc8.contiguous(), b.sc8.contiguous()
     as32, bs32 = a.sc32.contiguous().float(), b.sc32.contiguous().float()
     lib, dev = _lib.load(), ap.device

@@ -325,3 +325,25 @@ def test_scales_inside_larger_arrays():
     c = K.gemm_t128(K.operand_rows(*xq, (1, 128)), w)
     at = xq[0], _shifted(xq[1].view(torch.uint8), 1).view(xq[1].dtype), _shifted(xq[2], 1)
     assert at[1].data_ptr() % 4 and torch.equal(K.gemm_t128(K.operand_rows(*at, (1, 128)), w), c)
+
+
+@pytest.mark.parametrize("rows", [5, 33, 200])
+def test_payload_at_any_offset(rows):
+    """A payload of fewer than 256 rows that starts at no multiple of 16 bytes, as
+    the kernels of more tiles take it (they copy it): the same products, on the
+    split-K kernel and its requantizing form, and through the public product."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    xq, wq = K.quantize(_randn((rows, 512), 3), (1, 128)), K.quantize(_randn((512, 1024), 4), (128, 128))
+    at = (_shifted(xq[0].view(torch.uint8), 8).view(xq[0].dtype),) + xq[1:]
+    assert at[0].data_ptr() % 16
+    w = K.operand_transposed(*wq, (128, 128))
+    a, b = K.operand_rows(*xq, (1, 128)), K.operand_rows(*at, (1, 128))
+    assert torch.equal(K.gemm_t128(b, w), K.gemm_t128(a, w))
+    for got, want in zip(K.gemm_t128_fq(b, w, torch.bfloat16), K.gemm_t128_fq(a, w, torch.bfloat16)):
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    mk = Q.QArrayImpl._tree_unflatten
+    W = mk((True, (128, 128)), wq)
+    for dt in (torch.bfloat16, torch.float32):
+        y, z = ((mk((True, (1, 128)), t) @ W).astype(dt) for t in (xq, at))
+        assert torch.equal(y, z)
