@@ -436,12 +436,18 @@ def _flat_scales(shape, grid) -> bool:
 _WGRAD_PAIRS_F32 = [(0, 0), (3, 1), (1, 3), (3, 2), (1, 1), (2, 3)]
 
 
+def _plane_scales(shape, go) -> bool:
+    """Whether the planes of a cotangent take its output's scales themselves."""
+    return int(go[0]) == 1 and int(go[1]) % 8 == 0 and _flat_scales(shape, go)
+
+
 def _plane_backward(g, scales, saved, grids, need_x, need_y):
     """f32 cotangents of dequant(x) and dequant(y) (Q:618-622) on the bf16 MFMA
     kernel, from operands read as few exact bf16 planes, or (None, None) for
     what its layouts do not take.  ``g``: the product's cotangent (bf16 or f32),
-    ``scales`` (sc_fp8, sc_fp32, grid): those of the output's quantization when
-    g is the cotangent before dequantize_impl_bwd, else None.
+    ``scales`` (sc_fp8, sc_fp32, grid, one that _plane_scales takes): those of the
+    output's quantization when g is the cotangent before dequantize_impl_bwd,
+    else None.
 
     x's cotangent: a quantized weight is one bf16 plane (its e4m3fn values and
     powers of two) times its group maxima's mantissas, which the kernel applies
@@ -460,8 +466,6 @@ def _plane_backward(g, scales, saved, grids, need_x, need_y):
     gs8 = gs32 = go = None
     if scales is not None:
         gs8, gs32, go = scales
-        if int(go[0]) != 1 or int(go[1]) % 8 or not _flat_scales(tuple(g.shape), go):
-            g, gs8, gs32, go = K.dequantize_bwd(g, gs8, gs32, go), None, None, None
     bf = g.dtype == torch.bfloat16
     gxf = gyf = None
     try:
@@ -503,6 +507,8 @@ def _matmul_cotangents(g, saved, grids, need_x, need_y, scales=None):
         res = _fp8_backward(g, x8, xs8, xs32, y8, ys8, ys32, gx, gy, need_x, need_y)
         if res is not None:
             return res[:2]
+    if scales is not None and not _plane_scales(tuple(g.shape), scales[2]):
+        g, scales = K.dequantize_bwd(g, *scales), None     # once, for the planes and what they leave
     gxf, gyf = _plane_backward(g, scales, saved, grids, need_x, need_y)
     if (need_x and gxf is None) or (need_y and gyf is None):
         if scales is not None:

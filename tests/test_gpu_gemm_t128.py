@@ -347,3 +347,18 @@ def test_payload_at_any_offset(rows):
     for dt in (torch.bfloat16, torch.float32):
         y, z = ((mk((True, (1, 128)), t) @ W).astype(dt) for t in (xq, at))
         assert torch.equal(y, z)
+
+
+def test_cotangent_scaled_once(monkeypatch):
+    """The default backward of an output head ((1, 1) output blocks, a weight in
+    one-column blocks): the cotangent goes through dequantize_impl_bwd once,
+    whichever products take it."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    x, w = _randn((300, 256), 1, torch.bfloat16).requires_grad_(), _randn((256, 640), 2, torch.bfloat16, 0.02)
+    w.requires_grad_()
+    y = (Q.QArrayImpl(x, (1, 128)) @ Q.QArrayImpl(w, (128, 1))).astype(torch.bfloat16)
+    calls, scale = [], K.dequantize_bwd
+    monkeypatch.setattr(K, "dequantize_bwd", lambda *a: calls.append(a[0].shape) or scale(*a))
+    torch.autograd.grad(y, (x, w), torch.ones_like(y))
+    assert len(calls) == 1
