@@ -857,7 +857,9 @@ F32_PLANE_PAIRS = ((0, 0), (3, 1), (1, 3), (3, 2), (1, 1), (2, 3))
 def _matmul_f32_planes(a, b, a_t, b_t, M, N, Kd):
     """matmul_f32 on 128x128 tiles, the operands' planes in their own layouts
     (each written once, no transposed copies)."""
-    if a.dtype == torch.bfloat16 or ((not a_t or b_t) and Kd % 64):
+    # what planes() and gemm_planes() take: whole chunks of 8 of every plane's
+    # rows (4 of the output's), K a multiple of 64 unless both are padded along it
+    if a.dtype == torch.bfloat16 or ((not a_t or b_t) and Kd % 64) or (a_t and M % 8) or N % (4 if b_t else 8):
         raise PratchyaUnsupported("matmul_f32: packed pieces")
     if b.dtype == torch.bfloat16:
         flags = torch.zeros(2, dtype=torch.int32, device=a.device)

@@ -362,3 +362,20 @@ def test_cotangent_scaled_once(monkeypatch):
     monkeypatch.setattr(K, "dequantize_bwd", lambda *a: calls.append(a[0].shape) or scale(*a))
     torch.autograd.grad(y, (x, w), torch.ones_like(y))
     assert len(calls) == 1
+
+
+
+@pytest.mark.parametrize("M,N,Kd,a_t,b_t", [(100, 520, 192, True, False), (96, 524, 192, False, False),
+                                            (96, 102, 192, False, True), (96, 102, 192, False, False),
+                                            (96, 520, 200, False, False)])
+@pytest.mark.parametrize("bdt", [torch.float32, torch.bfloat16])
+def test_no_planes_for_refused_products(M, N, Kd, a_t, b_t, bdt, monkeypatch):
+    """An f32 product whose planes the 128x128 kernel would refuse (a side of its
+    K-major operands no multiple of 8, an N no multiple of 4) writes none."""
+    K = _K()
+    a, b = _randn((Kd, M) if a_t else (M, Kd), 1), _randn((N, Kd) if b_t else (Kd, N), 2, bdt)
+    calls, planes = [], K.planes
+    monkeypatch.setattr(K, "planes", lambda *a, **k: calls.append(a[0]) or planes(*a, **k))
+    c = K.matmul_f32(a, b, a_t, b_t)
+    ref = (a.T if a_t else a).double() @ (b.T if b_t else b).double()
+    assert not calls and _rel(c, ref) <= TOL
