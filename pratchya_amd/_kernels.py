@@ -873,6 +873,21 @@ def _matmul_f32_planes(a, b, a_t, b_t, M, N, Kd):
     return gemm_planes(pa, pb, F32_PLANE_PAIRS, a_t, b_k_major=not b_t)
 
 
+def _packed_on_few_tiles(M: int, N: int, Kd: int) -> bool:
+    """Whether a product of packed pieces (Kd columns in all) takes 128x128 tiles:
+    few_tiles, where those are the faster ones also for a short K.  Measured (us,
+    whole products of bf16 operands, 256x256 / 128x128 tiles): [2048, 512] . [512,
+    2048] 31 / 41, K 768 39 / 42, K 1024 47 / 44 (from 512 on K is split in two
+    there, which pays from 1024); [4096, 256] . [256, 2048] 26 / 30, K 512 36 /
+    35 (128 tiles: K is not split).  Fewer than 256 rows or columns would have
+    to be padded for the 256x256 kernel."""
+    if not few_tiles(M, N) or min(M, N) < GEMM_TILE_ROWS:
+        return few_tiles(M, N)
+    if -(-M // GEMM_TILE_ROWS) * -(-N // GEMM_TILE_ROWS) > 64:
+        return Kd >= 512
+    return Kd < 512 or Kd >= 1024
+
+
 def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = False) -> torch.Tensor:
     """f32 ``op(a) @ op(b)`` for 2-D f32 / bf16 tensors on the bf16 MFMA
     kernel: ``op(a)`` is ``a`` [M, K] (``a_t``: ``a`` is [K, M] and is used
@@ -896,7 +911,10 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
         return torch.empty((M, N), dtype=torch.float32, device=a.device)
     if Kd == 0:
         return torch.zeros((M, N), dtype=torch.float32, device=a.device)
-    if few_tiles(M, N) and M > 32:
+    # (a bf16 b of a short K: two packs of it cost the host and the chip no more
+    # than a flag word, two passes of planes and a pass that repairs them:
+    # [256, 256] . [256, 256] 34 us packed, 38 as planes; K 512 48 / 42)
+    if few_tiles(M, N) and M > 32 and (b.dtype == torch.float32 or Kd >= 384):
         try:
             return _matmul_f32_planes(a, b, a_t, b_t, M, N, Kd)
         except PratchyaUnsupported:
@@ -915,7 +933,7 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, a_t: bool = False, b_t: bool = 
     A = _split_pack(a, a_t, a_planes, kp)
     B = _split_pack(b, not b_t, b_planes, kp, n_rows)
     c = None
-    if few_tiles(M, n_rows):
+    if _packed_on_few_tiles(M, n_rows, len(pairs) * kp):
         try:
             c = gemm_planes(A[None], B[None], [(0, 0)], False)
         except PratchyaUnsupported:      # few rows of more than 2^24 columns

@@ -379,3 +379,26 @@ def test_no_planes_for_refused_products(M, N, Kd, a_t, b_t, bdt, monkeypatch):
     c = K.matmul_f32(a, b, a_t, b_t)
     ref = (a.T if a_t else a).double() @ (b.T if b_t else b).double()
     assert not calls and _rel(c, ref) <= TOL
+
+
+@pytest.mark.parametrize("M,N,Kd,adt,bdt,planes,few", [
+    (256, 256, 256, "f", "b", 0, False), (1024, 1024, 128, "f", "b", 0, True), (256, 256, 384, "f", "b", 2, True),
+    (256, 256, 64, "f", "f", 2, True), (2048, 2048, 448, "b", "b", 0, True), (2048, 2048, 512, "b", "b", 0, False),
+    (2048, 2048, 960, "b", "b", 0, False), (2048, 2048, 1024, "b", "b", 0, True), (4096, 2048, 448, "b", "b", 0, False),
+    (4096, 2048, 512, "b", "b", 0, True), (512, 1024, 256, "b", "f", 0, False), (40, 8192, 768, "b", "b", 0, True),
+    (264, 136, 600, "b", "b", 0, True)])
+def test_routes_of_short_products(M, N, Kd, adt, bdt, planes, few, monkeypatch):
+    """On both sides of the lines that choose an f32 product's tiles: the route,
+    and the product against float64."""
+    K = _K()
+    dt = {"f": torch.float32, "b": torch.bfloat16}
+    a, b = _randn((M, Kd), 1, dt[adt]), _randn((Kd, N), 2, dt[bdt])
+    calls = {"planes": 0, "gemm_planes": 0, "gemm_bf16_nt": 0}
+    for name in calls:
+        def spy(*args, _f=getattr(K, name), _n=name, **kw):
+            calls[_n] += 1
+            return _f(*args, **kw)
+        monkeypatch.setattr(K, name, spy)
+    c = K.matmul_f32(a, b)
+    assert calls == {"planes": planes, "gemm_planes": int(few), "gemm_bf16_nt": int(not few)}
+    assert _rel(c, a.double() @ b.double()) <= TOL
