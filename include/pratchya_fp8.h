@@ -501,8 +501,8 @@ int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps, 
 
 /* pratchya_gemm_bs_nt on 128-row tiles (32-row tiles up to M = 32): the same
  * operands and scale layouts, summed in another order.  Operands are read up
- * to their last row only, e8m0 bytes one at a time.  N a multiple of 4 (f32) or
- * 8 (bf16), groups of a power of two of blocks, B's group maxima shared by
+ * to their last row and scale arrays up to their last entry only.  N a multiple
+ * of 4 (f32) or 8 (bf16), groups of a power of two of blocks, B's group maxima shared by
  * aligned runs of 4 rows (PRATCHYA_EUNSUPPORTED otherwise). */
 int pratchya_gemm_bs_t128(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, const float* a_sc32, int64_t a_rdiv,
                           int64_t a_sr, int64_t a_sk, int64_t a_kg, const uint8_t* B, int64_t ldb,

@@ -262,7 +262,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   uint32_t ea_n[MI], eb_n[NI];
   v4f fa_n[MI];
   float fb_g = 1.0f;
-  const bool a_words = SC == 1 && p.a.sk2 == 2 && p.a.s_r % 4 == 0 && (reinterpret_cast<uintptr_t>(p.a.e8) & 3) == 0;
+  // (a last word that the array holds in part would be out of range: zeros)
+  const bool a_words = SC == 1 && p.a.sk2 == 2 && p.a.s_r % 4 == 0 && p.a.e8_bytes % 4 == 0 &&
+                       (reinterpret_cast<uintptr_t>(p.a.e8) & 3) == 0;
   int a_shift = 0;
   float ga_n[MI], gb_n[NI][4];
   int seg = k_begin / p.spp, s = k_begin - seg * p.spp;

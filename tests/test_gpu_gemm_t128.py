@@ -402,3 +402,38 @@ def test_routes_of_short_products(M, N, Kd, adt, bdt, planes, few, monkeypatch):
     c = K.matmul_f32(a, b)
     assert calls == {"planes": planes, "gemm_planes": int(few), "gemm_bf16_nt": int(not few)}
     assert _rel(c, a.double() @ b.double()) <= TOL
+
+
+@pytest.mark.parametrize("M,Kd,sr", [(100, 768, 8), (7, 768, 8), (100, 640, 0), (33, 1152, 12), (100, 1024, 8)])
+def test_strided_scale_rows(M, Kd, sr):
+    """The C entry on rows of e8m0 bytes in wider rows (or one row's shared by
+    all: sr 0) whose last row ends with its last used byte: the product of the
+    same scales packed, all K steps of the last rows included."""
+    K = _K()
+    lib = K._lib.load()
+    N, nk, kg = 256, Kd // 128, 2
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    a = K.quantize(_randn((M, Kd), 1), (1, 128))[0]
+    rows = M if sr else 1
+    e8 = torch.randint(121, 128, (rows, nk), generator=gen, device="cuda", dtype=torch.uint8)
+    g32 = torch.rand((rows, -(-nk // kg)), generator=gen, device="cuda") + 0.5
+    w = K.operand_transposed(*K.quantize(_randn((Kd, N), 2), (128, 128)), (128, 128))
+
+    def product(e, g, a_sr, a_kg):
+        c = torch.empty((M, N), device="cuda")
+        ws_bytes = lib.pratchya_gemm_t128_workspace_bytes(M, N, nk, 1)
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device="cuda")
+        K._lib.check(lib.pratchya_gemm_bs_t128(
+            K._ptr(a), Kd, K._ptr(e), K._ptr(g), 1, a_sr, 1, a_kg, K._ptr(w.payload), Kd, K._ptr(w.sc8), K._ptr(w.sc32),
+            *w.desc, M, N, Kd, K._ptr(c), N, K._dtype_code(c.dtype), K._ptr(ws), ws_bytes, K._stream(a)), "gemm_t128")
+        return c
+
+    wide = torch.full(((rows - 1) * sr + nk,), 255, dtype=torch.uint8, device="cuda")
+    gw = torch.full((wide.numel() // kg + 1,), float("nan"), device="cuda")
+    for r in range(rows):
+        wide[r * sr:r * sr + nk] = e8[r]
+        gw[r * sr // kg:r * sr // kg + g32.shape[1]] = g32[r]
+    # packed, one block per group
+    ep = e8.expand(M, nk).contiguous()
+    gp = g32.repeat_interleave(kg, 1)[:, :nk].expand(M, nk).contiguous()
+    assert _rel(product(wide, gw, sr, kg), product(ep, gp, nk, 1).double()) <= TOL
