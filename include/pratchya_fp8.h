@@ -560,6 +560,7 @@ int pratchya_gemm_fine(const void* A, int64_t lda, const float* a_sc32, const vo
 /* bf16 planes [planes][T_pad][W] of a row-major [T, W] matrix quantized (a, b)
  * (rows T .. T_pad zeros; W and b multiples of 8, b a power of two):
  *   0 payload -> its power-of-two plane f32(q) * (2^(e-127) * 2^floor(log2 G)) / 128
+ *     (with flags also as mode 3: a second plane)
  *   1 payload -> the three exact pieces of the dequantized f32 value; flags[0]
  *     |= 1 where a third piece is not zero
  *   2 f32 (times its block's scale / 128 if sc8 is given, dequantize_impl_bwd) ->
@@ -567,7 +568,8 @@ int pratchya_gemm_fine(const void* A, int64_t lda, const float* a_sc32, const vo
  *   3 bf16 (likewise scaled, rounded once to bf16) -> that value, and where any is
  *     not finite (flags[1] |= 1) a second plane with those as 0
  *   4 payload -> mode 2's planes of the dequantized f32 value
- * flags: two words the caller has zeroed on this stream (modes 1 and 3). */
+ * flags: two words the caller has zeroed on this stream (modes 1 and 3; may be
+ * null in mode 0). */
 int pratchya_planes(int mode, const void* src, const uint8_t* sc8, const float* sc32, int64_t T, int64_t W, int64_t a,
                     int64_t b, int64_t T_pad, void* dst, uint32_t* flags, hipStream_t stream);
 

@@ -953,7 +953,7 @@ def planes(mode: int, src: torch.Tensor, sc8, sc32, tgrid, flags=None, pad: int 
     its scales (PLANE_POW2, PLANE_SPLIT3, PLANE_SPLIT4Q), an f32 matrix (PLANE_SPLIT4) or a bf16
     one (PLANE_BF16), the last two taken through dequantize_impl_bwd with the
     scales if given.  ``flags``: two zeroed uint32 words that say which planes
-    the product needs.  ``PratchyaUnsupported`` for layouts it does not take."""
+    the product needs (PLANE_POW2: if given, a second plane as PLANE_BF16's).  ``PratchyaUnsupported`` for layouts it does not take."""
     _require_gpu(src)
     T, W = int(src.shape[0]), int(src.shape[1])
     Tp = -(-T // pad) * pad
@@ -963,7 +963,8 @@ def planes(mode: int, src: torch.Tensor, sc8, sc32, tgrid, flags=None, pad: int 
     a, b = (int(tgrid[0]), int(tgrid[1])) if sc8 is not None else (1, 8)
     e8 = sc8.contiguous() if sc8 is not None else None
     g32 = sc32.contiguous().float() if sc8 is not None else None
-    out = torch.empty((_PLANE_COUNT[mode], Tp, W), dtype=torch.bfloat16, device=src.device)
+    count = 2 if mode == PLANE_POW2 and flags is not None else _PLANE_COUNT[mode]
+    out = torch.empty((count, Tp, W), dtype=torch.bfloat16, device=src.device)
     _lib.check(_lib.load().pratchya_planes(mode, _ptr(x), _ptr(e8) if e8 is not None else None,
                                            _ptr(g32) if g32 is not None else None, T, W, a, b, Tp, _ptr(out),
                                            _ptr(flags) if flags is not None else None, _stream(x)), "planes")

@@ -1054,7 +1054,8 @@ extern "C" int pratchya_gemm_fine(const void* A, int64_t lda, const float* a_sc3
 // planes keep the layout, rows T .. T_pad are zeros).
 //   POW2    payload with its scales -> one plane, f32(q) * (2^(e-127) * G') / 128
 //           with G' the group maximum's power of two: 4 significant bits, exact.
-//           (A value whose dequantization is not finite is that value.)
+//           (A value whose dequantization is not finite is that value; with flags,
+//           flags[1] and the second plane as for BF16.)
 //   SPLIT3  payload with its scales -> the three pieces of the dequantized f32
 //           value (k_split_pack's: the top 8 significant bits, the next 8, the
 //           rest; their sum is the value).  A payload quantized from bf16 has
@@ -1130,7 +1131,10 @@ __global__ __launch_bounds__(256) void k_planes(PlanesArgs p) {
       v[k] = is_finite_f(full) ? (v[k] * sp) * 0.0078125f : full;
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o[0][k] = pack_bf16x2(v[2 * k], v[2 * k + 1]);
+    for (int k = 0; k < 4; ++k) {
+      o[0][k] = pack_bf16x2(v[2 * k], v[2 * k + 1]);
+      odd |= (uint32_t)((o[0][k] & 0x7F80u) == 0x7F80u) | (uint32_t)((o[0][k] & 0x7F800000u) == 0x7F800000u);
+    }
   } else {
     if (p.e8) {
 #pragma unroll
@@ -1166,10 +1170,10 @@ __global__ __launch_bounds__(256) void k_planes(PlanesArgs p) {
   for (int j = 0; j < NP; ++j)
     *reinterpret_cast<uint4*>(dst + j * p.pstride) = make_uint4(o[j][0], o[j][1], o[j][2], o[j][3]);
   // one store per wave at most, and none once the flag is seen set
-  if constexpr (MODE == PL_SPLIT3 || MODE == PL_BF16) {
-    uint32_t* f = p.flags + (MODE == PL_BF16 ? 1 : 0);
-    const uint64_t any = __ballot((MODE == PL_BF16 ? odd : third) != 0u);
-    if (any != 0u && (threadIdx.x & 63) == (uint32_t)__builtin_ctzll(any) &&
+  if constexpr (MODE == PL_SPLIT3 || MODE == PL_BF16 || MODE == PL_POW2) {
+    uint32_t* f = p.flags + (MODE == PL_SPLIT3 ? 0 : 1);
+    const uint64_t any = __ballot((MODE == PL_SPLIT3 ? third : odd) != 0u);
+    if (p.flags && any != 0u && (threadIdx.x & 63) == (uint32_t)__builtin_ctzll(any) &&
         __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
       __hip_atomic_fetch_or(f, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -1218,12 +1222,13 @@ extern "C" int pratchya_planes(int mode, const void* src, const uint8_t* sc8, co
                (uint32_t)(W / 8), (uint32_t)a, (uint32_t)(lb < 0 ? 0 : lb), (uint32_t)nbc, (uint32_t)lk, T_pad * W};
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
   switch (mode) {
-    case PL_POW2: hipLaunchKernelGGL(k_planes<PL_POW2>, grid, block, 0, stream, p); break;
     case PL_SPLIT3: hipLaunchKernelGGL(k_planes<PL_SPLIT3>, grid, block, 0, stream, p); break;
     case PL_SPLIT4Q: hipLaunchKernelGGL(k_planes<PL_SPLIT4Q>, grid, block, 0, stream, p); break;
     case PL_SPLIT4: hipLaunchKernelGGL(k_planes<PL_SPLIT4>, grid, block, 0, stream, p); break;
     default: {
-      hipLaunchKernelGGL(k_planes<PL_BF16>, grid, block, 0, stream, p);
+      if (mode == PL_POW2) hipLaunchKernelGGL(k_planes<PL_POW2>, grid, block, 0, stream, p);
+      else hipLaunchKernelGGL(k_planes<PL_BF16>, grid, block, 0, stream, p);
+      if (!flags) break;
       const int64_t blocks = (n + 255) / 256;
       hipLaunchKernelGGL(k_plane_finite, dim3((unsigned)(blocks < 1024 ? blocks : 1024)), block, 0, stream, p.dst,
                          p.pstride, n, flags);

@@ -475,9 +475,14 @@ def _plane_backward(g, scales, saved, grids, need_x, need_y):
         return None, None
     if need_x:
         try:
-            pw = K.planes(K.PLANE_POW2, y8, ys8, ys32, gy)
-            gxf = K.gemm_planes(pg[:1 if bf else 3, :rows], pw, [(i, 0) for i in range(1 if bf else 3)], False,
-                                units=(ys32, gy, K.group_layout(Kd, N, gy)[1]))
+            units = (ys32, gy, K.group_layout(Kd, N, gy)[1])
+            if bf:
+                pw = K.planes(K.PLANE_POW2, y8, ys8, ys32, gy)
+                gxf = K.gemm_planes(pg[:1, :rows], pw, [(0, 0)], False, units=units)
+            else:                        # (a non-finite weight meets the first piece only: not 0 * inf)
+                pw = K.planes(K.PLANE_POW2, y8, ys8, ys32, gy, flags)
+                gxf = K.gemm_planes(pg[:3, :rows], pw, [(0, 0), (1, 0), (2, 0)], False, short=3, b_alt=[0, 1, 1],
+                                    flags=flags, units=units)
             gxf = gxf.reshape(tuple(g.shape[:-1]) + (Kd,))
         except K.PratchyaUnsupported:
             gxf = None

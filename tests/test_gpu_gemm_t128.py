@@ -437,3 +437,25 @@ def test_strided_scale_rows(M, Kd, sr):
     ep = e8.expand(M, nk).contiguous()
     gp = g32.repeat_interleave(kg, 1)[:, :nk].expand(M, nk).contiguous()
     assert _rel(product(wide, gw, sr, kg), product(ep, gp, nk, 1).double()) <= TOL
+
+
+def test_input_gradient_of_a_non_finite_weight():
+    """A weight too large to dequantize (inf): an f32 cotangent's products with it
+    are inf, -inf and NaN where the f32 products of the dequantized operands are
+    (a zero piece of a finite value meets no inf)."""
+    from pratchya_amd import qarr as Q
+    K = _K()
+    rows, Kd, N, blk = 192, 256, 384, 128
+    x, w, g = _randn((rows, Kd), 1), _randn((Kd, N), 2), _randn((rows, N), 3)
+    g = torch.where(torch.rand((rows, N), device="cuda", generator=torch.Generator(device="cuda").manual_seed(4)) < 0.3,
+                    g.to(torch.bfloat16).float(), g)        # values of one piece among those of three
+    w[3, 5], w[200, 300] = 3e38, -3e38
+    xq, wq = K.quantize(x, (1, blk)), K.quantize(w, (blk, blk))
+    wd = K.dequantize(*wq, torch.float32, (blk, blk))
+    assert int(torch.isinf(wd).sum()) == 2
+    gx = Q._plane_backward(g, None, xq + wq, ((1, blk), (blk, blk)), True, False)[0]
+    ref = g.double() @ wd.double().T
+    assert torch.equal(torch.isnan(gx), torch.isnan(ref)) and torch.equal(torch.isposinf(gx), torch.isposinf(ref))
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(gx), fin) and not bool(fin.all())
+    assert _rel(torch.where(fin, gx, 0.0), torch.where(fin, ref, 0.0)) <= TOL
