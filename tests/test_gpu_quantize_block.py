@@ -1,12 +1,12 @@
 """Quantization with a workgroup per block (grids whose block is 4096 to 65536
 elements in rows of 64 or more) or per group (blocks of 16 x 16 and 32 x 32) against the oracle and, bit for bit, against
-the flat kernels, which take the same values from an unaligned buffer."""
+the flat kernels, which take the outputs that start at no multiple of 16 bytes."""
 import numpy as np
 import pytest
 import torch
 
 from oracle import qarr_oracle as O
-from tests.helpers import assert_bytes_equal, assert_f32_bits_equal, f32, u8
+from tests.helpers import assert_bytes_equal, assert_f32_bits_equal, assert_payload_equal, f32, u8
 
 pytestmark = pytest.mark.gpu
 
@@ -35,11 +35,12 @@ def _values(shape, dtype, seed):
     return x.view(shape).to(dtype)
 
 
-def _unaligned(x):
-    buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)
-    y = buf[1:].view(x.shape)
-    y.copy_(x)
-    return y
+def _unaligned(shape, dtype):
+    """A buffer that the kernels of 16-byte stores do not take."""
+    n = 1
+    for d in shape:
+        n *= d
+    return torch.empty(n + 1, dtype=dtype, device="cuda")[1:].view(shape)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -47,18 +48,26 @@ def _unaligned(x):
 def test_block_per_workgroup(shape, grid, dtype):
     from pratchya_amd import _kernels as K
     x = _values(shape, dtype, 7)
-    other = _unaligned(x)
     q, s8, s32 = K.quantize(x, grid)
-    for got, want in zip(K.quantize(other, grid), (q, s8, s32)):
+    flat = (_unaligned(shape, torch.uint8), torch.empty_like(s8), torch.empty_like(s32))
+    assert flat[0].data_ptr() % 16
+    for got, want in zip(K.quantize(x, grid, out=flat), (q, s8, s32)):
         assert_bytes_equal(u8(got.contiguous().view(torch.uint8)), u8(want.contiguous().view(torch.uint8)), "flat")
     wq, we, wg = O.quantize_impl(f32(x), grid)
     assert_bytes_equal(u8(s8).reshape(-1), we.view(np.uint8).reshape(-1), "e8m0")
     assert_f32_bits_equal(f32(s32).reshape(-1), wg.reshape(-1), "group maxima")
+    assert_payload_equal(u8(q), wq.view(np.uint8), "payload")
     for out in (torch.bfloat16, torch.float32):
         for fix in (False, True):
-            a, b = K.quantize_dequantize(x, grid, out, fix), K.quantize_dequantize(other, grid, out, fix)
-            for got, want in zip(a, b):
+            a = K.quantize_dequantize(x, grid, out, fix)
+            flat = (_unaligned(shape, out), torch.empty_like(a[1]), torch.empty_like(a[2]))
+            assert flat[0].data_ptr() % 16
+            for got, want in zip(a, K.quantize_dequantize(x, grid, out, fix, out=flat)):
                 assert torch.equal(got.contiguous().view(torch.uint8), want.contiguous().view(torch.uint8))
+            e = np.where(we.view(np.uint8) == 0xFF, np.uint8(0x7F), we.view(np.uint8)) if fix else we
+            want = O.dequantize_impl(wq, e, wg, "float32" if out == torch.float32 else "bfloat16", grid)
+            want = want if out == torch.float32 else O.bf16_bits_to_f32(want)
+            assert_f32_bits_equal(f32(a[0]), want, "fake quantization")
 
 
 @pytest.mark.parametrize("ids_shape,out_grid", [((256,), (128, 128)), ((2, 192), (64, 64)), ((100,), (50, 128)),
