@@ -504,6 +504,12 @@ __device__ __forceinline__ void load_chunk(const void* x, int64_t off, float (&v
 #pragma unroll
       for (int k = 0; k < E; ++k) v[j * E + k] = elem_f32<IS_BF16>(w, k);
     }
+  } else if constexpr (VEC && IS_BF16 && CH == 4) {
+    const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const char*>(x) + off * ESZ);
+    v[0] = u2f(w.x << 16);
+    v[1] = u2f(w.x & 0xFFFF0000u);
+    v[2] = u2f(w.y << 16);
+    v[3] = u2f(w.y & 0xFFFF0000u);
   } else {
 #pragma unroll
     for (int k = 0; k < CH; ++k) v[k] = load_elem<IS_BF16>(x, off + k);
@@ -657,15 +663,21 @@ __global__ __launch_bounds__(256) void k_cast_general(const void* __restrict__ x
   }
 }
 
+// (elements per thread and step of the block kernels' casts: one 16-byte store,
+// consecutive lanes on consecutive chunks of a row, so that each store
+// instruction writes whole lines.  With two or four stores side by side per lane,
+// f32 results of [8192, 8192]: (128, 128) 131 -> 82 us, (16, 16) 334 -> 60 (bf16
+// x) and 345 -> 80, (32, 32) 230 -> 73 and 239 -> 98)
+constexpr int tile_cast_chunk(int out) { return out == 0 ? 16 : (out == 1 ? 8 : 4); }
+
 // Blocks of 16 x 16 in groups of 16 and of 32 x 32 in groups of 64 (the block
 // size 16 and 32 presets' weights and their gradients): a workgroup owns a group
 // and holds it in registers, one pass and one launch where the flat kernels take
 // four (fill, block maxima with atomics, group scales, cast).  [2048, 2048] in
-// blocks of 16: bf16 to payloads 24 -> 5.2 us, f32 to bf16 22 -> 6.2 us; in
-// blocks of 32, back to back from a graph, 12.6 -> 6.8 and 15.2 -> 12.1 us,
-// [4096, 4096] 21.0 -> 9.1 and 31.5 -> 21.8 us.  (Of 4 groups, where few CUs have
-// work, the time is one group's chain: [512, 512] f32 9.8 -> 11.2 us from a
-// graph, less than the three launches saved cost an eager caller.)  A thread holds 16 consecutive values of one row in every RG-th row of a block;
+// blocks of 16, back to back from a graph: bf16 to payloads 16 -> 5.9 us, f32 to
+// bf16 20 -> 5.1; in blocks of 32 11.9 -> 6.7 and 15.4 -> 10.6 us; [512, 512]
+// (4 groups: one group's chain) 10.6 -> 6.4 and 10.1 -> 9.6.  A
+// thread holds CH consecutive values of one row in every RG-th row of a block;
 // consecutive threads hold consecutive pieces of a row of the group's blocks.
 template <bool IS_BF16, int OUT, int B>
 __global__ __launch_bounds__(B == 16 ? 256 : 1024) void k_group_square(const void* __restrict__ x,
@@ -673,12 +685,12 @@ __global__ __launch_bounds__(B == 16 ? 256 : 1024) void k_group_square(const voi
                                                                        uint8_t* __restrict__ sc8,
                                                                        float* __restrict__ sc32, int64_t W,
                                                                        int fix_nan) {
-  constexpr int CH = 16, OSZ = OUT == 0 ? 1 : (OUT == 1 ? 2 : 4);
+  constexpr int CH = tile_cast_chunk(OUT), OSZ = 16 / CH, NT = B == 16 ? 256 : 1024;
   constexpr int K = B == 16 ? 16 : 64, P = B / CH;              // blocks of a group, pieces of a block's row
-  constexpr int RG = (B == 16 ? 256 : 1024) / (K * P), R = B / RG;
-  constexpr int NW = K * P < 64 ? RG * K * P / 64 : RG;         // maxima of a block that meet in the LDS
+  constexpr int ROW = K * P, RG = NT / ROW, R = B / RG;         // threads on a row of the group's blocks
+  constexpr int NW = ROW < 64 ? NT / 64 : RG;                   // maxima of a block that meet in the LDS
   __shared__ uint32_t lds[NW][K];
-  const int c = threadIdx.x % (K * P), j = c / P, r = threadIdx.x / (K * P);
+  const int c = threadIdx.x % ROW, j = c / P, r = threadIdx.x / ROW;
   const int64_t blk = (int64_t)blockIdx.x * K + j, bpr = W / B, bi = blk / bpr;
   const int64_t off = (bi * B + r) * W + (blk - bi * bpr) * B + c % P * CH;
   float v[R][CH];
@@ -689,26 +701,23 @@ __global__ __launch_bounds__(B == 16 ? 256 : 1024) void k_group_square(const voi
   for (int i = 0; i < R; ++i)
 #pragma unroll
     for (int k = 0; k < CH; ++k) m = umax(m, abs_bits(v[i][k]));
-  if constexpr (B == 16) {
-    m = xor_max_u32<32>(xor_max_u32<16>(m));                    // a wave holds four rows of every block
-    if ((threadIdx.x & 63) < 16) lds[threadIdx.x >> 6][j] = m;
-  } else {
-    m = lane_group_max<P>(m);
-    if (c % P == 0) lds[r][j] = m;
-  }
+  m = lane_group_max<P>(m);
+  if constexpr (ROW <= 16) m = xor_max_u32<16>(m);              // a wave holds 64 / ROW rows of every block
+  if constexpr (ROW <= 32) m = xor_max_u32<32>(m);
+  const int l = threadIdx.x & 63;
+  if (c % P == 0 && (ROW >= 64 || l < ROW)) lds[ROW < 64 ? threadIdx.x >> 6 : r][j] = m;
   __syncthreads();
   m = 0;
 #pragma unroll
   for (int i = 0; i < NW; ++i) m = umax(m, lds[i][j]);
   uint32_t g = m;
   if constexpr (B != 16) {
-    // a wave's 64 lanes hold half of the group's blocks
-    const int l = threadIdx.x & 63;
+    // a wave's 64 lanes hold some of the group's blocks
     g = 0;
 #pragma unroll
     for (int i = 0; i < NW; ++i) g = umax(g, lds[i][l]);
   }
-  const float G = u2f(lane_group_max<K>(g));
+  const float G = u2f(lane_group_max<B == 16 ? ROW : 64>(g));
   const uint32_t e = e8m0_of(u2f(m), G);
   if (r == 0 && c % P == 0) sc8[blk] = (uint8_t)e;
   if (threadIdx.x == 0) sc32[blockIdx.x] = G;
@@ -719,12 +728,9 @@ __global__ __launch_bounds__(B == 16 ? 256 : 1024) void k_group_square(const voi
   const float dq = e8m0_decode((fix_nan && e == 0xFFu) ? 0x7Fu : e) * G;
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    uint32_t w[CH * OSZ / 4];
+    uint32_t w[4];
     cast_words<CH, OUT>(v[i], yv, S, ok, dq, w);
-#pragma unroll
-    for (int q = 0; q < CH * OSZ / 16; ++q)
-      store_stream16(static_cast<char*>(outv) + (off + (int64_t)i * RG * W) * OSZ + 16 * q,
-                     u32x4_t{w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]});
+    store_stream16(static_cast<char*>(outv) + (off + (int64_t)i * RG * W) * OSZ, u32x4_t{w[0], w[1], w[2], w[3]});
   }
 }
 
@@ -757,15 +763,12 @@ __global__ __launch_bounds__(256) void k_tile_max(const void* __restrict__ x, ui
   if (threadIdx.x == 0) ws[blk] = m;
 }
 
-// (elements per thread: 16 bytes of the output, and of the input at least)
-constexpr int tile_cast_chunk(bool bf16, int out) { return out == 0 ? 16 : (out == 1 || bf16 ? 8 : 4); }
-
 template <bool IS_BF16, int OUT>
 __global__ __launch_bounds__(256) void k_tile_cast(const void* __restrict__ x, void* __restrict__ outv,
                                                    const uint32_t* __restrict__ ws, uint8_t* __restrict__ sc8,
                                                    float* __restrict__ sc32, int64_t W, int a, int b, int64_t K,
                                                    int seg_log2, int fix_nan) {
-  constexpr int CH = tile_cast_chunk(IS_BF16, OUT), OSZ = OUT == 0 ? 1 : (OUT == 1 ? 2 : 4), U = 4;
+  constexpr int CH = tile_cast_chunk(OUT), OSZ = 16 / CH, U = 4;
   __shared__ uint32_t lds[4];
   const uint32_t blk = blockIdx.x, bpr = (uint32_t)(W / b), bi = blk / bpr, bj = blk - bi * bpr;
   const int RT = 256 >> seg_log2, r0 = threadIdx.x >> seg_log2, c = (threadIdx.x & ((1 << seg_log2) - 1)) * CH;
@@ -792,12 +795,10 @@ __global__ __launch_bounds__(256) void k_tile_cast(const void* __restrict__ x, v
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (r + u * RT >= a) break;
-      uint32_t w[CH * OSZ / 4];
+      uint32_t w[4];
       cast_words<CH, OUT>(v[u], yv, S, ok, dq, w);
-#pragma unroll
-      for (int j = 0; j < CH * OSZ / 16; ++j)
-        store_stream16(static_cast<char*>(outv) + (base + (int64_t)(r + u * RT) * W) * OSZ + 16 * j,
-                       u32x4_t{w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]});
+      store_stream16(static_cast<char*>(outv) + (base + (int64_t)(r + u * RT) * W) * OSZ,
+                     u32x4_t{w[0], w[1], w[2], w[3]});
     }
   }
 }
@@ -1289,7 +1290,7 @@ int launch_general(const void* x, void* q, uint8_t* sc8, float* sc32, uint32_t* 
                    const Layout& L, hipStream_t st, int fix_nan = 0, bool premax = false) {
   const int64_t n_blocks_total = L.S * L.n_blk;
   const int64_t n_groups = L.S * L.M;
-  constexpr int CIN = IS_BF16 ? 8 : 4, COUT = tile_cast_chunk(IS_BF16, OUT);
+  constexpr int CIN = IS_BF16 ? 8 : 4, COUT = tile_cast_chunk(OUT);
   if (tile_fits(L.a, L.b, CIN, COUT, OUT == 0 ? 1 : (OUT == 1 ? 2 : 4), n_blocks_total) && aligned(x, 16) && aligned(q, 16)) {
     const dim3 grid((unsigned)n_blocks_total);
     if (!premax)
@@ -1299,8 +1300,11 @@ int launch_general(const void* x, void* q, uint8_t* sc8, float* sc32, uint32_t* 
                        (int)L.b, L.K, ilog2(L.b / COUT), fix_nan);
     return check_launch("quantize(block)");
   }
+  // (a group of 32 x 32 blocks is 65536 values: f32 results of few such groups
+  // leave the chip to as many CUs, from a graph [512, 512] 10 / 16 us on the flat
+  // kernels / a workgroup per group, [2048, 2048] 16.5 / 16.7, [2048, 4096] 22 / 18)
   if (!premax && L.a == L.b && ((L.a == 16 && L.K == 16) || (L.a == 32 && L.K == 64)) && n_groups <= 0x7FFFFFFF &&
-      aligned(x, 16) && aligned(q, 16)) {
+      (OUT != 2 || L.a == 16 || n_groups >= 128) && aligned(x, 16) && aligned(q, 16)) {
     if (L.a == 16)
       hipLaunchKernelGGL((k_group_square<IS_BF16, OUT, 16>), dim3((unsigned)n_groups), dim3(256), 0, st, x, q, sc8,
                          sc32, L.W, fix_nan);

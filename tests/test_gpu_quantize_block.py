@@ -82,3 +82,26 @@ def test_gathered_rows(ids_shape, out_grid):
     rows = K.gather_dequantize(*table, (128, 128), ids, torch.float32)
     for got, want in zip(K.gather_quantize(*table, (128, 128), ids, out_grid), K.quantize(rows, out_grid)):
         assert torch.equal(got.contiguous().view(torch.uint8), want.contiguous().view(torch.uint8))
+
+
+# (both sides of the lines between the kernels: groups of 32 x 32 blocks for f32
+# results, a block's bytes, blocks for each CU, elements in all)
+LINES = [((2048, 4096), (32, 32)), ((2048, 4064), (32, 32)), ((768, 512), (192, 128)), ((800, 512), (200, 128)),
+         ((4096, 1024), (256, 64)), ((3840, 1088), (256, 64)), ((4096, 4096), (64, 64)), ((4096, 4160), (64, 64)),
+         ((8192, 8192), (128, 128)), ((8192, 8320), (128, 128))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,grid", LINES, ids=lambda v: "x".join(map(str, v)))
+def test_lines_of_the_dispatch(shape, grid, dtype):
+    from pratchya_amd import _kernels as K
+    x = _values(shape, dtype, 8)
+    got = K.quantize(x, grid)
+    flat = (_unaligned(shape, torch.uint8), torch.empty_like(got[1]), torch.empty_like(got[2]))
+    K.quantize(x, grid, out=flat)
+    assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, flat))
+    for out in (torch.bfloat16, torch.float32):
+        got = K.quantize_dequantize(x, grid, out, True)
+        flat = (_unaligned(shape, out), torch.empty_like(got[1]), torch.empty_like(got[2]))
+        K.quantize_dequantize(x, grid, out, True, out=flat)
+        assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, flat))
