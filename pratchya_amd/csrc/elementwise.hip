@@ -23,7 +23,7 @@
 //     block and group maxima by lane shuffles, e8m0 scales, payload;
 //   * general (any grid): the block maxima of the results into a workspace,
 //     then a second pass that recomputes the results and casts them (two
-//     launches, a workgroup per block, where tile_fits; else four: a fill,
+//     launches, a workgroup per block, where ew_tile_fits; else four: a fill,
 //     maxima with atomics, the group scales, the cast).  The operands are
 //     read twice.
 // The operands may have block grids of their own (QArrayImpl's operators on
@@ -362,7 +362,23 @@ __global__ __launch_bounds__(256) void k_ew_cast(QOperand X, QOperand Y, uint8_t
   }
 }
 
-// Workgroup per result block (tile_fits), 16 results per thread and step.
+// Where a workgroup per result block is the faster split: blocks of 4096 to 16384
+// results (16 to 64 per thread) in rows of 64 or more, and at most a * b / 8 of
+// them, two groups' worth: every workgroup folds its group's maxima ahead of its
+// cast, and more rounds of workgroups add more such chains.  In rows of 64, up to
+// 2^24 results (the split lines).  Measured (us from a graph, add, four launches /
+// block per workgroup): (128, 128) [4096, 4096] 39 / 24, [8192, 8192] 77 / 83;
+// (256, 64) [8192, 4096] 51 / 68; (64, 128) [2048, 4096] 29 / 20, [8192, 4096] 51
+// / 64; (64, 64) [1024, 2048] 20 / 13, [2048, 4096] 29 / 33, [4096, 4096] 36 / 61;
+// (128, 256) [2048, 2048] 18 / 25; a lookup of 16352 rows of 4096, whose blocks
+// are (32, 128), 65 / 137.
+inline bool ew_tile_fits(int64_t a, int64_t b, int64_t n_blk_total) {
+  const bool p2 = b > 0 && (b & (b - 1)) == 0;
+  return p2 && b >= 64 && b <= 1024 && a * b >= 4096 && a * b <= 16384 && n_blk_total <= a * b / 8 &&
+         (b >= 128 || n_blk_total * a * b <= (1 << 24));
+}
+
+// Workgroup per result block (ew_tile_fits), 16 results per thread and step.
 template <int OP>
 __global__ __launch_bounds__(256) void k_ew_tile_max(QOperand X, QOperand Y, uint32_t* __restrict__ ws, int64_t W,
                                                      int a, int b, int seg_log2) {
@@ -520,7 +536,7 @@ void launch_general_t(const QOperand& X, const QOperand& Y, uint8_t* q, uint8_t*
                       int64_t n, int64_t W, int64_t a, int64_t b, int64_t K, int64_t n_blk_total,
                       int64_t n_groups, const EwPlan& p, hipStream_t st) {
   if constexpr (CH == 16 && VEC) {
-    if (tile_fits(a, b, 16, 16, 1, n_blk_total)) {
+    if (ew_tile_fits(a, b, n_blk_total)) {
       const dim3 grid((unsigned)n_blk_total);
       hipLaunchKernelGGL((k_ew_tile_max<OP>), grid, dim3(256), 0, st, X, Y, ws, W, (int)a, (int)b, log2_of(b / 16));
       hipLaunchKernelGGL((k_ew_tile_cast<OP>), grid, dim3(256), 0, st, X, Y, q, ws, sc8, sc32, W, (int)a, (int)b, K,

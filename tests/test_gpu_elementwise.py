@@ -207,3 +207,33 @@ def test_getitem_fuses_the_requantization(Q, K, monkeypatch):
     v, s8, s32 = qt._tree_flatten()[0]
     want = K.quantize(K.gather_dequantize(v, s8, s32, (128, 128), ids, torch.float32), (128, 128))
     _check(_triple(got), (u8(want[0]), u8(want[1]), f32(want[2])), "getitem")
+
+
+@pytest.mark.parametrize("shape,grid", [((2048, 1024), (64, 64)), ((2048, 1088), (64, 64)), ((4096, 2048), (64, 128)),
+                                        ((4096, 2176), (64, 128)), ((4096, 8192), (128, 128)), ((4096, 8320), (128, 128)),
+                                        ((256, 256), (256, 128)), ((4096, 4096), (256, 64)),
+                                        ((8192, 4096), (256, 64)), ((96, 256), (48, 64)), ((104, 256), (52, 128))],
+                         ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("op", ["add", "mul"])
+def test_lines_of_the_block_kernels(op, shape, grid):
+    """Both sides of the lines between a workgroup per block and the flat kernels:
+    the bytes of the flat kernels (which take results that start at no multiple
+    of 16 bytes), operands of one grid and of two."""
+    from pratchya_amd import _kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(11)
+
+    def operand(g):
+        v = torch.randn(shape, generator=gen, device="cuda")
+        v = v * torch.exp2(torch.randint(-9, 9, (shape[0], 1), generator=gen, device="cuda").float())
+        v[0, 3], v[1, 7], v[-1] = float("inf"), float("nan"), 0.0
+        return K.quantize(v, g)
+
+    x = operand(grid)
+    for gy in (grid, (1, 16)):
+        y = operand(gy)
+        got = K.elementwise(op, x, grid, y, gy, grid)
+        flat = (torch.empty(x[0].numel() + 1, dtype=torch.uint8, device="cuda")[1:].view(shape),
+                torch.empty_like(got[1]), torch.empty_like(got[2]))
+        K.elementwise(op, x, grid, y, gy, grid, out=flat)
+        for a, b in zip(got, flat):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
