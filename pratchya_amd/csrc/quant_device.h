@@ -342,25 +342,36 @@ static __global__ void k_fill_u32(uint32_t* __restrict__ p, int64_t n, uint32_t 
 
 // --------------------------------------------------------------------------
 // Workgroup-per-block passes, for the grids (a, b) whose block is a fair piece
-// of work for 256 threads (tile_fits): k_*tile_max stores each block's maximum
-// with one plain store, and k_*tile_cast folds its group's K maxima itself and
-// stores the block's e8m0 byte and, for a group's first block, the group
-// maximum.  Against the flat kernels below that takes out the workspace fill,
-// the atomics and the group-scale launch: two launches instead of four
-// (an embedding lookup of 8192 x 2048 in blocks of 128: 38.3 -> 21.4 us).
-// The payload is still read twice; a group spans up to a * b / 16 blocks, all
-// of which have to be seen before the first cast.
-// The bounds: 16 elements per thread at least, for the launch to be worth its
-// reduction, and 256 at most, for one block not to take longer than the whole
-// flat pass.  Row segments that store whole 128-byte lines, or at least 64
-// bytes in arrays of up to 2^24 elements, where the launches saved outweigh
-// the split lines (grid (64, 64), f32 to payloads: [1024, 4096] 14.3 -> 10.1
-// us, [4096, 16384] 92 -> 102 us).
+// of work for 256 threads: k_*tile_max stores each block's maximum with one
+// plain store, and k_*tile_cast folds its group's K maxima itself and stores the
+// block's e8m0 byte and, for a group's first block, the group maximum.  Against
+// the flat kernels that takes out the workspace fill, the atomics and the
+// group-scale launch: two launches instead of four (an embedding lookup of 8192
+// x 2048 in blocks of 128: 38.3 -> 20.4 us).  The payload is still read twice; a
+// group spans up to a * b / 16 blocks, all of which have to be seen before the
+// first cast.
+//
+// tile_fits, the quantizers' lines (elementwise.hip has its own; both sides
+// measured from a graph, flat / block per workgroup):
+// - 16 elements per thread at least, for the launch to be worth its reduction.
+// - A block's bytes, read and written, at most 96 KB, which one CU moves in the
+//   time of the launches saved: f32 to bf16 in one block of (128, 128) 9.4 / 8.0
+//   us, of (256, 128) 9.8 / 11.7, of (512, 128) 9.8 / 18.9; up to 16384 elements
+//   also where there is a block for each CU (f32 to f32 in (256, 64): 64 blocks
+//   11.6 / 11.9, 1024 blocks faster).
+// - Row segments that store whole 128-byte lines, or at least 64 bytes in arrays
+//   of up to 2^24 elements, where the launches saved outweigh the split lines.
+// - Up to 2^24 elements (blocks of 16384: 2^26), beyond which the flat kernels'
+//   longer runs of one row win: f32 to payloads in (32, 128) [8192, 4096] 50 /
+//   54, [8192, 8192] 92 / 103; bf16 in (128, 128) [8192, 8192] 60 / 60, [16384,
+//   8192] 105 / 112.
 // --------------------------------------------------------------------------
-inline bool tile_fits(int64_t a, int64_t b, int ch_in, int ch_out, int out_esz, int64_t n_blk_total) {
+inline bool tile_fits(int64_t a, int64_t b, int ch_in, int ch_out, int in_esz, int out_esz, int64_t n_blk_total) {
   const bool p2 = b > 0 && (b & (b - 1)) == 0;
-  return p2 && b >= 64 && b / ch_in <= 64 && b / ch_out <= 64 && a * b >= 4096 && a * b <= 65536 &&
-         n_blk_total <= 0x7FFFFFFF && (b * out_esz >= 128 || n_blk_total * a * b <= (1 << 24));
+  const int64_t n = n_blk_total * a * b;
+  return p2 && b >= 64 && b / ch_in <= 64 && b / ch_out <= 64 && a * b >= 4096 &&
+         (a * b * (in_esz + out_esz) <= 98304 || (a * b <= 16384 && n_blk_total >= 256)) &&
+         (b * out_esz >= 128 || n <= (1 << 24)) && n <= (a * b >= 16384 ? 1 << 26 : 1 << 24);
 }
 
 // Maximum over the 256 threads of a workgroup, for every thread (lds: 4 words).

@@ -1291,7 +1291,8 @@ int launch_general(const void* x, void* q, uint8_t* sc8, float* sc32, uint32_t* 
   const int64_t n_blocks_total = L.S * L.n_blk;
   const int64_t n_groups = L.S * L.M;
   constexpr int CIN = IS_BF16 ? 8 : 4, COUT = tile_cast_chunk(OUT);
-  if (tile_fits(L.a, L.b, CIN, COUT, OUT == 0 ? 1 : (OUT == 1 ? 2 : 4), n_blocks_total) && aligned(x, 16) && aligned(q, 16)) {
+  if (tile_fits(L.a, L.b, CIN, COUT, IS_BF16 ? 2 : 4, OUT == 0 ? 1 : (OUT == 1 ? 2 : 4), n_blocks_total) && aligned(x, 16) &&
+      aligned(q, 16)) {
     const dim3 grid((unsigned)n_blocks_total);
     if (!premax)
       hipLaunchKernelGGL((k_tile_max<IS_BF16>), grid, dim3(256), 0, st, x, ws, L.W, (int)L.a, (int)L.b,
