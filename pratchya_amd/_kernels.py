@@ -1217,12 +1217,16 @@ def mfma_ceiling(a: torch.Tensor, b: torch.Tensor, bf16: bool, iters: int) -> in
     return int(flop.value)
 
 
-def _few_then_requantize(a: Operand, b: Operand, out_dtype, tgrid, fix_nan, lead):
-    """gemm_nt_q11 of a product of few tiles, as its two steps."""
+def _few_then_requantize(a: Operand, b: Operand, out_dtype, lead, scales: bool):
+    """gemm_nt_q11 of a product of few tiles, as its two steps, the second of
+    which stores the scales of every element (dropped without ``scales``).
+    Measured (us, without scales, the epilogue's one launch / the two steps): 4 x
+    [2048, 4096] 48 / 30, x [2048, 32768] 48 / 31, x [2048, 131072] 89 / 46; 1000 x
+    [2048, 4096] 44 / 39; 4096 x [2048, 1024] 44 / 39."""
     lead = tuple(lead) if lead else (a.rows,)
     c = gemm_t128(a, b, torch.float32)
-    y, s8, s32 = quantize_dequantize(c.view(lead + (b.rows,)), tgrid, out_dtype, fix_nan)
-    return y.view(a.rows, b.rows), s8, s32
+    y, s8, s32 = quantize_dequantize(c.view(lead + (b.rows,)), (1, 1), out_dtype)
+    return (y.view(a.rows, b.rows),) + ((s8, s32) if scales else (None, None))
 
 
 def gemm_t128_fq(a: Operand, b: Operand, out_dtype: torch.dtype, fix_nan: bool = False, lead=None,
@@ -1315,7 +1319,8 @@ def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None, few: 
     (1, 1), out_dtype)``, the scales shaped per slice of ``lead`` as there.
     Raises ``PratchyaUnsupported`` unless N is a multiple of 16.  ``few``: as
     for gemm_nt_fq.  Without ``scales`` the scale arrays, five of the seven
-    bytes written per bf16 element, are neither allocated nor stored (None)."""
+    bytes written per bf16 element, are not returned (None), and unless the
+    product ran as one of few tiles neither allocated nor stored."""
     _require_gpu(a.payload, b.payload)
     if a.k != b.k:
         raise ValueError(f"contraction mismatch: {a.k} vs {b.k}")
@@ -1325,7 +1330,7 @@ def gemm_nt_q11(a: Operand, b: Operand, out_dtype: torch.dtype, lead=None, few: 
     if N % 16:
         raise PratchyaUnsupported(f"gemm_q11: N must be a multiple of 16 (got {N})")
     if few and not a.k_major and prefers_t128(M, a.desc[3], b):
-        return _few_then_requantize(a, b, out_dtype, (1, 1), False, lead)
+        return _few_then_requantize(a, b, out_dtype, lead, scales)
     lib = _lib.load()
     ap, bp = _tile_readable(_u8(a.payload).contiguous()), _tile_readable(_u8(b.payload).contiguous())
     as8, bs8 = _word_readable(_u8(a.sc8).contiguous()), _word_readable(_u8(b.sc8).contiguous())

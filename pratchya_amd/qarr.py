@@ -558,8 +558,8 @@ def _linear_forward_fused(x8, xs8, xs32, y8, ys8, ys32, gx, gy, go, dtype, scale
     tiles make it K.gemm_t128_fq); (1, 1), the
     output of a weight quantized (a, 1) (lm_head, LoRA), N a multiple of 16.
     (A (1, 1) product of few tiles runs as the two steps: ``K.prefers_t128``.)
-    ``scales`` False: the caller keeps only y; the (1, 1) scales, larger than
-    y itself, and those of a product of few tiles are then not stored."""
+    ``scales`` False: the caller keeps only y; the scales are then not returned,
+    and not stored either but for a (1, 1) product of few tiles."""
     go = tuple(go)
     if go not in ((1, 128), (1, 1)) or dtype not in (torch.float32, torch.bfloat16) or y8.dim() != 2:
         return None

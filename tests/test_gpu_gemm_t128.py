@@ -459,3 +459,16 @@ def test_input_gradient_of_a_non_finite_weight():
     fin = torch.isfinite(ref)
     assert torch.equal(torch.isfinite(gx), fin) and not bool(fin.all())
     assert _rel(torch.where(fin, gx, 0.0), torch.where(fin, ref, 0.0)) <= TOL
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 200])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_few_row_head_without_scales(rows, dt):
+    """The output head's product of few rows without its scale arrays: the same
+    values, and no scale arrays."""
+    K = _K()
+    a = K.operand_rows(*K.quantize(_randn((rows, 2048), 1, torch.bfloat16), (1, 128)), (1, 128))
+    b = K.operand_transposed(*K.quantize(_randn((2048, 528), 2, torch.bfloat16, 0.02), (128, 1)), (128, 1))
+    y, s8, s32 = K.gemm_nt_q11(a, b, dt, few=True)
+    z, n8, n32 = K.gemm_nt_q11(a, b, dt, few=True, scales=False)
+    assert s8 is not None and s32 is not None and n8 is None and n32 is None and torch.equal(y, z)
