@@ -5,8 +5,9 @@ entry points only enqueue work (no allocation, no host synchronisation, no
 memset nodes): the general quantizer clears its block-max workspace with a
 kernel on every replay, and the fused elementwise general path and the Gram
 product's partial-tile flags likewise; the (1, 1) requantization epilogue,
-the elementwise (1, 1) quantizer, and the weight gradient's block maxima with
-the requantization that starts from them are captured too."""
+the elementwise (1, 1) quantizer, the weight gradient's block maxima with
+the requantization that starts from them, and the products of few tiles with
+their device flags and partial sums are captured too."""
 import numpy as np
 import pytest
 import torch
@@ -42,7 +43,9 @@ def test_graph_replays_match_eager():
 
     def work():
         xq = K.quantize(x, (1, 128))                                    # one-pass kernel
-        wq = K.quantize(w, (128, 128))                                  # general path, workspace
+        wq = K.quantize(w, (128, 128))                                  # a workgroup per block, maxima in the workspace
+        wf = K.quantize(w, (8, 32))                                     # general path: workspace cleared by a kernel
+        wd = K.quantize_dequantize(w, (8, 32), torch.float32)           # the same, dequantized
         yq = K.quantize(y, (1, 128))
         a = K.operand_rows(*xq, (1, 128))
         b = K.operand_transposed(*wq, (128, 128))
@@ -58,7 +61,7 @@ def test_graph_replays_match_eager():
         x11 = K.quantize(x, (1, 1))                                     # elementwise (1, 1) kernel
         c32, bm = K.gemm_nt_blockmax(a, b)                              # block maxima from the epilogue
         wg = K.quantize_dequantize_premax(c32, bm, (128, 128), torch.bfloat16)
-        return [*xq, *wq, c, *s, *d, *t, q, gr, ns, *o11, *x11, c32, bm, *wg]
+        return [*xq, *wq, *wf, *wd, c, *s, *d, *t, q, gr, ns, *o11, *x11, c32, bm, *wg]
 
     fill()
     torch.cuda.synchronize()
@@ -80,3 +83,56 @@ def test_graph_replays_match_eager():
     # and the replayed quantize is the oracle's
     xo = O.quantize_impl(x.float().cpu().numpy(), (1, 128))
     assert np.array_equal(outs[0].view(torch.uint8).cpu().numpy(), xo[0])
+
+
+def test_graph_of_few_tile_products():
+    """Split-K products, products of planes whose flags the device sets anew on
+    every replay (a third piece that is zero or not, a cotangent that is finite
+    or not), fine-block products and batched slices."""
+    from pratchya_amd import optim
+    from pratchya_amd import qarr as Q
+    K = _K()
+    gen = torch.Generator(device="cuda").manual_seed(43)
+    M, Kd, N = 200, 1024, 512
+    x = torch.empty((M, Kd), device="cuda")
+    w = torch.empty((Kd, N), dtype=torch.bfloat16, device="cuda")
+    g = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    s = torch.empty((3, 128, 320), dtype=torch.bfloat16, device="cuda")
+
+    def fill(rep):
+        v = torch.randn((M, Kd), generator=gen, device="cuda")
+        x.copy_(v.to(torch.bfloat16) if rep % 2 else v)
+        w.copy_(torch.randn((Kd, N), generator=gen, device="cuda") * 0.02)
+        g.copy_(torch.randn((M, N), generator=gen, device="cuda"))
+        if rep == 2:
+            g[3, 5], w[7, 9] = float("inf"), float("nan")
+        s.copy_(torch.randn(s.shape, generator=gen, device="cuda"))
+
+    def work():
+        xq, wq = K.quantize(x, (1, 128)), K.quantize(w, (128, 128))
+        a, b = K.operand_rows(*xq, (1, 128)), K.operand_transposed(*wq, (128, 128))
+        c, f = K.gemm_t128(a, b), K.gemm_t128_fq(a, b, torch.bfloat16)
+        grids = ((1, 128), (128, 128))
+        gb = Q._plane_backward(g, (f[1], f[2], (1, 128)), xq + wq, grids, True, True)
+        gf = Q._plane_backward(g.float(), (f[1], f[2], (1, 128)), xq + wq, grids, True, True)
+        fine = Q._fine_forward(*K.quantize(x, (1, 16)), *K.quantize(w, (16, 16)), (1, 16), (16, 16))
+        fq = K.quantize_dequantize(c, (1, 16), torch.bfloat16)
+        ns = optim._newton_schulz_bf16(K.ns_normalize_batch(s), 2)
+        return [c, *f, *gb, *gf, fine, *fq, K.matmul_f32(x, w), K.matmul_f32(x, w.float()), ns]
+
+    fill(0)
+    torch.cuda.synchronize()
+    work()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = work()
+    for rep in range(4):
+        fill(rep)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = work()
+        torch.cuda.synchronize()
+        for i, (got, ref) in enumerate(zip(outs, want)):
+            _same(got, ref, f"replay {rep}, output {i}")
