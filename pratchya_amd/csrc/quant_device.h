@@ -357,21 +357,21 @@ static __global__ void k_fill_u32(uint32_t* __restrict__ p, int64_t n, uint32_t 
 // - A block's bytes, read and written, at most 96 KB, which one CU moves in the
 //   time of the launches saved: f32 to bf16 in one block of (128, 128) 9.4 / 8.0
 //   us, of (256, 128) 9.8 / 11.7, of (512, 128) 9.8 / 18.9; up to 16384 elements
-//   also where there is a block for each CU (f32 to f32 in (256, 64): 64 blocks
-//   11.6 / 11.9, 1024 blocks faster).
+//   in rows of up to 128 also where there is a block for each CU (f32 to f32 in
+//   (256, 64): 64 blocks 11.6 / 11.9, 1024 blocks 41 / 38; in (64, 256) 38 / 41).
 // - Row segments that store whole 128-byte lines, or at least 64 bytes in arrays
 //   of up to 2^24 elements, where the launches saved outweigh the split lines.
-// - Up to 2^24 elements (blocks of 16384: 2^26), beyond which the flat kernels'
-//   longer runs of one row win: f32 to payloads in (32, 128) [8192, 4096] 50 /
-//   54, [8192, 8192] 92 / 103; bf16 in (128, 128) [8192, 8192] 60 / 60, [16384,
-//   8192] 105 / 112.
+// - Up to 2^24 elements (2^26 in blocks of 16384 and rows of up to 128), beyond
+//   which the flat kernels' longer runs of one row win: f32 to payloads in (32,
+//   128) [8192, 4096] 50 / 54, [8192, 8192] 92 / 103; bf16 in (64, 512) of 2^25
+//   elements 35 / 37, in (128, 128) [8192, 8192] 60 / 60, [16384, 8192] 105 / 112.
 // --------------------------------------------------------------------------
 inline bool tile_fits(int64_t a, int64_t b, int ch_in, int ch_out, int in_esz, int out_esz, int64_t n_blk_total) {
   const bool p2 = b > 0 && (b & (b - 1)) == 0;
   const int64_t n = n_blk_total * a * b;
   return p2 && b >= 64 && b / ch_in <= 64 && b / ch_out <= 64 && a * b >= 4096 &&
-         (a * b * (in_esz + out_esz) <= 98304 || (a * b <= 16384 && n_blk_total >= 256)) &&
-         (b * out_esz >= 128 || n <= (1 << 24)) && n <= (a * b >= 16384 ? 1 << 26 : 1 << 24);
+         (a * b * (in_esz + out_esz) <= 98304 || (a * b <= 16384 && b <= 128 && n_blk_total >= 256)) &&
+         (b * out_esz >= 128 || n <= (1 << 24)) && n <= (a * b >= 16384 && b <= 128 ? 1 << 26 : 1 << 24);
 }
 
 // Maximum over the 256 threads of a workgroup, for every thread (lds: 4 words).

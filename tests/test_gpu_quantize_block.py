@@ -88,7 +88,7 @@ def test_gathered_rows(ids_shape, out_grid):
 # results, a block's bytes, blocks for each CU, elements in all)
 LINES = [((2048, 4096), (32, 32)), ((2048, 4064), (32, 32)), ((768, 512), (192, 128)), ((800, 512), (200, 128)),
          ((4096, 1024), (256, 64)), ((3840, 1088), (256, 64)), ((4096, 4096), (64, 64)), ((4096, 4160), (64, 64)),
-         ((8192, 8192), (128, 128)), ((8192, 8320), (128, 128))]
+         ((4096, 4096), (64, 256)), ((8192, 4096), (64, 512)), ((8192, 8192), (128, 128)), ((8192, 8320), (128, 128))]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
