@@ -97,9 +97,11 @@ size_t pratchya_quantize_noalloc_max_bytes(void);
  * quantize_impl -> quantize_impl_bwd (Q:512-526) that a requantized matmul
  * cotangent (Q:637-638) takes back to its f32 input.  sc_fp8 / sc_fp32 receive
  * quantize_impl's scales unrepaired.  out: `out_dtype` values [slices*H*W].
- * `workspace`: pratchya_quantize_dequantize_workspace_bytes(...) bytes (0, and
- * NULL allowed, for tgrid (1, 128) with K = 8 when x and out are 16-byte and
- * sc_fp8 8-byte aligned). */
+ * `workspace`: pratchya_quantize_dequantize_workspace_bytes(...) bytes, what the
+ * layout needs with buffers of any alignment (0, and NULL allowed, for tgrid (1,
+ * 128) with K = 8 when x and out are 16-byte and sc_fp8 8-byte aligned); other
+ * one-pass kernels ((1, b) row groups, square blocks of 16 and 32) leave it
+ * untouched. */
 size_t pratchya_quantize_dequantize_workspace_bytes(int x_dtype, int64_t slices, int64_t H,
                                                     int64_t W, int64_t a, int64_t b);
 int pratchya_quantize_dequantize(const void* x, int x_dtype, int64_t slices, int64_t H, int64_t W,
@@ -465,16 +467,18 @@ int64_t pratchya_ns_normalize_workspace_bytes(void);
 int pratchya_ns_normalize(const void* g, void* x, int64_t n, void* workspace, int64_t workspace_bytes,
                           hipStream_t stream);
 
+/* The same of `batch` (up to 65535) bf16 arrays of n elements one after the
+ * other, each by its own norm (n a multiple of 8 unless batch is 1; g and x
+ * 16-byte aligned); workspace: batch times
+ * pratchya_ns_normalize_workspace_bytes() bytes. */
+int pratchya_ns_normalize_batch(const void* g, void* x, int64_t n, int64_t batch, void* workspace,
+                                int64_t workspace_bytes, hipStream_t stream);
+
 /* The same normalization of an f32 input (_optimizer.py:17 on the f32 leaves
  * of 2-D quantized parameters, _optimizer.py:157-163): each square rounded to
  * f32, their f32 sum (the fixed order of pratchya_ns_normalize), sqrt and the
  * sum with 1e-7 in f32, IEEE f32 quotients.  g, x: f32 [n], 16-byte aligned;
  * x may be g; workspace as pratchya_ns_normalize. */
-/* The same of `batch` bf16 arrays of n elements one after the other, each by its
- * own norm (n a multiple of 8 unless batch is 1); workspace: batch times
- * pratchya_ns_normalize_workspace_bytes() bytes. */
-int pratchya_ns_normalize_batch(const void* g, void* x, int64_t n, int64_t batch, void* workspace,
-                                int64_t workspace_bytes, hipStream_t stream);
 int pratchya_ns_normalize_f32(const float* g, float* x, int64_t n, void* workspace, int64_t workspace_bytes,
                               hipStream_t stream);
 
@@ -502,8 +506,8 @@ int64_t pratchya_gemm_t128_workspace_bytes(int64_t M, int64_t N, int64_t steps, 
 /* pratchya_gemm_bs_nt on 128-row tiles (32-row tiles up to M = 32): the same
  * operands and scale layouts, summed in another order.  Operands are read up
  * to their last row and scale arrays up to their last entry only.  N a multiple
- * of 4 (f32) or 8 (bf16), groups of a power of two of blocks, B's group maxima shared by
- * aligned runs of 4 rows (PRATCHYA_EUNSUPPORTED otherwise). */
+ * of 4 (f32) or 8 (bf16), groups of a power of two of blocks, B's group maxima
+ * shared by aligned runs of 4 rows (PRATCHYA_EUNSUPPORTED otherwise). */
 int pratchya_gemm_bs_t128(const uint8_t* A, int64_t lda, const uint8_t* a_sc8, const float* a_sc32, int64_t a_rdiv,
                           int64_t a_sr, int64_t a_sk, int64_t a_kg, const uint8_t* B, int64_t ldb,
                           const uint8_t* b_sc8, const float* b_sc32, int64_t b_rdiv, int64_t b_sr, int64_t b_sk,

@@ -155,10 +155,12 @@ __device__ __forceinline__ void wg_barrier() {
 // The joins (16 multiply-adds per lane and MFMA, 64 clocks beside its 32) run
 // as a pipeline with the MFMAs (fine_step), where one after the other they left
 // both units waiting: forward of 8192 x [4096, 4096] in blocks of 32 469 -> 426
-// us, of which the product is about 330 (the six-pair f32 product took 1585).  flags (bf16): flags[0] == 0 says that the planes of the segments
-// past segs_short are all zero (the segments are left out); flags[1] != 0 that
-// B's plane 0 holds non-finite values, which may take part in the first
-// segment only (0 * inf): the others then read planes_alt, a copy without.
+// us, four fifths of it the product (400 us by itself at a trace's lower clocks;
+// the six-pair f32 product took 1585).  flags (bf16): flags[0] == 0 says that the
+// planes of the segments past segs_short are all zero (the segments are left
+// out); flags[1] != 0 that B's plane 0 holds non-finite values, which may take
+// part in the first segment only (0 * inf): the others then read planes_alt, a
+// copy without.
 template <bool BF, int TM, bool TNA, bool TNB, int SC, int OUT>
 __global__ __launch_bounds__(256, 2) void k_gemm_t128(T128Args p) {
   static_assert(BF || (!TNA && !TNB), "K-major operands are bf16");

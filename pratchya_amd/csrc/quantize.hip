@@ -1523,7 +1523,9 @@ extern "C" size_t pratchya_quantize_dequantize_workspace_bytes(int x_dtype, int6
   Layout L;
   if (make_layout(slices, H, W, a, b, &L)) return 0;
   // the single-pass group-per-wave kernel (tgrid (1, 128), K = 8, 16-byte
-  // aligned x and out) needs none; every other layout runs the general path
+  // aligned x and out) needs none; every other layout may run on the general
+  // path: the one-pass kernels of row groups and of square blocks do not touch
+  // the workspace, but buffers that are not aligned for them do
   if (g8_layout(L)) return 0;
   return (size_t)(L.S * L.n_blk) * sizeof(uint32_t);
 }
