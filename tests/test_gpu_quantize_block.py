@@ -1,6 +1,7 @@
-"""Quantization with a workgroup per block (grids whose block is 4096 to 65536
-elements in rows of 64 or more) or per group (blocks of 16 x 16 and 32 x 32) against the oracle and, bit for bit, against
-the flat kernels, which take the outputs that start at no multiple of 16 bytes."""
+"""Quantization with a workgroup per block (grids whose block is 4096 to 32768
+elements in rows of 64 or more) or per group (blocks of 16 x 16 and 32 x 32)
+against the oracle and, bit for bit, against the flat kernels, which take the
+outputs that start at no multiple of 16 bytes (and larger blocks anyway)."""
 import numpy as np
 import pytest
 import torch
